@@ -31,15 +31,25 @@ template <typename Tc> struct acc4;
 template <> struct acc4<double> {
   typedef d4_t type;
   static __device__ __forceinline__ int row(int group, int v) { return group + 4 * v; }
+  // lane group and accumulator element that hold a row
+  static __device__ __forceinline__ int group(int row) { return row & 3; }
+  static __device__ __forceinline__ int elem(int row) { return row >> 2; }
 };
 template <> struct acc4<float> {
   typedef f4_t type;
   static __device__ __forceinline__ int row(int group, int v) { return 4 * group + v; }
+  static __device__ __forceinline__ int group(int row) { return row >> 2; }
+  static __device__ __forceinline__ int elem(int row) { return row & 3; }
 };
 
-// Workgroup = 4 waves as 2 x 2; each wave owns (16*TM) rows x (8*TN) complex columns.
-// BK complex k per LDS stage (2 BK real k = BK / 2 MFMA k-steps); LDS holds two
-// stages (double buffer).
+// A group of 4 waves (2 x 2) owns a BM x BN tile; each wave owns (16*TM) rows x
+// (8*TN) complex columns. A workgroup holds WK such groups on the same tile,
+// group w taking the w-th part of the k-stages; their sums are added in the
+// order of the groups through LDS at the end. Splitting k inside the workgroup
+// gives a product with few tiles more waves in flight and a shorter chain of
+// dependent stages without a workspace or a second launch.
+// BK complex k per LDS stage (BK / 4 steps of two MFMAs per tile); a group's LDS
+// holds two stages (double buffer).
 template <int TM, int TN, int BK_ = 8> struct TileCfg {
   static constexpr int WM = 16 * TM;
   static constexpr int WN = 8 * TN;
@@ -49,9 +59,11 @@ template <int TM, int TN, int BK_ = 8> struct TileCfg {
   static constexpr int NA = BM * BK / 256;
   static constexpr int NB = BN * BK / 256;
 };
-// FP32 stages twice as deep as FP64 ones: same LDS bytes per stage
-template <typename Tc> struct StageK { static constexpr int value = 8; };
-template <> struct StageK<float> { static constexpr int value = 16; };
+// k-stage depth: FP32 stages twice as deep as FP64 ones (same LDS bytes), and the
+// smallest tile twice as deep (256 threads stage at least one element each)
+template <typename Tc, int TM> struct StageK {
+  static constexpr int value = (TM == 1 || sizeof(Tc) == 4) ? 16 : 8;
+};
 
 struct GemmKArgs {
   int64_t M, N, K;
@@ -73,6 +85,8 @@ struct GemmKArgs {
   // skip[z * skip_stride] != 0
   const int* skip;
   int64_t skip_stride;
+  // byte offsets inside a tile's operand rows fit 32 bits (launch_cfg)
+  int fast;
 };
 
 // masked products keep their stage list in LDS: K / BK at most this many stages
@@ -153,74 +167,105 @@ __device__ __forceinline__ void tile_coords(int wg, int nwg, int tiles_m, int ti
   tn = in / rows;
 }
 
-template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, bool A_KCONTIG,
-          bool B_NCONTIG>
-__global__ __launch_bounds__(256) void zgemm_kernel(GemmKArgs g) {
-  typedef TileCfg<TM, TN, StageK<Tc>::value> T;
+// Operands are staged as whole complex elements, [k][row] and [k][column]. A step
+// takes four complex k: lane group kk = lane / 16 holds complex k = 4 step + kk of
+// its row of A and of its column of B, and one MFMA multiplies the real parts of
+// A with (Re B | Im B), a second one the imaginary parts with (-Im B | Re B) for
+// the (even | odd) real columns: the order of the real k inside a step is free as
+// long as A and B agree, and this one reads every staged element once, as one
+// LDS access, and needs no arithmetic on B but a select.
+//
+// What bounds it: FP64 MFMA issue on the large tile. The addresses of a stage
+// are a uniform base plus a 32-bit offset per thread that is constant over the
+// k-loop (rows and columns beyond the matrix are clamped to the last one: their
+// results are not stored), so a stage's loads need no per-element address
+// arithmetic and no predicates; only the last, partial k-stage and operands
+// whose offsets exceed 32 bits take the general path.
+template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, int WK,
+          bool A_KCONTIG, bool B_NCONTIG>
+__global__ __launch_bounds__(256 * WK) void zgemm_kernel(GemmKArgs g) {
+  typedef TileCfg<TM, TN, StageK<Tc, TM>::value> T;
   constexpr int BM = T::BM, BN = T::BN, BK = T::BK, NA = T::NA, NB = T::NB;
   typedef typename acc4<Tc>::type acc_t;
+  typedef typename cplx_of<Tc>::type C2;
+  static_assert(NA >= 1 && NB >= 1, "a stage holds at least one element per thread");
 
-  __shared__ Tc As[2][2 * BK][BM + 1];
-  __shared__ Tc Bs[2][BK][2 * BN + 2];
+  struct Stage {
+    C2 A[2][BK][BM + 1];
+    C2 B[2][BK][BN + 1];
+  };
+  __shared__ __align__(16) Stage stage_mem[WK];
   if (g.skip && g.skip[blockIdx.z * g.skip_stride]) return;
 
-  const int tid = threadIdx.x;
+  const int grp = WK == 1 ? 0 : (int)(threadIdx.x >> 8);
+  const int tid = threadIdx.x & 255;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm0 = (wave >> 1) * T::WM;
   const int wn0 = (wave & 1) * T::WN;
+  auto& As = stage_mem[grp].A;
+  auto& Bs = stage_mem[grp].B;
 
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * BM;
   const int64_t n0 = (int64_t)tn * BN;
   const int64_t bz = blockIdx.z;
-  const TA* __restrict__ A = (const TA*)g.A + bz * g.bz_a;
-  const TB* __restrict__ B = (const TB*)g.B + bz * g.bz_b;
+  const TA* __restrict__ A = (const TA*)g.A + bz * g.bz_a + m0 * g.a_m;
+  const TB* __restrict__ B = (const TB*)g.B + bz * g.bz_b + n0 * g.b_n;
   TC* __restrict__ C = (TC*)g.C + bz * g.bz_c;
   const Tc sa = g.conjA ? (Tc)-1 : (Tc)1;
   const Tc sb = g.conjB ? (Tc)-1 : (Tc)1;
 
-  Tc ra[NA][2], rb[NB][2];
-  auto load_tiles = [&](int64_t k0) {
+  // element i of this thread in a stage: row / column (clamped) and k
+  auto arow = [&](int i) -> int { return A_KCONTIG ? (tid + 256 * i) / BK : (tid + 256 * i) % BM; };
+  auto ak = [&](int i) -> int { return A_KCONTIG ? (tid + 256 * i) % BK : (tid + 256 * i) / BM; };
+  auto bcol = [&](int i) -> int { return B_NCONTIG ? (tid + 256 * i) % BN : (tid + 256 * i) / BK; };
+  auto bk = [&](int i) -> int { return B_NCONTIG ? (tid + 256 * i) / BN : (tid + 256 * i) % BK; };
+  const int mlast = (int)(g.M - m0 < BM ? g.M - m0 : BM) - 1;
+  const int nlast = (int)(g.N - n0 < BN ? g.N - n0 : BN) - 1;
+  uint32_t offa[NA], offb[NB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+    offa[i] = (uint32_t)((min(arow(i), mlast) * g.a_m + ak(i) * g.a_k) * (int64_t)sizeof(TA));
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    offb[i] = (uint32_t)((min(bcol(i), nlast) * g.b_n + bk(i) * g.b_k) * (int64_t)sizeof(TB));
+
+  C2 ra[NA], rb[NB];
+  // stage at k0, all of it inside K, 32-bit offsets
+  auto load_fast = [&](int64_t k0) {
+    const char* Ak = (const char*)(A + k0 * g.a_k);
+    const char* Bk = (const char*)(B + k0 * g.b_k);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) load_c<Tc>((const TA*)(Ak + offa[i]), ra[i].x, ra[i].y);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) load_c<Tc>((const TB*)(Bk + offb[i]), rb[i].x, rb[i].y);
+  };
+  // any stage (zeros beyond K)
+  auto load_general = [&](int64_t k0) {
+    const TA* Ak = A + k0 * g.a_k;
+    const TB* Bk = B + k0 * g.b_k;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      int e = tid + 256 * i;
-      int row, kc;
-      if (A_KCONTIG) { row = e / BK; kc = e % BK; } else { kc = e / BM; row = e % BM; }
-      int64_t m = m0 + row, k = k0 + kc;
-      Tc re = 0, im = 0;
-      if (m < g.M && k < g.K) load_c<Tc>(A + m * g.a_m + k * g.a_k, re, im);
-      ra[i][0] = re; ra[i][1] = sa * im;
+      ra[i] = C2{0, 0};
+      if (k0 + ak(i) < g.K)
+        load_c<Tc>(Ak + (int64_t)min(arow(i), mlast) * g.a_m + (int64_t)ak(i) * g.a_k, ra[i].x,
+                   ra[i].y);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      int e = tid + 256 * i;
-      int col, kc;
-      if (B_NCONTIG) { kc = e / BN; col = e % BN; } else { col = e / BK; kc = e % BK; }
-      int64_t n = n0 + col, k = k0 + kc;
-      Tc re = 0, im = 0;
-      if (n < g.N && k < g.K) load_c<Tc>(B + k * g.b_k + n * g.b_n, re, im);
-      rb[i][0] = re; rb[i][1] = sb * im;
+      rb[i] = C2{0, 0};
+      if (k0 + bk(i) < g.K)
+        load_c<Tc>(Bk + (int64_t)min(bcol(i), nlast) * g.b_n + (int64_t)bk(i) * g.b_k, rb[i].x,
+                   rb[i].y);
     }
   };
   auto store_tiles = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      int e = tid + 256 * i;
-      int row, kc;
-      if (A_KCONTIG) { row = e / BK; kc = e % BK; } else { kc = e / BM; row = e % BM; }
-      As[buf][2 * kc][row] = ra[i][0];
-      As[buf][2 * kc + 1][row] = ra[i][1];
-    }
+    for (int i = 0; i < NA; ++i) As[buf][ak(i)][arow(i)] = C2{ra[i].x, sa * ra[i].y};
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      int e = tid + 256 * i;
-      int col, kc;
-      if (B_NCONTIG) { kc = e / BN; col = e % BN; } else { col = e / BK; kc = e % BK; }
-      Bs[buf][kc][2 * col] = rb[i][0];
-      Bs[buf][kc][2 * col + 1] = rb[i][1];
-    }
+    for (int i = 0; i < NB; ++i) Bs[buf][bk(i)][bcol(i)] = C2{rb[i].x, sb * rb[i].y};
   };
 
   acc_t acc[TM][TN];
@@ -229,61 +274,118 @@ __global__ __launch_bounds__(256) void zgemm_kernel(GemmKArgs g) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
 
-  // per-lane selection of the expanded B operand: real k parity (a) and real
-  // column parity (b): (0,0) Re, (0,1) Im, (1,0) -Im, (1,1) Re
-  const int kk = lane >> 4;
-  const int pa = kk & 1, pb = lane & 1;
-  const bool take_im = (pa != pb);
-  const Tc im_sign = (pa == 1) ? (Tc)-1 : (Tc)1;
+  const int l16 = lane & 15, kk = lane >> 4;
+  const int pb = lane & 1;
 
-  // k-stages to visit: all of them, or (with masks) the list of stages where
-  // the A and B tile masks overlap, built once in LDS so that the main loop is
-  // a plain counted loop (keeps the accumulators in place across iterations)
+  // k-stages to visit: a group's share [st0, st0 + per) of all of them, or (with
+  // masks) those of its share where the A and B tile masks overlap, listed once
+  // in LDS so that the main loop is a plain counted loop (keeps the accumulators
+  // in place across iterations). The shares do not depend on the masks, so a
+  // masked product adds in the order of the unmasked one. Every group runs
+  // `iters` iterations (the barriers are the workgroup's).
   const int nk = (int)((g.K + BK - 1) / BK);
   __shared__ unsigned short stages[MAX_MASKED_STAGES];
-  __shared__ int nstage_s;
-  int nst = nk;
+  __shared__ int nstage_s[WK];
+  const int per = (nk + WK - 1) / WK;
+  const int st0 = grp * per, st1 = min(st0 + per, nk);
+  int mine = max(0, st1 - st0), iters = per;
   if (g.maskA) {
     if (tid == 0) {
       int c = 0;
-      for (int t = next_stage(g, tm, tn, 0, nk); t < nk; t = next_stage(g, tm, tn, t + 1, nk))
-        stages[c++] = (unsigned short)t;
-      nstage_s = c;
+      for (int t = next_stage(g, tm, tn, st0, st1); t < st1;
+           t = next_stage(g, tm, tn, t + 1, st1))
+        stages[st0 + c++] = (unsigned short)t;
+      nstage_s[grp] = c;
     }
     __syncthreads();
-    nst = nstage_s;
-  }
-  auto stage_of = [&](int it) -> int { return g.maskA ? (int)stages[it] : it; };
-  // stage pipeline: global loads of the next stage into registers, MFMAs on
-  // the current LDS buffer, registers into the other buffer, one barrier
-  int buf = 0;
-  if (nst > 0) {
-    load_tiles((int64_t)stage_of(0) * BK);
-    store_tiles(0);
-  }
-  __syncthreads();
-  for (int it = 0; it < nst; ++it) {
-    const bool more = it + 1 < nst;
-    if (more) load_tiles((int64_t)stage_of(it + 1) * BK);
+    mine = nstage_s[grp];
+    iters = 0;
 #pragma unroll
-    for (int ks = 0; ks < BK / 2; ++ks) {
-      Tc av[TM], bv[TN];
+    for (int w = 0; w < WK; ++w) iters = max(iters, nstage_s[w]);
+  }
+  auto stage_of = [&](int it) -> int64_t {
+    return g.maskA ? (int64_t)stages[st0 + it] : (int64_t)(st0 + it);
+  };
+  auto multiply = [&](int buf) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i) av[i] = As[buf][4 * ks + kk][wm0 + 16 * i + (lane & 15)];
+    for (int ks = 0; ks < BK / 4; ++ks) {
+      C2 av[TM];
+      Tc b0[TN], b1[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) av[i] = As[buf][4 * ks + kk][wm0 + 16 * i + l16];
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const Tc* p = &Bs[buf][2 * ks + (kk >> 1)][2 * (wn0 + 8 * j + ((lane & 15) >> 1))];
-        Tc re = p[0], im = p[1];
-        bv[j] = take_im ? im_sign * im : re;
+        const C2 b = Bs[buf][4 * ks + kk][wn0 + 8 * j + (l16 >> 1)];
+        b0[j] = pb ? b.y : b.x;
+        b1[j] = pb ? b.x : -b.y;
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(av[i], bv[j], acc[i][j]);
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(av[i].x, b0[j], acc[i][j]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(av[i].y, b1[j], acc[i][j]);
     }
+  };
+  // stage pipeline: global loads of the next stage into registers, MFMAs on
+  // the current LDS buffer, registers into the other buffer, one barrier. The
+  // first loop runs while the next stage is a whole one, without a branch in
+  // its body.
+  int buf = 0, it = 0;
+  if (mine > 0) {
+    load_general(stage_of(0) * BK);
+    store_tiles(0);
+  }
+  __syncthreads();
+  if (g.fast && !g.maskA) {
+    // iterations whose next stage lies inside K, for every group
+    const int nfast = min(per, (int)(g.K / BK) - (WK - 1) * per) - 1;
+    for (; it < nfast; ++it) {
+      load_fast((int64_t)(st0 + it + 1) * BK);
+      multiply(buf);
+      store_tiles(buf ^ 1);
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+  for (; it < iters; ++it) {
+    const bool more = it + 1 < mine;
+    if (more) load_general(stage_of(it + 1) * BK);
+    if (it < mine) multiply(buf);
     if (more) store_tiles(buf ^ 1);
     __syncthreads();
     buf ^= 1;
+  }
+  if constexpr (WK > 1) {
+    // groups 1 .. WK - 1 hand their sums to group 0 through the stage buffers (one
+    // row of tiles at a time), group 0 adds them in order and stores the tile
+    constexpr int ROW = TN * 4 * 256;
+    static_assert((WK - 1) * ROW * sizeof(Tc) <= sizeof(stage_mem), "sums fit the stage buffers");
+    Tc* pool = (Tc*)&stage_mem[0];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if (grp > 0) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            pool[(grp - 1) * ROW + (j * 4 + v) * 256 + tid] = acc[i][j][v];
+      }
+      __syncthreads();
+      if (grp == 0) {
+#pragma unroll
+        for (int w = 1; w < WK; ++w)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              acc[i][j][v] += pool[(w - 1) * ROW + (j * 4 + v) * 256 + tid];
+      }
+      __syncthreads();
+    }
+    if (grp > 0) return;
   }
 
   // epilogue: lane holds the real (pb = 0) or imaginary (pb = 1) part of
@@ -294,20 +396,20 @@ __global__ __launch_bounds__(256) void zgemm_kernel(GemmKArgs g) {
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      Tc mine[4], other[4];
+      Tc mine_[4], other[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        mine[v] = acc[i][j][v];
-        other[v] = __shfl_xor(mine[v], 1);
+        mine_[v] = acc[i][j][v];
+        other[v] = __shfl_xor(mine_[v], 1);
       }
-      const int64_t n = n0 + wn0 + 8 * j + ((lane & 15) >> 1);
+      const int64_t n = n0 + wn0 + 8 * j + (l16 >> 1);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         // constant register indices only (a lane-dependent index would force scratch)
         const int v = 2 * pb + h;
         const int64_t m = m0 + wm0 + 16 * i + acc4<Tc>::row(kk, v);
-        double re = pb ? (double)other[2 + h] : (double)mine[h];
-        double im = pb ? (double)mine[2 + h] : (double)other[h];
+        double re = pb ? (double)other[2 + h] : (double)mine_[h];
+        double im = pb ? (double)mine_[2 + h] : (double)other[h];
         if (m < g.M && n < g.N) {
           TC* p = C + m * g.c_m + n * g.c_n;
           if (g.accumulate) {
@@ -319,6 +421,121 @@ __global__ __launch_bounds__(256) void zgemm_kernel(GemmKArgs g) {
         }
       }
     }
+  }
+}
+
+// The smallest products. A workgroup of WK waves owns 16 rows x (8*TN) complex
+// columns and every wave takes its part of k: a product of a few thousand
+// outputs then reaches all CUs, which the 2 x 2-wave tiles above do not (64 x 256
+// outputs are 8 workgroups of 64 x 32), and its chain of dependent MFMAs is
+// K / (4 WK) steps long. A lane loads the complex elements that it feeds to the
+// MFMAs straight from global memory (16 rows x 4 k of A, 4 k x 8 columns of B per
+// step: whole 64- or 128-byte runs in either order of the operands), U steps
+// ahead of their use; there is no staging and no barrier in the loop. The WK
+// partial tiles are added in the order of the waves through LDS.
+template <int TN_> struct WaveTile {
+  static constexpr int TN = TN_;
+  static constexpr int BM = 16;
+  static constexpr int BN = 8 * TN_;
+};
+template <typename Tc, typename TA, typename TB, typename TC, typename Tile, int WK,
+          bool A_KCONTIG, bool B_NCONTIG>
+__global__ __launch_bounds__(64 * WK) void zgemm_kernel(GemmKArgs g) {
+  constexpr int TN = Tile::TN, BM = Tile::BM, BN = Tile::BN;
+  constexpr int U = 4;                       // steps per batch of loads
+  typedef typename acc4<Tc>::type acc_t;
+  typedef typename cplx_of<Tc>::type C2;
+  __shared__ __align__(16) Tc red[WK][TN * 4][64];
+  if (g.skip && g.skip[blockIdx.z * g.skip_stride]) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, kk = lane >> 4, pb = lane & 1;
+  int tm, tn;
+  tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
+  const int64_t bz = blockIdx.z;
+  const Tc sa = g.conjA ? (Tc)-1 : (Tc)1;
+  const Tc sb = g.conjB ? (Tc)-1 : (Tc)1;
+  const TA* __restrict__ A = (const TA*)g.A + bz * g.bz_a + min(m0 + l16, g.M - 1) * g.a_m;
+  const TB* __restrict__ B[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+    B[j] = (const TB*)g.B + bz * g.bz_b + min(n0 + 8 * j + (l16 >> 1), g.N - 1) * g.b_n;
+  // steps of four k; this wave's are [s0, s1)
+  const int nstep = (int)((g.K + 3) / 4);
+  const int per = (nstep + WK - 1) / WK;
+  const int s0 = wave * per, s1 = min(s0 + per, nstep);
+
+  acc_t acc[TN][2];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) acc[j][0] = acc[j][1] = acc_t{0, 0, 0, 0};
+  struct Batch {
+    C2 a[U], b[U][TN];
+  };
+  // steps s .. s + U - 1, k clamped to the last one; a step beyond s1 is not used
+  auto load = [&](int s, Batch& q) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t k = min((int64_t)4 * (s + u) + kk, g.K - 1);
+      load_c<Tc>(A + k * g.a_k, q.a[u].x, q.a[u].y);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) load_c<Tc>(B[j] + k * g.b_k, q.b[u][j].x, q.b[u][j].y);
+    }
+  };
+  auto multiply = [&](int s, const Batch& q) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s + u < s1) {
+        const bool in = (int64_t)4 * (s + u) + kk < g.K;
+        const Tc ar = in ? q.a[u].x : Tc(0), ai = in ? sa * q.a[u].y : Tc(0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const Tc br = in ? q.b[u][j].x : Tc(0), bi = in ? sb * q.b[u][j].y : Tc(0);
+          acc[j][0] = mfma16(ar, pb ? bi : br, acc[j][0]);
+          acc[j][1] = mfma16(ai, pb ? br : -bi, acc[j][1]);
+        }
+      }
+    }
+  };
+  if (s0 < s1) {
+    Batch q0, q1;
+    load(s0, q0);
+    for (int s = s0; s < s1; s += 2 * U) {
+      load(s + U, q1);
+      multiply(s, q0);
+      if (s + U < s1) {
+        load(s + 2 * U, q0);
+        multiply(s + U, q1);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][j * 4 + v][lane] = acc[j][0][v] + acc[j][1][v];
+  __syncthreads();
+  // one complex output per thread: its real part sits in an even lane of the
+  // result layout, the imaginary part in the next one
+  TC* __restrict__ C = (TC*)g.C + bz * g.bz_c;
+  for (int e = threadIdx.x; e < BM * BN; e += 64 * WK) {
+    const int r = e / BN, c = e % BN;
+    const int64_t m = m0 + r, n = n0 + c;
+    if (m >= g.M || n >= g.N) continue;
+    const int src = acc4<Tc>::group(r) * 16 + 2 * (c & 7);
+    const int slot = (c >> 3) * 4 + acc4<Tc>::elem(r);
+    double re = 0, im = 0;
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      re += (double)red[w][slot][src];
+      im += (double)red[w][slot][src + 1];
+    }
+    TC* p = C + m * g.c_m + n * g.c_n;
+    if (g.accumulate) {
+      double pr, pi;
+      load_c<double>(p, pr, pi);
+      re += pr;
+      im += pi;
+    }
+    store_c(p, re, im);
   }
 }
 
@@ -334,17 +551,21 @@ inline double gemm_bytes(const ZGemm& z) {
 }
 // kernel instance name as a profiler lists it (template arguments, without
 // the namespace and the argument list), e.g.
-// zgemm_kernel<float, c64, c64, c128, 4, 8, true, true>
-template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN>
+// zgemm_kernel<float, c64, c64, c128, 4, 8, 1, true, true> (TM = 0: the wave tile)
+template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, int WK = 1>
 inline const char* gemm_kernel_name(bool ak, bool bn, const char* kernel = "zgemm_kernel") {
   static std::mutex mu;
   static std::unordered_map<std::string, std::string> names;
   char buf[160];
-  // the split-bf16 kernel has no compute-type argument
+  // the split-bf16 kernel has no compute-type and no k-group argument
   const bool with_tc = strcmp(kernel, "zgemm_kernel") == 0;
-  snprintf(buf, sizeof(buf), "%s<%s%s%s, %s, %s, %d, %d, %s, %s>", kernel,
+  char tile[32], wk[16] = "";
+  if (TM > 0) snprintf(tile, sizeof(tile), "%d, %d", TM, TN);
+  else snprintf(tile, sizeof(tile), "WaveTile<%d>", TN);
+  if (with_tc) snprintf(wk, sizeof(wk), "%d, ", WK);
+  snprintf(buf, sizeof(buf), "%s<%s%s%s, %s, %s, %s, %s%s, %s>", kernel,
            with_tc ? type_tag<Tc>::s : "", with_tc ? ", " : "", type_tag<TA>::s,
-           type_tag<TB>::s, type_tag<TC>::s, TM, TN, ak ? "true" : "false",
+           type_tag<TB>::s, type_tag<TC>::s, tile, wk, ak ? "true" : "false",
            bn ? "true" : "false");
   std::lock_guard<std::mutex> lk(mu);
   auto it = names.find(buf);
@@ -363,7 +584,9 @@ inline int build_masks(const ZGemm& z, GemmKArgs& g, int BM, int BN, int BK, voi
   if (nk > MAX_MASKED_STAGES) return PTN_OK;   // dense product (correct, no skipping)
   const int words = (int)((nk + 63) / 64);
   const size_t need = (size_t)((int64_t)g.tiles_m + g.tiles_n) * words * 8;
-  if (mws_bytes < need) return PTN_ERR_WORKSPACE;
+  // the workspace is sized for 64 x 32 tiles; the masks of a short product on smaller
+  // tiles may not fit it: no skipping then, the result is the same
+  if (mws_bytes < need) return PTN_OK;
   uint64_t* ma = (uint64_t*)mws;
   uint64_t* mb = ma + (int64_t)g.tiles_m * words;
   tile_mask_kernel<TA><<<dim3((unsigned)g.tiles_m, (unsigned)words), 256, 0, s>>>(
@@ -375,70 +598,157 @@ inline int build_masks(const ZGemm& z, GemmKArgs& g, int BM, int BN, int BK, voi
   return PTN_OK;
 }
 
-template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN>
-inline int launch_cfg(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t mws_bytes = 0) {
-  typedef TileCfg<TM, TN, StageK<Tc>::value> T;
-  GemmKArgs g;
+// kernel arguments of a product on BM x BN tiles; false if the grid is too large
+inline bool fill_args(const ZGemm& z, GemmKArgs& g, int BM, int BN) {
   g.M = z.M; g.N = z.N; g.K = z.K;
   g.A = z.A; g.a_m = z.a_m; g.a_k = z.a_k; g.conjA = z.conjA;
   g.B = z.B; g.b_k = z.b_k; g.b_n = z.b_n; g.conjB = z.conjB;
   g.C = z.C; g.c_m = z.c_m; g.c_n = z.c_n;
   g.accumulate = z.accumulate;
   g.bz_a = z.bz_a; g.bz_b = z.bz_b; g.bz_c = z.bz_c;
-  g.tiles_m = (int)((z.M + T::BM - 1) / T::BM);
-  g.tiles_n = (int)((z.N + T::BN - 1) / T::BN);
+  g.tiles_m = (int)((z.M + BM - 1) / BM);
+  g.tiles_n = (int)((z.N + BN - 1) / BN);
+  g.maskA = nullptr; g.maskB = nullptr; g.mwords = 0;
   g.skip = skip_flag().p;
   g.skip_stride = skip_flag().stride;
-  int64_t nwg = (int64_t)g.tiles_m * g.tiles_n;
-  if (nwg > 0x7fffffff || z.batch > 65535) return PTN_ERR_ARG;
+  g.fast = 0;
+  return (int64_t)g.tiles_m * g.tiles_n <= 0x7fffffff && z.batch <= 65535;
+}
+
+// launch of the kernel instance for the operands' contiguity: a K-contiguous A
+// when its k stride is 1 (or K == 1), else M-contiguous; B alike
+#define PTN_GEMM_LAUNCH(nm, z, g, s, threads, ...)                                              \
+  do {                                                                                          \
+    const bool ak_ = (z.a_k == 1) || (z.a_m != 1), bn_ = (z.b_n == 1) || (z.b_k != 1);          \
+    const dim3 grid_((unsigned)((int64_t)g.tiles_m * g.tiles_n), 1, (unsigned)z.batch);         \
+    const double fl_ = gemm_flop(z), by_ = gemm_bytes<TA, TB, TC>(z);                           \
+    if (ak_ && bn_)                                                                             \
+      tlaunch(nm(true, true), fl_, by_, zgemm_kernel<Tc, TA, TB, TC, __VA_ARGS__, true, true>,  \
+              grid_, dim3(threads), s, g);                                                      \
+    else if (ak_)                                                                               \
+      tlaunch(nm(true, false), fl_, by_,                                                        \
+              zgemm_kernel<Tc, TA, TB, TC, __VA_ARGS__, true, false>, grid_, dim3(threads), s,  \
+              g);                                                                               \
+    else if (bn_)                                                                               \
+      tlaunch(nm(false, true), fl_, by_,                                                        \
+              zgemm_kernel<Tc, TA, TB, TC, __VA_ARGS__, false, true>, grid_, dim3(threads), s,  \
+              g);                                                                               \
+    else if constexpr (sizeof(Tc) == 8)                                                         \
+      tlaunch(nm(false, false), fl_, by_,                                                       \
+              zgemm_kernel<Tc, TA, TB, TC, __VA_ARGS__, false, false>, grid_, dim3(threads), s, \
+              g);                                                                               \
+    else                                                                                        \
+      return PTN_ERR_UNSUPPORTED;   /* no reduced-precision product has this layout */          \
+    PTN_LAUNCH_CHECK();                                                                         \
+    return PTN_OK;                                                                              \
+  } while (0)
+
+template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, int WK = 1>
+inline int launch_cfg(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t mws_bytes = 0) {
+  typedef TileCfg<TM, TN, StageK<Tc, TM>::value> T;
+  GemmKArgs g;
+  if (!fill_args(z, g, T::BM, T::BN)) return PTN_ERR_ARG;
+  const int64_t lim = (int64_t)1 << 31;   // non-negative strides with offsets below 2 GiB
+  g.fast = z.a_m >= 0 && z.a_k >= 0 && z.b_k >= 0 && z.b_n >= 0 && z.a_m < lim && z.a_k < lim &&
+           z.b_k < lim && z.b_n < lim &&
+           (T::BM * z.a_m + T::BK * z.a_k) * (int64_t)sizeof(TA) < lim &&
+           (T::BN * z.b_n + T::BK * z.b_k) * (int64_t)sizeof(TB) < lim;
   int st = build_masks<TA, TB>(z, g, T::BM, T::BN, T::BK, mws, mws_bytes, s);
   if (st) return st;
-  dim3 grid((unsigned)nwg, 1, (unsigned)z.batch);
-  // a K-contiguous A when its k stride is 1 (or K == 1), else M-contiguous
-  const bool ak = (z.a_k == 1) || (z.a_m != 1);
-  const bool bn = (z.b_n == 1) || (z.b_k != 1);
-  const char* nm = gemm_kernel_name<Tc, TA, TB, TC, TM, TN>(ak, bn);
-  const double fl = gemm_flop(z), by = gemm_bytes<TA, TB, TC>(z);
-  if (ak && bn)
-    tlaunch(nm, fl, by, zgemm_kernel<Tc, TA, TB, TC, TM, TN, true, true>, grid, dim3(256), s, g);
-  else if (ak && !bn)
-    tlaunch(nm, fl, by, zgemm_kernel<Tc, TA, TB, TC, TM, TN, true, false>, grid, dim3(256), s, g);
-  else if (!ak && bn)
-    tlaunch(nm, fl, by, zgemm_kernel<Tc, TA, TB, TC, TM, TN, false, true>, grid, dim3(256), s, g);
-  else
-    tlaunch(nm, fl, by, zgemm_kernel<Tc, TA, TB, TC, TM, TN, false, false>, grid, dim3(256), s, g);
-  PTN_LAUNCH_CHECK();
-  return PTN_OK;
+  auto nm = [](bool ak, bool bn) {   // formatted once per instance
+    static const char* const n[4] = {gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(false, false),
+                                     gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(false, true),
+                                     gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(true, false),
+                                     gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(true, true)};
+    return n[2 * ak + bn];
+  };
+  PTN_GEMM_LAUNCH(nm, z, g, s, 256 * WK, TM, TN, WK);
+}
+
+// the wave-tile kernel for the smallest products
+template <typename Tc, typename TA, typename TB, typename TC, int TN, int WK>
+inline int launch_wave(const ZGemm& z, hipStream_t s) {
+  typedef WaveTile<TN> T;
+  GemmKArgs g;
+  if (!fill_args(z, g, T::BM, T::BN)) return PTN_ERR_ARG;
+  auto nm = [](bool ak, bool bn) {
+    static const char* const n[4] = {gemm_kernel_name<Tc, TA, TB, TC, 0, TN, WK>(false, false),
+                                     gemm_kernel_name<Tc, TA, TB, TC, 0, TN, WK>(false, true),
+                                     gemm_kernel_name<Tc, TA, TB, TC, 0, TN, WK>(true, false),
+                                     gemm_kernel_name<Tc, TA, TB, TC, 0, TN, WK>(true, true)};
+    return n[2 * ak + bn];
+  };
+  PTN_GEMM_LAUNCH(nm, z, g, s, 64 * WK, T, WK);
 }
 
 // opt-in autotuning of the tile shape (ptn_set_autotune): set once per process
 bool autotune_enabled();
 
-// tile choice: the large tile (128 x 64 complex) when it still gives at least
-// two workgroups per CU, else the small one (64 x 32)
+// Tile choice, from the times of every configuration over shapes M, N, K = 16 ..
+// 5120 (FP64 figures, us or TFLOP/s at M x N x K):
+//  * at most 320 outputs tiles of 16 x 8: one wave tile per CU or so. The product is
+//    latency-bound and the wave kernel is the shortest chain (64 x 256 x 320: 6.0 us
+//    against 11.3 of the next best; 128 x 256 x 640: 9.1 against 18.5; equal at
+//    200 x 400 x 1000 = 650 tiles); below K = 192 four waves have work enough.
+//  * large tiles (128 x 64; FP32 also 128 x 128) where their number fills whole waves
+//    of two workgroups per CU: full waves 65.4 TFLOP/s against 63.0 of 64 x 32 tiles
+//    (1024 x 4096 x 5120), but 53.6 against 62.3 with 640 tiles in 512 slots
+//    (5120 x 1024 x 2048). FP32: 128 x 128 down to 0.8 of a wave's slots.
+//  * 64 x 32 tiles from 192 up. Fewer than about two per CU leave the matrix cores
+//    waiting for operands: then k is split over two or four groups of the workgroup
+//    (256 tiles, 512 x 1024 x 2560: 44.4 / 49.6 / 55.0 TFLOP/s with 1 / 2 / 4 groups;
+//    1280 tiles, 1024 x 2560 x 512: 59.0 / 55.9 / 51.2).
+//  * tile-skipping products (mask workspace given) never take the large tiles: the
+//    small one skips the zero blocks of sector-structured operands at finer
+//    granularity, which outweighs its lower efficiency per flop (U(1) two-site DMRG
+//    at L=128, D=2048: 76 s against 82 s per sweep). The split of k is that of the
+//    unmasked product, so both add in the same order.
+//  * 32 x 16 tiles for fewer, or where 64-row tiles would be a third padding (the
+//    32-row products of the blocked QR, 32 x 1984 x 248 x 8: 27.8 us against 42.2).
+inline double wave_fill(int64_t tiles, int64_t slots) {
+  return (double)tiles / (double)((tiles + slots - 1) / slots * slots);
+}
+inline int64_t tiles_of(const ZGemm& z, int BM, int BN) {
+  return ((z.M + BM - 1) / BM) * ((z.N + BN - 1) / BN) * z.batch;
+}
+inline bool wave_tile_product(const ZGemm& z) { return tiles_of(z, 16, 8) <= 320; }
+
 template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_heuristic(const ZGemm& z, hipStream_t s, void* mws, size_t mws_bytes) {
-  // FP32: 128 x 128 complex tiles (half the operand bytes per flop of 128 x 64)
-  // when they still give two workgroups per CU
-  if constexpr (sizeof(Tc) == 4) {
-    int64_t wide = ((z.M + 127) / 128) * ((z.N + 127) / 128) * z.batch;
-    if (wide >= 512) return launch_cfg<Tc, TA, TB, TC, 4, 8>(z, s, mws, mws_bytes);
+  if (wave_tile_product(z)) {
+    if (z.K >= 192) return launch_wave<Tc, TA, TB, TC, 1, 8>(z, s);
+    return launch_wave<Tc, TA, TB, TC, 1, 4>(z, s);
   }
-  int64_t big = ((z.M + 127) / 128) * ((z.N + 63) / 64) * z.batch;
-  if (big >= 512) return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s, mws, mws_bytes);
-  return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
+  const bool masked = mws && z.batch == 1;
+  if constexpr (sizeof(Tc) == 4) {
+    const int64_t wide = tiles_of(z, 128, 128);
+    if (!masked && wide >= 512 && wave_fill(wide, 512) >= 0.8)
+      return launch_cfg<Tc, TA, TB, TC, 4, 8>(z, s);
+  }
+  const int64_t t44 = tiles_of(z, 128, 64), t22 = tiles_of(z, 64, 32), t11 = tiles_of(z, 32, 16);
+  if (!masked && t44 >= 512 && wave_fill(t44, 512) >= 0.95)
+    return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s);
+  if (t22 >= 192 && 3 * t22 <= t11) {   // t11 / t22 is 4 without padding
+    if (t22 >= 600 || z.K < 64) return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
+    if (z.K < 256) return launch_cfg<Tc, TA, TB, TC, 2, 2, 2>(z, s, mws, mws_bytes);
+    return launch_cfg<Tc, TA, TB, TC, 2, 2, 4>(z, s, mws, mws_bytes);
+  }
+  if (z.K < 64 || t11 >= 512) return launch_cfg<Tc, TA, TB, TC, 1, 1>(z, s, mws, mws_bytes);
+  if (z.K < 256) return launch_cfg<Tc, TA, TB, TC, 1, 1, 2>(z, s, mws, mws_bytes);
+  return launch_cfg<Tc, TA, TB, TC, 1, 1, 4>(z, s, mws, mws_bytes);
 }
 
 template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_choice(int c, const ZGemm& z, hipStream_t s) {
-  if (c == 0) return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s);
-  if (c == 1) return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s);
+  if (c == 0) return launch_heuristic<Tc, TA, TB, TC>(z, s, nullptr, 0);
+  if (c == 1) return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s);
+  if (c == 2) return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s);
   if constexpr (sizeof(Tc) == 4) return launch_cfg<Tc, TA, TB, TC, 4, 8>(z, s);
   return PTN_ERR_ARG;
 }
 
 // Tile autotuner: the first product of a given shape (M, N, K, batch and the
-// contiguity of the operands) times every tile configuration (two timed
+// contiguity of the operands) times the rule's choice and the other large tiles (two timed
 // launches each after one untimed, HIP events on the caller's stream) and
 // keeps the fastest for that shape. Only products that overwrite C are tuned
 // (a repeated launch then leaves the same result); the tuning launch of the
@@ -467,7 +777,7 @@ inline int launch_tuned(const ZGemm& z, hipStream_t s) {
     auto it = best.find(key);
     if (it != best.end()) return launch_choice<Tc, TA, TB, TC>(it->second, z, s);
   }
-  const int nc = sizeof(Tc) == 4 ? 3 : 2;
+  const int nc = sizeof(Tc) == 4 ? 4 : 3;
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess) return PTN_ERR_HIP;
   if (hipEventCreate(&e1) != hipSuccess) { (void)hipEventDestroy(e0); return PTN_ERR_HIP; }
@@ -497,12 +807,9 @@ inline int launch_tuned(const ZGemm& z, hipStream_t s) {
 
 template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_typed(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t mws_bytes = 0) {
-  // tile-skipping products (mask workspace given): the small tile skips the
-  // zero blocks of sector-structured operands at finer granularity, which
-  // outweighs its lower efficiency per flop (U(1) two-site DMRG at L=128,
-  // D=2048: 76 s against 82 s per sweep)
-  if (mws && z.batch == 1) return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
-  if (!z.accumulate && autotune_enabled() && !noalloc_mode()) {
+  if (mws && z.batch == 1) return launch_heuristic<Tc, TA, TB, TC>(z, s, mws, mws_bytes);
+  // (the wave tile is not in question for the products that the rule gives it)
+  if (!z.accumulate && autotune_enabled() && !noalloc_mode() && !wave_tile_product(z)) {
     // tuning synchronises the stream, which a stream capture does not allow
     hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cst) == hipSuccess && cst == hipStreamCaptureStatusNone)

@@ -75,7 +75,7 @@ struct GLaunch {
 template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, bool A_KCONTIG,
           bool B_NCONTIG>
 __global__ __launch_bounds__(256) void zgemm_grouped_kernel(GLaunch g) {
-  typedef TileCfg<TM, TN, StageK<Tc>::value> T;
+  typedef TileCfg<TM, TN, StageK<Tc, TM>::value> T;
   constexpr int BM = T::BM, BN = T::BN, BK = T::BK, NA = T::NA, NB = T::NB;
   typedef typename acc4<Tc>::type acc_t;
   __shared__ Tc As[2][2 * BK][BM + 1];
