@@ -127,8 +127,10 @@ int zgemm(const ZGemm& g, int compute, int ta, int tb, int tc,
           void* ws, size_t ws_bytes, hipStream_t s);
 
 // Y[l, o, r] = sum_i Wm[o, i] X[l, i, r]   (complex; Wm complex128 on device);
-// `batch` independent problems with contiguous X and Y and Wm stride bw
+// `batch` independent problems with contiguous X and Y and Wm stride bw;
+// wtrans: Wm is stored transposed, as [i][o]
 int mode_mix(int64_t nl, int64_t ni, int64_t no, int64_t nr, const void* wm, const void* x, int tx,
-             void* y, int ty, hipStream_t s, int64_t batch = 1, int64_t bw = 0);
+             void* y, int ty, hipStream_t s, int64_t batch = 1, int64_t bw = 0,
+             bool wtrans = false);
 
 }  // namespace ptn

@@ -25,19 +25,6 @@ static inline size_t csize(int prec) { return prec == PTN_FP64 ? 16 : 8; }
 static inline int ctype(int prec) { return prec == PTN_FP64 ? PTN_T_C128 : PTN_T_C64; }
 static inline int gemm_compute(int prec) { return prec; }
 
-// ---------------------------------------------------------------------------
-// W (Ml, d, d, Mr) viewed as the matrix Wmat[(m, sb), (s, m')]; the left
-// environment needs its transpose Wt[(s, m'), (m, sb)].
-__global__ void transpose_w_kernel(int64_t rows, int64_t cols, const double2* __restrict__ w,
-                                   double2* __restrict__ wt) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= rows * cols) return;
-  w += blockIdx.y * rows * cols;     // problem of a batch
-  wt += blockIdx.y * rows * cols;
-  int64_t i = t / cols, j = t % cols;
-  wt[j * rows + i] = w[t];
-}
-
 __global__ void convert_c128_c64_kernel(int64_t n, const double2* __restrict__ x,
                                         float2* __restrict__ y) {
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
@@ -94,15 +81,14 @@ size_t heff_ws_bytes(int prec, const Dims& D, int64_t batch) {
 size_t env_ws_bytes(int prec, const Dims& D, int64_t batch) {
   prec = base_prec(prec);
   // right step: T1 (Dl*d, Mr*Dr), T2 (Dl*Ml, d*Dr); left step: T1 (Dl*Ml, d*Dr),
-  // T2 (Dl*d, Mr*Dr); plus the transposed MPO tensor
+  // T2 (Dl*d, Mr*Dr)
   size_t a = (size_t)batch * (size_t)(D.Dl * D.d) * (size_t)(D.Mr * D.Dr) * csize(prec);
   size_t b = (size_t)batch * (size_t)(D.Dl * D.Ml) * (size_t)(D.d * D.Dr) * csize(prec);
-  size_t wt = (size_t)batch * (size_t)(D.Ml * D.d * D.d * D.Mr) * 16;
   const size_t mr = mask_bytes2(D.Dl * D.d, D.Mr * D.Dr, D.Dr, D.Dl * D.Ml, D.Dl, D.d * D.Dr);
   const size_t ml = mask_bytes2(D.Dl * D.Ml, D.d * D.Dr, D.Dl, D.Dr, D.Mr * D.Dr, D.Dl * D.d);
   const size_t sr = split2(prec, batch, D.Dl * D.d, D.Mr * D.Dr, D.Dr, D.Dl * D.Ml, D.Dl, D.d * D.Dr);
   const size_t sl = split2(prec, batch, D.Dl * D.Ml, D.d * D.Dr, D.Dl, D.Dr, D.Mr * D.Dr, D.Dl * D.d);
-  return 2 * align256(a > b ? a : b) + align256(wt) + (mr > ml ? mr : ml) + 256 +
+  return 2 * align256(a > b ? a : b) + (mr > ml ? mr : ml) + 256 +
          (sr > sl ? sr : sl);
 }
 
@@ -187,9 +173,8 @@ int env_right(int prec, const Dims& D, const void* a, const void* b, const void*
   void* t1 = p;
   p += align256(ta > tb ? ta : tb);
   void* t2 = p;
-  const size_t wtb = align256((size_t)batch * (size_t)(D.Ml * D.d * D.d * D.Mr) * 16);
   const size_t mb = mask_bytes2(D.Dl * D.d, D.Mr * D.Dr, D.Dr, D.Dl * D.Ml, D.Dl, D.d * D.Dr);
-  void* mws = sp ? (char*)ws + 2 * align256(ta > tb ? ta : tb) + wtb : nullptr;
+  void* mws = sp ? (char*)ws + 2 * align256(ta > tb ? ta : tb) : nullptr;
   const int64_t nA = D.Dl * D.d * D.Dr, nR = D.Dr * D.Mr * D.Dr, nO = D.Dl * D.Ml * D.Dl;
   int st;
   ZGemm g1 = {D.Dl * D.d, D.Mr * D.Dr, D.Dr,
@@ -226,15 +211,9 @@ int env_left(int prec, const Dims& D, const void* a, const void* b, const void* 
   char* p = (char*)ws;
   void* t1 = p;
   void* t2 = p + big;
-  void* wt = p + 2 * big;
   const int64_t nW = D.Ml * D.d * D.d * D.Mr;
-  const size_t wtb = align256((size_t)batch * (size_t)nW * 16);
   const size_t mb = mask_bytes2(D.Dl * D.Ml, D.d * D.Dr, D.Dl, D.Dr, D.Mr * D.Dr, D.Dl * D.d);
-  void* mws = sp ? p + 2 * big + wtb : nullptr;
-  int64_t rows = D.Ml * D.d, cols = D.d * D.Mr;
-  transpose_w_kernel<<<dim3((unsigned)((rows * cols + 255) / 256), (unsigned)batch), 256, 0, s>>>(
-      rows, cols, (const double2*)w, (double2*)wt);
-  PTN_LAUNCH_CHECK();
+  void* mws = sp ? p + 2 * big : nullptr;
   const int64_t nA = D.Dl * D.d * D.Dr, nL = D.Dl * D.Ml * D.Dl, nO = D.Dr * D.Mr * D.Dr;
   int st;
   // T1[(l, m), (sb, rb)] = sum_lb L[(l, m), lb] conj(B[lb, (sb, rb)])
@@ -243,8 +222,9 @@ int env_left(int prec, const Dims& D, const void* a, const void* b, const void* 
               b, D.d * D.Dr, 1, 1,
               t1, D.d * D.Dr, 1, 0, batch, nL, nA, n1, sws, spb};
   if ((st = zgemm(g1, cp, tl, PTN_T_C128, ct, mws, mb, s))) return st;
-  // T2[l, (s, m'), rb] = sum_{(m, sb)} W[m, sb, s, m'] T1[l, (m, sb), rb]
-  if ((st = mode_mix(D.Dl, D.Ml * D.d, D.d * D.Mr, D.Dr, wt, t1, ct, t2, ct, s, batch, nW)))
+  // T2[l, (s, m'), rb] = sum_{(m, sb)} W[m, sb, s, m'] T1[l, (m, sb), rb]: the mix
+  // with W read as the transpose of Wmat[(m, sb), (s, m')]
+  if ((st = mode_mix(D.Dl, D.Ml * D.d, D.d * D.Mr, D.Dr, w, t1, ct, t2, ct, s, batch, nW, true)))
     return st;
   // out[r, (m', rb)] = sum_{(l, s)} A[(l, s), r] T2[(l, s), (m', rb)]
   ZGemm g3 = {D.Dr, D.Mr * D.Dr, D.Dl * D.d,

@@ -92,3 +92,21 @@ def test_fp32_contractions_over_the_tile_rules(Dl, Dr, d):
     ref = orc.apply_local_hamiltonian(a, w, l, r)
     got = backend.to_host(backend.heff_apply(a, w, l, r, "fp32"))
     assert np.abs(got - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("Dl,Dr,d,Ml,Mr", [(1, 1, 2, 1, 1), (3, 15, 2, 5, 5), (7, 16, 2, 3, 5),
+                                           (5, 17, 2, 5, 4), (4, 32, 4, 5, 5), (3, 33, 4, 8, 8),
+                                           (9, 64, 4, 4, 8), (2, 65, 3, 5, 10), (301, 517, 2, 5, 5)])
+def test_mode_mix_units(Dl, Dr, d, Ml, Mr):
+    """The mode mix at the edges of its column units (16, 32 and 64 columns, several
+    rows per unit, more units than workgroups), with the largest and smallest index
+    pairs, and read transposed (left environment); W mostly zero, as an MPO's."""
+    rng = np.random.default_rng(Dl * 1000 + Dr)
+    a, b = orc.crandn((Dl, d, Dr), rng), orc.crandn((Dl, d, Dr), rng)
+    w = orc.crandn((Ml, d, d, Mr), rng) * (rng.random((Ml, d, d, Mr)) < 0.2)
+    l, r = orc.crandn((Dl, Ml, Dl), rng), orc.crandn((Dr, Mr, Dr), rng)
+    for got, ref in ((backend.heff_apply(a, w, l, r), orc.apply_local_hamiltonian(a, w, l, r)),
+                     (backend.env_left(a, b, w, l), orc.contraction_operator_step_left(a, b, w, l)),
+                     (backend.env_right(a, b, w, r),
+                      orc.contraction_operator_step_right(a, b, w, r))):
+        assert np.abs(backend.to_host(got) - ref).max() <= 1e-12 * max(np.abs(ref).max(), 1e-300)
