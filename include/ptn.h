@@ -266,8 +266,8 @@ int ptn_svd(int64_t m, int64_t n, const void* a, int64_t lda, void* u, int64_t l
  * Only the isometric factor's singular vectors are computed (one-sided Jacobi
  * on the QR-preconditioned matrix without accumulating the rotations); the
  * other factor is the projection of Theta onto them (one product).
- * precond32 != 0 starts the Jacobi iteration with FP32 sweeps (the FP64 output
- * accuracy is kept). The call synchronises the stream (k sizes the outputs).
+ * precond32 is accepted and changes nothing: without accumulated rotations the
+ * FP64 sweeps cost less than FP32 ones before them. The call synchronises the stream (k sizes the outputs).
  * Returns PTN_ERR_NONFINITE when a singular value is not finite. */
 #define PTN_SPLIT_LEFT  0
 #define PTN_SPLIT_RIGHT 1

@@ -428,7 +428,8 @@ def svd_split(a, distr, tol=0.0, max_bond=None, precond32=False):
     (a0, a1, s) with distr "right": a0 = U_k, a1 = Sigma_k V_k^H; "left":
     a0 = U_k Sigma_k, a1 = V_k^H; s = all singular values (host, descending).
     k follows the reference's discarded-weight rule with `tol` (bond_ops.py:23-38)
-    and the cap `max_bond`. Synchronises the stream."""
+    and the cap `max_bond`. precond32 is accepted for both settings and changes
+    nothing (the FP64 sweeps are the faster ones here). Synchronises the stream."""
     a = as_dev(a)
     m, n = a.shape
     code = {"left": _lib.PTN_SPLIT_LEFT, "right": _lib.PTN_SPLIT_RIGHT}[distr]

@@ -10,9 +10,9 @@ size_t krylov_ws_bytes(const ptn_local_op* op, int numiter, int64_t batch);
 int krylov_run(const ptn_local_op* op, int mode, const void* v, double dt_re, double dt_im,
                int numiter, void* out, double* energy, int32_t* info, double* alpha_beta,
                void* ws, size_t ws_bytes, hipStream_t s, int64_t batch);
-size_t svd_split_ws_bytes(int64_t m, int64_t n, int distr, bool precond32);
+size_t svd_split_ws_bytes(int64_t m, int64_t n, int distr);
 int svd_split_run(int64_t m, int64_t n, const void* theta, int64_t lda, int distr, double tol,
-                  int64_t max_bond, bool precond32, void* a0, void* a1, double* s_host,
+                  int64_t max_bond, void* a0, void* a1, double* s_host,
                   int64_t* k_out, int32_t* info_host, void* ws, size_t ws_bytes, hipStream_t st);
 int krylov_expm_noalloc(const ptn_local_op* op, const void* v, double dt_re, double dt_im,
                         int numiter, void* out, int32_t* info, double* alpha_beta, hipStream_t s);
@@ -379,14 +379,17 @@ int ptn_svd(int64_t m, int64_t n, const void* a, int64_t lda, void* u, int64_t l
                  0, 0, 0, 0, false);
 }
 
+// the split runs FP64 sweeps with and without precond32 (see split_layout)
 size_t ptn_svd_split_workspace(int64_t m, int64_t n, int distr, int precond32) {
-  return svd_split_ws_bytes(m, n, distr, precond32 != 0);
+  (void)precond32;
+  return svd_split_ws_bytes(m, n, distr);
 }
 
 int ptn_svd_split(int64_t m, int64_t n, const void* theta, int64_t lda, int distr, double tol,
                   int64_t max_bond, int precond32, void* a0, void* a1, double* s_host,
                   int64_t* k_out, int32_t* info_host, void* ws, size_t ws_bytes, void* stream) {
-  return svd_split_run(m, n, theta, lda, distr, tol, max_bond, precond32 != 0, a0, a1, s_host,
+  (void)precond32;
+  return svd_split_run(m, n, theta, lda, distr, tol, max_bond, a0, a1, s_host,
                        k_out, info_host, ws, ws_bytes, (hipStream_t)stream);
 }
 

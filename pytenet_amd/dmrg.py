@@ -66,7 +66,7 @@ def dmrg_twosite(hamiltonian: MPO, psi: MPS, numsweeps: int, numiter_lanczos: in
                  tol_split: float = 0, precision: str = "fp64", max_bond=None,
                  svd_precond32=None):
     """Two-site DMRG (dmrg.py:96-178): returns the energy after each sweep.
-    svd_precond32: split SVD with FP32 Jacobi preconditioning sweeps (FP64
+    svd_precond32: block-sparse split SVD with FP32 Jacobi preconditioning sweeps (FP64
     output accuracy); None = on when precision is not "fp64"."""
     pre32 = (precision != "fp64") if svd_precond32 is None else bool(svd_precond32)
     nsites = hamiltonian.nsites

@@ -266,7 +266,7 @@ def mps_split_tensor_svd(a, qsite0, qsite1, qbonds_outer, svd_distr: str, tol=0,
     SVD with discarded-weight truncation; sigma multiplied into the left or right
     factor, or its square root into both (mps.py:538-568). Extensions: `max_bond`
     caps the new bond (None reproduces the reference); `svd_precond32` starts the
-    Jacobi SVD with FP32 sweeps (FP64 output accuracy)."""
+    Jacobi SVD of a block-sparse split with FP32 sweeps (FP64 output accuracy)."""
     host = _is_host(a)
     a = backend.as_dev(a)
     assert a.dim() == 3

@@ -9,9 +9,9 @@ reference-preserving defaults:
              contractions (Krylov scalars, QR and SVD stay FP64);
   max_bond:  bond-dimension cap for the two-site split (None = no cap, as
              in the reference);
-  svd_precond32: two-site split SVD with FP32 Jacobi preconditioning sweeps
-             finished in FP64 (same output accuracy); None = on when
-             precision is not "fp64".
+  svd_precond32: block-sparse two-site split SVD with FP32 Jacobi
+             preconditioning sweeps finished in FP64 (same output accuracy);
+             None = on when precision is not "fp64".
 
 Reference:
     J. Haegeman, C. Lubich, I. Oseledets, B. Vandereycken, F. Verstraete
