@@ -6,6 +6,7 @@ namespace ptn {
 
 constexpr int QR_NB = 32;       // panel width (columns per compact-WY block)
 constexpr int QR_SPLITK = 8;    // K chunks of the V^H C products
+constexpr int QR_VTV_PARTS = 8; // row segments of the V^H V products (at most)
 
 // Factorisation B = Q R of an m x n complex128 matrix, held in device workspace:
 //   W     column-major m x n; its strict upper triangle is that of R

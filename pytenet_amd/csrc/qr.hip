@@ -9,10 +9,12 @@
 //
 // Blocked right-looking algorithm on a column-major copy (panels of QR_NB
 // columns):
-//   panel:    for each pair of columns j, j+1 one launch (k_qr_col2) computes
-//             reflectors j and j+1 in every workgroup (the same deterministic
-//             reductions) and applies them to one remaining column of the panel
-//             per workgroup (k_qr_col for a last odd column);
+//   panel:    up to 256 rows one workgroup with the panel in its registers
+//             (k_qr_panel); up to 2048 rows one launch for every four columns
+//             (k_qr_col4) and above for every two (k_qr_col2r, k_qr_col2; k_qr_col
+//             for a last odd column): every workgroup computes the launch's
+//             reflectors (the same deterministic reductions) and applies them to
+//             one remaining column of the panel;
 //   WY form:  T from V^H V (k_qr_vtv, k_qr_tmat), H_j0 ... = I - V T V^H;
 //   trailing: A <- A - V (T^H (V^H A)): V^H A as a split-K complex product on
 //             MFMA, the sum of the K chunks and the small T^H product in
@@ -24,10 +26,63 @@
 
 namespace ptn {
 
+// sum over the wave, in every lane: rotations inside the rows of 16 lanes (DPP), then the
+// four row sums read as scalars (an exchange through LDS per step takes several
+// times as long)
+template <int CTRL> __device__ __forceinline__ double dpp_rot(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
 __device__ __forceinline__ double wave_sum(double v) {
+  v += dpp_rot<0x128>(v);   // row rotate right by 8, 4, 2, 1
+  v += dpp_rot<0x124>(v);
+  v += dpp_rot<0x122>(v);
+  v += dpp_rot<0x121>(v);
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+// Eight sums over the wave at once: two values fold into one register per step (the
+// halves of the wave, then the rows of 16, then of 8 lanes keep one each and add the
+// other's partner), so the eight cost little more than one. Lane group g = lane / 8
+// ends with the sum of value sum8_slot(g).
+__device__ __forceinline__ int sum8_slot(int g) { return (g >> 2) | (g & 2) | ((g & 1) << 2); }
+template <bool HALF> __device__ __forceinline__ double swap_add(double a, double b) {
+  typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a),
+                           y = (unsigned long long)__double_as_longlong(b);
+  u2 lo, hi;
+  if constexpr (HALF) {
+    lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  } else {
+    lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  }
+  const double p = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
+  const double q = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+  return p + q;
+}
+__device__ __forceinline__ double wave_sum8(const double (&v)[8]) {
+  double a[4];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  for (int k = 0; k < 4; ++k) a[k] = swap_add<true>(v[2 * k], v[2 * k + 1]);
+  const double b0 = swap_add<false>(a[0], a[1]), b1 = swap_add<false>(a[2], a[3]);
+  const bool upper = (threadIdx.x & 8) != 0;
+  double c = upper ? b1 : b0;
+  const double d = upper ? b0 : b1;
+  c += dpp_rot<0x128>(d);   // row rotate right by 8
+  c += dpp_rot<0xB1>(c);    // quad: lanes 1 0 3 2
+  c += dpp_rot<0x4E>(c);    // quad: lanes 2 3 0 1
+  c += dpp_rot<0x141>(c);   // half-row mirror: the other quad
+  return c;
 }
 
 // sums of a and b over a 256-thread workgroup, returned to every thread; the
@@ -84,6 +139,41 @@ __device__ __forceinline__ Refl make_refl(double2 alpha, double xnorm) {
   const double den = dr * dr + di * di;
   h.sc = make_double2(dr / den, -di / den);
   h.tau = make_double2((beta - alpha.x) / beta, -alpha.y / beta);
+  h.rd = make_double2(beta, 0.0);
+  return h;
+}
+// 1 / x and 1 / sqrt(x) to full precision from the hardware's estimates (normal x)
+__device__ __forceinline__ double rcp_full(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(y, fma(-x, y, 1.0), y);
+  return fma(y, fma(-x, y, 1.0), y);
+}
+__device__ __forceinline__ double rsq_full(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+// the same reflector from the sum of squares s2 = |x|^2, with the short chain of
+// operations that the panel kernels wait for; norms far outside the usual range
+// take the scaled form
+__device__ __forceinline__ Refl make_refl2(double2 alpha, double s2) {
+  const double n2 = fma(alpha.x, alpha.x, fma(alpha.y, alpha.y, s2));
+  if (!(n2 > 0x1p-900 && n2 < 0x1p900)) return make_refl(alpha, sqrt(s2));
+  Refl h;
+  if (s2 == 0.0 && alpha.y == 0.0) {
+    h.tau = make_double2(0.0, 0.0);
+    h.rd = alpha;
+    h.sc = make_double2(0.0, 0.0);
+    return h;
+  }
+  const double y = rsq_full(n2);
+  double nrm = n2 * y;
+  nrm = fma(0.5 * y, fma(-nrm, nrm, n2), nrm);
+  const double beta = -copysign(nrm, alpha.x);
+  const double dr = alpha.x - beta, di = alpha.y;
+  const double iden = rcp_full(fma(dr, dr, di * di)), ib = rcp_full(beta);
+  h.sc = make_double2(dr * iden, -di * iden);
+  h.tau = make_double2(-dr * ib, -di * ib);
   h.rd = make_double2(beta, 0.0);
   return h;
 }
@@ -471,6 +561,278 @@ __global__ __launch_bounds__(256) void k_qr_col2r(int64_t m, int64_t j, double2*
   }
 }
 
+// A whole panel of at most 64 R rows factored by one workgroup with its columns
+// j0 .. j0+nbp-1 (nbp <= C NW) in registers: column j0 + q NW + w in element q of
+// wave w, row j0 + lane + 64 u in element u. The current column y is read from
+// LDS (two buffers, one barrier per column) as it stands before its reflector is
+// known: every wave forms |y|^2 and the products y^H x with its own columns in the
+// same pass, sums them inside the wave and derives the reflector itself,
+//   v = [1, sc y],  x_j -= f,  x -= f sc y  with  f = conj(tau) (x_j + conj(sc) y^H x),
+// so the chain per column is one pass, one sum and one update. Bound by the
+// instructions of one CU: 32 columns of 256 rows take 48 us (95 with two columns
+// per launch), of 128 rows 40 us.
+// Writes v_j (rows >= j0), tau_j, R[j][j] and the rows j0 .. j-1 of R above it.
+template <int R, int C, int NW>
+__global__ __launch_bounds__(64 * NW) void k_qr_panel(int64_t m, int64_t j0, int nbp,
+                                                      double2* __restrict__ W,
+                                                      double2* __restrict__ Vf,
+                                                      double2* __restrict__ tau,
+                                                      double2* __restrict__ rdiag, QrStrides bs) {
+  __shared__ double2 Ys[2][64 * R];
+  W += blockIdx.x * bs.W;
+  Vf += blockIdx.x * bs.V;
+  tau += blockIdx.x * bs.k;
+  rdiag += blockIdx.x * bs.k;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double2 x[C][R];
+#pragma unroll
+  for (int q = 0; q < C; ++q) {
+    const int c = q * NW + wave;
+    const double2* src = W + (j0 + c) * m;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int64_t i = j0 + lane + 64 * u;
+      x[q][u] = (c < nbp && i < m) ? src[i] : make_double2(0.0, 0.0);
+    }
+  }
+  if (wave == 0) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) Ys[0][64 * u + lane] = x[0][u];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < C; ++q) {
+    for (int wo = 0; wo < NW; ++wo) {
+      const int jj = q * NW + wo;
+      if (jj >= nbp) break;
+      const int buf = jj & 1;
+      const double2 alpha = Ys[buf][jj];
+      double2 y[R];
+#pragma unroll
+      for (int u = 0; u < R; ++u) y[u] = Ys[buf][64 * u + lane];
+      if (lane <= jj) y[0] = make_double2(0.0, 0.0);
+      double s2 = 0.0, dr[C] = {}, di[C] = {};
+#pragma unroll
+      for (int u = 0; u < R; ++u) s2 += y[u].x * y[u].x + y[u].y * y[u].y;
+#pragma unroll
+      for (int p = q; p < C; ++p) {
+        dr[p] = di[p] = 0.0;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          dr[p] += y[u].x * x[p][u].x + y[u].y * x[p][u].y;
+          di[p] += y[u].x * x[p][u].y - y[u].y * x[p][u].x;
+        }
+      }
+      {
+        // eight sums at a time; |y|^2 takes a free slot when the first column is done
+        static_assert(C % 4 == 0, "four products per group of eight sums");
+        if (q == 0) s2 = wave_sum(s2);
+#pragma unroll
+        for (int p0 = q / 4 * 4; p0 < C; p0 += 4) {
+          double v8[8];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            v8[2 * k] = p0 + k >= q ? dr[p0 + k] : (p0 + k == q - 1 ? s2 : 0.0);
+            v8[2 * k + 1] = p0 + k >= q ? di[p0 + k] : 0.0;
+          }
+          const double sums = wave_sum8(v8);
+          if (q > 0 && q % 4 != 0 && p0 < q) s2 = lane_value(sums, 8 * sum8_slot(2 * (q - 1 - p0)));
+          if (q > 0 && q % 4 == 0 && p0 == q) s2 = wave_sum(s2);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (p0 + k >= q) {
+              dr[p0 + k] = lane_value(sums, 8 * sum8_slot(2 * k));
+              di[p0 + k] = lane_value(sums, 8 * sum8_slot(2 * k + 1));
+            }
+        }
+      }
+      const Refl h = make_refl2(alpha, s2);
+      // later columns (element q only of the waves after the owner)
+#pragma unroll
+      for (int p = q; p < C; ++p) {
+        const double2 xj = make_double2(lane_value(x[p][0].x, jj), lane_value(x[p][0].y, jj));
+        const double2 d = cmul2(conj2(h.sc), make_double2(dr[p], di[p]));
+        double2 f = cmul2(conj2(h.tau), make_double2(xj.x + d.x, xj.y + d.y));
+        if (p == q && wave <= wo) f = make_double2(0.0, 0.0);
+        const double2 g = cmul2(f, h.sc);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          x[p][u].x -= g.x * y[u].x - g.y * y[u].y;
+          x[p][u].y -= g.x * y[u].y + g.y * y[u].x;
+        }
+        if (lane == jj) {
+          x[p][0].x -= f.x;
+          x[p][0].y -= f.y;
+        }
+        // the next column goes out first
+        if (p == q + (wo == NW - 1) && wave == (wo + 1) % NW) {
+#pragma unroll
+          for (int u = 0; u < R; ++u) Ys[buf ^ 1][64 * u + lane] = x[p][u];
+        }
+      }
+      if (wave == wo) {
+        double2* vj = Vf + (j0 + jj) * m;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          const int64_t i = j0 + lane + 64 * u;
+          double2 v = cmul2(y[u], h.sc);
+          if (u == 0 && lane == jj) v = make_double2(1.0, 0.0);
+          if (i < m) vj[i] = v;
+        }
+        if (lane < jj) W[(j0 + jj) * m + j0 + lane] = x[q][0];   // finished rows of R
+        if (lane == 0) {
+          tau[j0 + jj] = h.tau;
+          rdiag[j0 + jj] = h.rd;
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// Columns j .. j+nc-1 (nc <= 4) of a panel that starts at j0, at most 256 R rows below j,
+// in one launch: workgroup b handles column j + b. Every workgroup factors the nc
+// columns for itself in registers (row j + t + 256 u in element u of thread t; the
+// same reductions in the same order, so the reflectors agree bitwise), each with
+// one reduction over the workgroup: |y|^2 and the products y^H x with the columns that
+// follow, before the reflector is known (as in k_qr_panel). Workgroups b < nc
+// store v_{j+b}, tau, R[j+b][j+b] and, into rup (QR_NB x QR_NB, panel-local), the
+// rows j .. j+b-1 of R above it: the columns j .. j+nc-1 of W are read by every
+// workgroup during the launch and are not written. The others apply the
+// reflectors to their column. 8 rows per thread (2048 rows): 7.9 us for four columns, against
+// 14.8 for two launches of two columns; 4 rows: 6.5 against 12.8; 2 rows: 5.6.
+template <int R>
+__global__ __launch_bounds__(256) void k_qr_col4(int64_t m, int64_t j0, int64_t j, int nc,
+                                                 double2* __restrict__ W,
+                                                 double2* __restrict__ Vf,
+                                                 double2* __restrict__ tau,
+                                                 double2* __restrict__ rdiag,
+                                                 double2* __restrict__ rup, QrStrides bs) {
+  constexpr int K = 4;
+  __shared__ double red[2][2 * K + 1][4];   // |y|^2, then re / im of y^H x per later column
+  __shared__ double2 top[2][K + 1];         // row j + c of the columns, the own one last
+  W += blockIdx.y * bs.W;
+  Vf += blockIdx.y * bs.V;
+  tau += blockIdx.y * bs.k;
+  rdiag += blockIdx.y * bs.k;
+  rup += blockIdx.y * bs.G;
+  const int t = threadIdx.x, wave = t >> 6, b = blockIdx.x;
+  const bool own = b >= nc;
+  double2 x[K + 1][R];
+#pragma unroll
+  for (int c = 0; c <= K; ++c) {
+    const int64_t col = c < K ? j + c : j + b;
+    const bool on = c < K ? c < nc : own;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int64_t i = j + t + 256 * u;
+      x[c][u] = (on && i < m) ? W[col * m + i] : make_double2(0.0, 0.0);
+    }
+  }
+  Refl mine = {};
+#pragma unroll
+  for (int c = 0; c < K; ++c) {
+    if (c < nc) {
+      const double2 y0 = t > c ? x[c][0] : make_double2(0.0, 0.0);
+      double s[2 * K + 1];
+#pragma unroll
+      for (int v = 0; v < 2 * K + 1; ++v) s[v] = 0.0;
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const double2 y = u == 0 ? y0 : x[c][u];
+        s[0] += y.x * y.x + y.y * y.y;
+#pragma unroll
+        for (int p = c + 1; p <= K; ++p) {
+          s[2 * p - 1] += y.x * x[p][u].x + y.y * x[p][u].y;
+          s[2 * p] += y.x * x[p][u].y - y.y * x[p][u].x;
+        }
+      }
+      {
+        // eight products (the slots of finished columns are free: |y|^2 takes one)
+        double v8[8];
+#pragma unroll
+        for (int v = 0; v < 8; ++v) v8[v] = v + 1 > 2 * c ? s[v + 1] : (v == 0 ? s[0] : 0.0);
+        const double sums = wave_sum8(v8);
+        const int slot = sum8_slot((t & 63) >> 3);
+        if ((t & 7) == 0) red[c & 1][c > 0 && slot == 0 ? 0 : slot + 1][wave] = sums;
+        if (c == 0) {
+          const double r = wave_sum(s[0]);
+          if ((t & 63) == 0) red[0][0][wave] = r;
+        }
+      }
+      if (t == c) {
+#pragma unroll
+        for (int p = c; p <= K; ++p) top[c & 1][p] = x[p][0];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < 2 * K + 1; ++v)
+        if (v == 0 || v > 2 * c) {
+          const double* r = red[c & 1][v];
+          s[v] = (r[0] + r[1]) + (r[2] + r[3]);
+        }
+      const Refl h = make_refl2(top[c & 1][c], s[0]);
+      if (b == c) mine = h;
+#pragma unroll
+      for (int p = c + 1; p <= K; ++p) {
+        const double2 xj = top[c & 1][p];
+        const double2 d = cmul2(conj2(h.sc), make_double2(s[2 * p - 1], s[2 * p]));
+        const double2 f = cmul2(conj2(h.tau), make_double2(xj.x + d.x, xj.y + d.y));
+        const double2 g = cmul2(f, h.sc);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          const double2 y = u == 0 ? y0 : x[c][u];
+          x[p][u].x -= g.x * y.x - g.y * y.y;
+          x[p][u].y -= g.x * y.y + g.y * y.x;
+        }
+        if (t == c) {
+          x[p][0].x -= f.x;
+          x[p][0].y -= f.y;
+        }
+      }
+    }
+  }
+  if (own) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int64_t i = j + t + 256 * u;
+      if (i < m) W[(j + b) * m + i] = x[K][u];
+    }
+    return;
+  }
+  double2* vj = Vf + (j + b) * m;
+  for (int64_t i = j0 + t; i < j; i += 256) vj[i] = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int c = 0; c < K; ++c) {
+    if (c == b) {
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const int64_t i = j + t + 256 * u;
+        double2 v = cmul2(x[c][u], mine.sc);
+        if (u == 0 && t <= c) v = make_double2(t == c ? 1.0 : 0.0, 0.0);
+        if (i < m) vj[i] = v;
+      }
+      if (t < c) rup[(j - j0 + t) * QR_NB + (j - j0 + c)] = x[c][0];
+      if (t == 0) {
+        tau[j + c] = mine.tau;
+        rdiag[j + c] = mine.rd;
+      }
+    }
+  }
+}
+
+// the entries of R inside the groups of four columns of a panel, from rup into W
+// after the panel
+__global__ void k_qr_fixup4(int64_t m, int64_t j0, int nbp, const double2* __restrict__ rup,
+                            double2* __restrict__ W, QrStrides bs) {
+  rup += blockIdx.x * bs.G;
+  W += blockIdx.x * bs.W;
+  for (int e = threadIdx.x; e < QR_NB * QR_NB; e += 256) {
+    const int a = e / QR_NB, b = e % QR_NB;
+    if (a < b && b < nbp && a / 4 == b / 4) W[(j0 + b) * m + j0 + a] = rup[e];
+  }
+}
+
 // R[jj][jj+1] of the two-reflector launches of a panel, written after the panel
 __global__ void k_qr_fixsup(int64_t m, int64_t j0, int64_t pe, const double2* __restrict__ rsup,
                             double2* __restrict__ W, QrStrides bs) {
@@ -480,67 +842,132 @@ __global__ void k_qr_fixsup(int64_t m, int64_t j0, int64_t pe, const double2* __
   if (jj + 1 < pe) W[(jj + 1) * m + jj] = rsup[jj];
 }
 
-// G[a][b] = v_a^H v_b for the panel's reflectors (rows j0 .. m-1), one workgroup per entry
-__global__ __launch_bounds__(256) void k_qr_vtv(int64_t m, int64_t j0, int nbp,
+// partial G[a][b] = v_a^H v_b (a <= b in steps of 16) of the panel's reflectors over the
+// rows j0 + rows blockIdx.x ..: FP64 MFMA on 16 x 16 tiles, the operands loaded as in the
+// cross Gram kernel of the Jacobi iteration (a lane holds rows 2 kk, 2 kk + 1 of every 8
+// of column l16); columns >= nbp count as zero. rows is a multiple of 128.
+__global__ __launch_bounds__(256) void k_qr_vtv(int64_t m, int64_t j0, int nbp, int rows,
                                                 const double2* __restrict__ Vf,
                                                 double2* __restrict__ G, QrStrides bs) {
+  static_assert(QR_NB == 32, "two 16-column tiles");
+  __shared__ double2 red[4][3][4][64];
   Vf += blockIdx.y * bs.V;
-  G += blockIdx.y * bs.G;
-  const int a = blockIdx.x / nbp, b = blockIdx.x % nbp;
-  if (b <= a) return;   // only the strict upper triangle is used
-  const double2* va = Vf + (j0 + a) * m;
-  const double2* vb = Vf + (j0 + b) * m;
-  double sr = 0, si = 0;
-  for (int64_t i = j0 + threadIdx.x; i < m; i += 256) {
-    const double2 x = va[i], y = vb[i];
-    sr += x.x * y.x + x.y * y.y;
-    si += x.x * y.y - x.y * y.x;
+  G += blockIdx.y * bs.G + (int64_t)blockIdx.x * QR_NB * QR_NB;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int l16 = lane & 15, kk = lane >> 4;
+  const int64_t end = j0 + (int64_t)(blockIdx.x + 1) * rows < m
+                          ? j0 + (int64_t)(blockIdx.x + 1) * rows : m;
+  d4_t re[3], im[3];
+#pragma unroll
+  for (int h = 0; h < 3; ++h) re[h] = im[h] = d4_t{0, 0, 0, 0};
+  const double2* __restrict__ V0 = Vf + (j0 + l16) * m;
+  const double2* __restrict__ V1 = V0 + 16 * m;
+  const bool in0 = l16 < nbp, in1 = 16 + l16 < nbp;
+  for (int64_t r0 = j0 + (int64_t)blockIdx.x * rows + 32 * wave; r0 < end; r0 += 128) {
+    double2 a[4][2], b[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int64_t i = r0 + 8 * u + 2 * kk + h;
+        a[u][h] = (in0 && i < end) ? V0[i] : make_double2(0.0, 0.0);
+        b[u][h] = (in1 && i < end) ? V1[i] : make_double2(0.0, 0.0);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double2 x[3] = {a[u][h], a[u][h], b[u][h]}, y[3] = {a[u][h], b[u][h], b[u][h]};
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          re[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].x, y[e].x, re[e], 0, 0, 0);
+          im[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].x, y[e].y, im[e], 0, 0, 0);
+          re[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].y, y[e].y, re[e], 0, 0, 0);
+          im[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[e].y, y[e].x, im[e], 0, 0, 0);
+        }
+      }
   }
-  block_sum2(sr, si);
-  if (threadIdx.x == 0) G[a * QR_NB + b] = make_double2(sr, si);
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][e][v][lane] = make_double2(re[e][v], im[e][v]);
+  __syncthreads();
+  const int i = t >> 4, j = t & 15, src = 16 * (i & 3) + j;
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    double2 sum = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const double2 v = red[w][e][i >> 2][src];
+      sum.x += v.x;
+      sum.y += v.y;
+    }
+    const int a0 = e == 2 ? 16 : 0, b0 = e == 0 ? 0 : 16;
+    G[(a0 + i) * QR_NB + b0 + j] = sum;
+  }
 }
 
-// compact WY factor (forward, columnwise): T[i][i] = tau_i,
-// T[0:i, i] = -tau_i T[0:i, 0:i] (V[:, 0:i]^H v_i); zero padded to QR_NB x QR_NB.
-// Thread r builds row r of T in registers (it only needs its own row and G),
-// so the column recurrence needs no barriers.
-__global__ __launch_bounds__(64) void k_qr_tmat(int nbp, const double2* __restrict__ G,
-                                                const double2* __restrict__ tau,
-                                                double2* __restrict__ T, QrStrides bs) {
+// compact WY factor (forward, columnwise; zero padded to QR_NB x QR_NB): T of a
+// single reflector is tau, and two neighbouring blocks combine to
+//   T = [[T1, -T1 (V1^H V2) T2], [0, T2]],
+// so five levels of doubling build the factor with all threads at work (a column by
+// column recurrence in one wave took 19 us). Sums the nparts partial G first.
+__global__ __launch_bounds__(256) void k_qr_tmat(int nbp, int nparts, const double2* __restrict__ G,
+                                                 const double2* __restrict__ tau,
+                                                 double2* __restrict__ T, QrStrides bs) {
   G += blockIdx.x * bs.G;
   tau += blockIdx.x * bs.k;
   T += blockIdx.x * bs.T;
-  __shared__ double2 Gs[QR_NB][QR_NB + 1];
-  __shared__ double2 taus[QR_NB];
-  const int r = threadIdx.x;
-  for (int e = r; e < QR_NB * QR_NB; e += 64) {
-    const int a = e / QR_NB, b = e % QR_NB;
-    Gs[a][b] = (a < b && b < nbp) ? G[e] : make_double2(0.0, 0.0);
-  }
-  if (r < QR_NB) taus[r] = (r < nbp) ? tau[r] : make_double2(0.0, 0.0);
-  __syncthreads();
-  if (r >= QR_NB) return;
-  double2 trow[QR_NB];
+  __shared__ double2 Gs[QR_NB][QR_NB + 1], Ts[QR_NB][QR_NB + 1], Ms[QR_NB][QR_NB + 1];
+  const int t = threadIdx.x;
 #pragma unroll
-  for (int c = 0; c < QR_NB; ++c) trow[c] = make_double2(0.0, 0.0);
-#pragma unroll
-  for (int i = 0; i < QR_NB; ++i) {
-    if (i < nbp) {
-      const double2 ti = taus[i];
-      double ar = 0, ai = 0;
-#pragma unroll
-      for (int s = 0; s < i; ++s) {
-        // T[r][s] is zero for s < r, so the full range gives the same sum
-        const double2 a = trow[s], g = Gs[s][i];
-        ar += a.x * g.x - a.y * g.y;
-        ai += a.x * g.y + a.y * g.x;
+  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
+    const int e = t + 256 * u, a = e / QR_NB, b = e % QR_NB;
+    double2 g = make_double2(0.0, 0.0);
+    if (a < b && b < nbp)
+      for (int p = 0; p < nparts; ++p) {
+        const double2 v = G[(int64_t)p * QR_NB * QR_NB + e];
+        g.x += v.x;
+        g.y += v.y;
       }
-      if (r < i) trow[i] = make_double2(-(ti.x * ar - ti.y * ai), -(ti.x * ai + ti.y * ar));
-      else if (r == i) trow[i] = ti;
+    Gs[a][b] = g;
+    Ts[a][b] = (a == b && a < nbp) ? tau[a] : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 1; h < QR_NB; h *= 2) {
+    // output (i, j) of block pair b: 16 h outputs in all
+    const int b = t / (h * h), i = (t / h) % h, j = t % h;
+    const int r0 = 2 * h * b, c0 = r0 + h;
+    const bool on = t < 16 * h;
+    if (on) {   // M = (V1^H V2) T2
+      double2 m = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int k = 0; k < h; ++k) {
+        const double2 x = cmul2(Gs[r0 + i][c0 + k], Ts[c0 + k][c0 + j]);
+        m.x += x.x;
+        m.y += x.y;
+      }
+      Ms[r0 + i][c0 + j] = m;
     }
+    __syncthreads();
+    if (on) {
+      double2 m = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int k = 0; k < h; ++k) {
+        const double2 x = cmul2(Ts[r0 + i][r0 + k], Ms[r0 + k][c0 + j]);
+        m.x -= x.x;
+        m.y -= x.y;
+      }
+      Ts[r0 + i][c0 + j] = m;
+    }
+    __syncthreads();
   }
 #pragma unroll
-  for (int c = 0; c < QR_NB; ++c) T[r * QR_NB + c] = trow[c];
+  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
+    const int e = t + 256 * u;
+    T[e] = Ts[e / QR_NB][e % QR_NB];
+  }
 }
 
 // Y = sum of the nparts partial products P[s] (QR_NB x nc, rows < nbp used);
@@ -592,6 +1019,12 @@ __global__ __launch_bounds__(256) void k_qr_reduce(int nbp, int64_t nc, int npar
 
 static inline size_t al(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// row segments of the V^H V products over `rows` rows: at least 128 rows each
+static int64_t vtv_parts(int64_t rows) {
+  const int64_t p = (rows + 127) / 128;
+  return p < QR_VTV_PARTS ? p : QR_VTV_PARTS;
+}
+
 static QrStrides qr_strides(int64_t m, int64_t n, int64_t ncmax) {
   const int64_t k = m < n ? m : n;
   const int64_t npan = (k + QR_NB - 1) / QR_NB;
@@ -601,7 +1034,7 @@ static QrStrides qr_strides(int64_t m, int64_t n, int64_t ncmax) {
   b.V = m * k;
   b.k = k + 1;
   b.T = (npan + 1) * QR_NB * QR_NB;
-  b.G = QR_NB * QR_NB;
+  b.G = vtv_parts(m) * QR_NB * QR_NB;
   b.P = (QR_SPLITK + 1) * QR_NB * nc;
   b.Z = QR_NB * nc;
   return b;
@@ -681,6 +1114,32 @@ static int apply_block(const QrFact& f, int64_t j0, int nbp, const double2* Tp, 
   return zgemm(g, PTN_FP64, PTN_T_C128, PTN_T_C128, PTN_T_C128, nullptr, 0, s);
 }
 
+// The panel j0 .. pe-1 of at most 2048 rows. One workgroup holds a panel of up to
+// 256 rows in its registers; beyond, four columns per launch with every column in a
+// workgroup of its own (512 rows: 45 us per panel against 66 in one workgroup; the
+// sub-panels of 16 and 8 columns that one CU can hold at 1024 and 2048 rows are bound by
+// that CU's FP64 and LDS rates: 90 and 200 us per panel against 52 and 63).
+template <int R> static void panel_one(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
+  k_qr_panel<R, 8, 4><<<(unsigned)f.batch, 256, 0, s>>>(f.m, j0, (int)(pe - j0), f.W, f.Vf, f.tau,
+                                                       f.rdiag, f.bs);
+}
+template <int R> static void panel_col4(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
+  const unsigned B = (unsigned)f.batch;
+  for (int64_t j = j0; j < pe; j += 4)
+    k_qr_col4<R><<<dim3((unsigned)(pe - j), B), 256, 0, s>>>(
+        f.m, j0, j, (int)(pe - j < 4 ? pe - j : 4), f.W, f.Vf, f.tau, f.rdiag, f.G, f.bs);
+  k_qr_fixup4<<<B, 256, 0, s>>>(f.m, j0, (int)(pe - j0), f.G, f.W, f.bs);
+}
+static void panel(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
+  const int64_t rows = f.m - j0;
+  if (rows <= 64) panel_one<1>(f, j0, pe, s);
+  else if (rows <= 128) panel_one<2>(f, j0, pe, s);
+  else if (rows <= 256) panel_one<4>(f, j0, pe, s);
+  else if (rows <= 512) panel_col4<2>(f, j0, pe, s);
+  else if (rows <= 1024) panel_col4<4>(f, j0, pe, s);
+  else panel_col4<8>(f, j0, pe, s);
+}
+
 int qr_factor(QrFact& f, const double2* a, int64_t lda, hipStream_t s, int64_t sa) {
   const int64_t m = f.m, n = f.n, k = f.k;
   if (m == 0 || n == 0) return PTN_OK;
@@ -700,26 +1159,28 @@ int qr_factor(QrFact& f, const double2* a, int64_t lda, hipStream_t s, int64_t s
     const int64_t j0 = p * QR_NB;
     const int64_t pe = (j0 + QR_NB < k) ? j0 + QR_NB : k;
     const int nbp = (int)(pe - j0);
-    int64_t j = j0;
-    for (; j + 1 < pe; j += 2) {
-      const dim3 g((unsigned)(pe - j), B);
-      const int64_t rows = m - j;
-      if (rows <= 256 * 4)
-        k_qr_col2r<4><<<g, 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.rsup, f.bs);
-      else if (rows <= 256 * 8)
-        k_qr_col2r<8><<<g, 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.rsup, f.bs);
-      else if (rows <= 256 * 16)
-        k_qr_col2r<16><<<g, 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.rsup, f.bs);
-      else
-        k_qr_col2<<<g, 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.rsup, f.bs);
+    if (m - j0 <= 2048) {
+      panel(f, j0, pe, s);
+    } else {
+      int64_t j = j0;
+      for (; j + 1 < pe; j += 2) {
+        const dim3 g((unsigned)(pe - j), B);
+        if (m - j <= 256 * 16)
+          k_qr_col2r<16><<<g, 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.rsup, f.bs);
+        else
+          k_qr_col2<<<g, 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.rsup, f.bs);
+      }
+      if (j < pe)
+        k_qr_col<<<dim3((unsigned)(pe - j), B), 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.bs);
+      if (pe - j0 >= 2) k_qr_fixsup<<<dim3(1, B), QR_NB / 2, 0, s>>>(m, j0, pe, f.rsup, f.W, f.bs);
     }
-    if (j < pe)
-      k_qr_col<<<dim3((unsigned)(pe - j), B), 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.bs);
-    if (pe - j0 >= 2) k_qr_fixsup<<<dim3(1, B), QR_NB / 2, 0, s>>>(m, j0, pe, f.rsup, f.W, f.bs);
     PTN_LAUNCH_CHECK();
     double2* Tp = f.T + p * QR_NB * QR_NB;
-    k_qr_vtv<<<dim3((unsigned)(nbp * nbp), B), 256, 0, s>>>(m, j0, nbp, f.Vf, f.G, f.bs);
-    k_qr_tmat<<<B, 64, 0, s>>>(nbp, f.G, f.tau + j0, Tp, f.bs);
+    const int64_t np = vtv_parts(m - j0);
+    const int64_t rows = ((m - j0 + np - 1) / np + 127) / 128 * 128;
+    const int parts = (int)((m - j0 + rows - 1) / rows);
+    k_qr_vtv<<<dim3((unsigned)parts, B), 256, 0, s>>>(m, j0, nbp, (int)rows, f.Vf, f.G, f.bs);
+    k_qr_tmat<<<B, 256, 0, s>>>(nbp, parts, f.G, f.tau + j0, Tp, f.bs);
     PTN_LAUNCH_CHECK();
     int st;
     if (pe < n && (st = apply_block(f, j0, nbp, Tp, 1, f.W, m, pe, n - pe, s, f.bs.W))) return st;
