@@ -195,8 +195,8 @@ int ptn_env_apply(const ptn_local_op* op, int side, const void* a, const void* b
 size_t ptn_krylov_workspace(const ptn_local_op* op, int numiter);
 
 /* hipGraph capture of the local solves (no counterpart in the reference):
- * with graphs on (the default), a solve whose vectors have at most 2^20
- * elements (all problems of a batch together) is captured once per shape
+ * with graphs on (off by default: direct launches cost the host less), a solve
+ * whose vectors have at most 2^20 elements (all problems of a batch together) is captured once per shape
  * bucket and replayed as one graph launch with the new pointers; breakdowns
  * are predicated on the device. on < 0 only queries. Returns the previous
  * setting. ptn_graph_launches() counts the graph launches of the process. */

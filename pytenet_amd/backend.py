@@ -41,20 +41,39 @@ def precision_code(precision, block_sparse=False):
     return PRECISIONS[precision] | (_lib.PTN_BLOCK_SPARSE if block_sparse else 0)
 
 
-def device():
-    """The current GPU; raises when none is visible (no CPU fallback)."""
+# The wrappers below run once per kernel call of a sweep; on short bonds their own time
+# is of the order of the kernels'. What does not change after the first call (a GPU is
+# visible, the library is loaded, the device objects) is therefore looked up once,
+# and the current device and stream are read without the checks of torch.cuda.
+_devices = None
+
+
+def _ready():
+    global _devices
     if not torch.cuda.is_available():
         raise RuntimeError("pytenet_amd needs a ROCm GPU; none is visible")
     _lib.load()
-    return torch.device("cuda", torch.cuda.current_device())
+    torch.cuda.current_device()     # initialises the runtime
+    _devices = [torch.device("cuda", i) for i in range(torch.cuda.device_count())]
+
+
+def device():
+    """The current GPU; raises when none is visible (no CPU fallback)."""
+    if _devices is None:
+        _ready()
+    return _devices[torch._C._cuda_getDevice()]
 
 
 def stream():
-    return c_p(torch.cuda.current_stream().cuda_stream)
+    """The current HIP stream (address) of the current GPU."""
+    if _devices is None:
+        _ready()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ptr(t):
-    return c_p(t.data_ptr())
+    """Device address of a tensor."""
+    return t.data_ptr()
 
 
 class _Workspace:
@@ -66,14 +85,14 @@ class _Workspace:
         self.buf = {}
 
     def get(self, nbytes):
-        dev = torch.cuda.current_device()
-        key = (dev, torch.cuda.current_stream().cuda_stream)
+        dev = device()
+        key = (dev.index, stream())
         cur = self.buf.get(key)
         if cur is None or cur.numel() < nbytes:
             nb = max(int(nbytes), 1 << 20)
             if cur is not None:
                 nb = max(nb, int(cur.numel() * 1.25))
-            cur = torch.empty(nb, dtype=torch.uint8, device=torch.device("cuda", dev))
+            cur = torch.empty(nb, dtype=torch.uint8, device=dev)
             self.buf[key] = cur
         return cur
 
@@ -88,6 +107,8 @@ def workspace(nbytes):
 def as_dev(x):
     """complex128, contiguous, on the current GPU (uploads NumPy arrays)."""
     dev = device()
+    if type(x) is torch.Tensor and x.dtype is torch.complex128 and x.device == dev:
+        return x.contiguous()
     if isinstance(x, np.ndarray) or np.isscalar(x):
         return torch.as_tensor(np.ascontiguousarray(x, dtype=np.complex128), device=dev)
     if not isinstance(x, torch.Tensor):
@@ -299,14 +320,14 @@ def krylov_local(kind, v, l, w, r, numiter, mode, dt=0.0, precision="fp64", info
     ws = workspace(nb)
     out = torch.empty_like(v)
     if info is None:
-        info = torch.zeros(4, dtype=torch.int32, device=v.device)
+        info = torch.empty(4, dtype=torch.int32, device=v.device)   # written by every solve
     if mode == "expm":
         dt = complex(dt)
         _check(lib.ptn_krylov_expm(ctypes.byref(op), ptr(v), dt.real, dt.imag, int(numiter),
                                    ptr(out), ptr(info), None, ptr(ws), ws.numel(), stream()),
                "ptn_krylov_expm")
         return out, None, info
-    energy = torch.zeros(1, dtype=torch.float64, device=v.device)
+    energy = torch.empty(1, dtype=torch.float64, device=v.device)
     _check(lib.ptn_krylov_eigh(ctypes.byref(op), ptr(v), int(numiter), ptr(out), ptr(energy),
                                ptr(info), None, ptr(ws), ws.numel(), stream()), "ptn_krylov_eigh")
     return out, energy, info
@@ -374,8 +395,8 @@ def timing_end(max_rows=64):
 
 
 def set_graphs(on=True):
-    """Switch the hipGraph capture of short local solves on or off (process-wide);
-    returns the previous setting."""
+    """Switch the hipGraph capture of short local solves on or off (process-wide, off
+    by default); returns the previous setting."""
     return bool(_lib.load().ptn_set_graphs(int(bool(on))))
 
 
@@ -751,14 +772,14 @@ def krylov_local_batched(kind, v, l, w, r, numiter, mode, dt=0.0, precision="fp6
     lib = _lib.load()
     ws = workspace(lib.ptn_krylov_workspace_batched(ctypes.byref(op), int(numiter), nb))
     out = torch.empty_like(v)
-    info = torch.zeros((nb, 4), dtype=torch.int32, device=v.device)
+    info = torch.empty((nb, 4), dtype=torch.int32, device=v.device)
     if mode == "expm":
         dt = complex(dt)
         _check(lib.ptn_krylov_expm_batched(ctypes.byref(op), nb, ptr(v), dt.real, dt.imag,
                                            int(numiter), ptr(out), ptr(info), ptr(ws), ws.numel(),
                                            stream()), "ptn_krylov_expm_batched")
         return out, None, info
-    energy = torch.zeros(nb, dtype=torch.float64, device=v.device)
+    energy = torch.empty(nb, dtype=torch.float64, device=v.device)
     _check(lib.ptn_krylov_eigh_batched(ctypes.byref(op), nb, ptr(v), int(numiter), ptr(out),
                                        ptr(energy), ptr(info), ptr(ws), ws.numel(), stream()),
            "ptn_krylov_eigh_batched")

@@ -10,9 +10,8 @@ batch axis, and every local operation of the sweep (Krylov exponential of the
 one-site and bond operators, QR, environment steps, bond absorption) is a
 single batched launch sequence for the whole bucket. The buckets run on
 separate streams and advance together, one site step at a time, so their
-launch sequences overlap on the GPU (the local solves of small buckets are
-replayed as captured graphs). Each chain gets exactly the result of its own
-tdvp_singlesite call (up to rounding).
+launch sequences overlap on the GPU. Each chain gets exactly the result of its
+own tdvp_singlesite call (up to rounding).
 """
 
 import numpy as np
@@ -57,7 +56,8 @@ class _Bucket:
             for p in psis:
                 for a in p.a:
                     a.record_stream(self.stream)
-            self.W = [torch.stack([backend.as_dev(H.a[i]) for H in hamiltonians])
+            # one upload per site: the MPO tensors of the chains stacked on the host
+            self.W = [backend.as_dev(np.stack([backend.to_host(H.a[i]) for H in hamiltonians]))
                       for i in range(self.n)]
         self.status = []
 

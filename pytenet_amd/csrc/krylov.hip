@@ -443,10 +443,9 @@ static int krylov_enqueue(const ptn_local_op* op, int mode, const void* v, doubl
                           int64_t batch, const SectorPlan* sp);
 
 // ---------------------------------------------------------------------------
-// hipGraph capture of the local solves. A solve whose vectors are short is
-// bound by kernel-launch latency (numiter x ~7 launches); its whole launch
-// sequence (state init, every Lanczos iteration with its matvec, the
-// tridiagonal eigensolver, the combination) is captured into a graph on a
+// hipGraph capture of the local solves (off unless ptn_set_graphs turns it on). A
+// solve's whole launch sequence (state init, every Lanczos iteration with its
+// matvec, the tridiagonal eigensolver, the combination) is captured into a graph on a
 // private stream and launched as one graph on the caller's stream. The
 // executable graphs are cached per shape bucket (operator kind and shapes,
 // precision, numiter, mode, batch, device) and updated in place with the
@@ -456,8 +455,11 @@ static int krylov_enqueue(const ptn_local_op* op, int mode, const void* v, doubl
 // ring of GRAPH_RING executables; an executable is updated only after its
 // previous launch has completed (an event per slot). Long vectors (MFMA-bound
 // matvecs of milliseconds) are launched directly.
+// Direct launches are the default: capturing and updating ~60 nodes costs the host more
+// than launching them (two-site expm at D = 64: 260 us against 272; a two-site
+// TDVP step of 12 sites 21.9 ms against 25.1; 24 batched chains 55.5 ms against 58.7).
 namespace {
-bool g_graphs_on = true;
+bool g_graphs_on = false;
 constexpr int64_t GRAPH_MAX_N = 1 << 20;   // vector length up to which solves are captured
 constexpr int GRAPH_RING = 3;
 constexpr size_t GRAPH_MAX_BUCKETS = 512;
