@@ -67,22 +67,45 @@ struct GLaunch {
   void* C;
   const int* skip;
   int conjB;                              // B read conjugated
+  // zero fill of the final output by fill_wgs workgroups spread over this launch (the
+  // first product is bound by its matrix instructions, the fill by memory)
+  double2* fill = nullptr;
+  int64_t nfill = 0;
+  unsigned fill_wgs = 0;
+  int fast = 0;                           // byte offsets inside a tile's operands fit 32 bits
 };
+constexpr int64_t FILL_PER_WG = 16384;    // elements per fill workgroup
 
-// One workgroup = one BM x BN tile of one block; the MFMA tile body is the one
-// of zgemm_kernel (real embedding of the complex product, double-buffered LDS
-// stages), with k running over the block's segments.
+// One workgroup = one BM x BN tile of one block; staging and MFMA steps are those of
+// zgemm_kernel (whole complex elements, uniform bases with constant 32-bit
+// offsets, rows and columns beyond the block clamped to its last ones, only the
+// partial last stage of a segment with predicates), with k running over the block's
+// segments. Two-site H_eff at D = 2048 (U(1)): first product 249 -> 232 us, output product
+// 305 -> 232 us.
 template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, bool A_KCONTIG,
           bool B_NCONTIG>
 __global__ __launch_bounds__(256) void zgemm_grouped_kernel(GLaunch g) {
   typedef TileCfg<TM, TN, StageK<Tc, TM>::value> T;
   constexpr int BM = T::BM, BN = T::BN, BK = T::BK, NA = T::NA, NB = T::NB;
   typedef typename acc4<Tc>::type acc_t;
-  __shared__ Tc As[2][2 * BK][BM + 1];
-  __shared__ Tc Bs[2][BK][2 * BN + 2];
+  typedef typename cplx_of<Tc>::type C2;
+  __shared__ __align__(16) C2 As[2][BK][BM + 1];
+  __shared__ __align__(16) C2 Bs[2][BK][BN + 1];
   if (g.skip && g.skip[0]) return;
-  // the block of this workgroup: the last block whose first tile <= blockIdx.x
-  const int64_t tile = blockIdx.x;
+  // fill workgroups come at even distances among the tiles' ones
+  int64_t tile = blockIdx.x;
+  if (g.fill_wgs) {
+    const uint64_t f = (uint64_t)blockIdx.x * g.fill_wgs / gridDim.x;
+    if ((uint64_t)(blockIdx.x + 1) * g.fill_wgs / gridDim.x > f) {
+      const int64_t e = (int64_t)(f + 1) * FILL_PER_WG < g.nfill ? (int64_t)(f + 1) * FILL_PER_WG
+                                                                 : g.nfill;
+      for (int64_t i = (int64_t)f * FILL_PER_WG + threadIdx.x; i < e; i += 256)
+        g.fill[i] = make_double2(0.0, 0.0);
+      return;
+    }
+    tile -= (int64_t)f;
+  }
+  // the block of this workgroup: the last block whose first tile <= its tile
   int lo = 0, hi = g.nblocks - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -95,64 +118,73 @@ __global__ __launch_bounds__(256) void zgemm_grouped_kernel(GLaunch g) {
   const int64_t m0 = (lt / bk->tiles_n) * BM, n0 = (lt % bk->tiles_n) * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm0 = (wave >> 1) * T::WM, wn0 = (wave & 1) * T::WN;
-  const TA* __restrict__ A = (const TA*)g.A;
-  const TB* __restrict__ B = (const TB*)g.B;
+  const TA* __restrict__ A = (const TA*)g.A + m0 * g.a_m;
+  const TB* __restrict__ B = (const TB*)g.B + n0 * g.b_n;
   TC* __restrict__ C = (TC*)g.C + bk->c_off;
   const Tc sb = g.conjB ? (Tc)-1 : (Tc)1;
-  int nst = 0;
-  for (int sg = 0; sg < nseg; ++sg) nst += (int)((bk->K[sg] + BK - 1) / BK);
 
-  Tc ra[NA][2], rb[NB][2];
-  // stage `it` of the concatenated segments: segment sg, k offset k0 in it
-  auto load_tiles = [&](int it) {
-    int sg = 0;
-    int64_t k0 = (int64_t)it * BK;
-    for (; sg < nseg - 1; ++sg) {
-      const int64_t ks = ((bk->K[sg] + BK - 1) / BK) * BK;
-      if (k0 < ks) break;
-      k0 -= ks;
-    }
-    const TA* Ap = A + bk->a_off[sg];
-    const TB* Bp = B + bk->b_off[sg];
-    const int64_t K = bk->K[sg];
+  auto arow = [&](int i) -> int { return A_KCONTIG ? (tid + 256 * i) / BK : (tid + 256 * i) % BM; };
+  auto ak = [&](int i) -> int { return A_KCONTIG ? (tid + 256 * i) % BK : (tid + 256 * i) / BM; };
+  auto bcol = [&](int i) -> int { return B_NCONTIG ? (tid + 256 * i) % BN : (tid + 256 * i) / BK; };
+  auto bkk = [&](int i) -> int { return B_NCONTIG ? (tid + 256 * i) / BN : (tid + 256 * i) % BK; };
+  const int mlast = (int)(bM - m0 < BM ? bM - m0 : BM) - 1;
+  const int nlast = (int)(bN - n0 < BN ? bN - n0 : BN) - 1;
+  uint32_t offa[NA], offb[NB];
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int e = tid + 256 * i;
-      int row, kc;
-      if (A_KCONTIG) { row = e / BK; kc = e % BK; } else { kc = e / BM; row = e % BM; }
-      const int64_t m = m0 + row, k = k0 + kc;
-      Tc re = 0, im = 0;
-      if (m < bM && k < K) load_c<Tc>(Ap + m * g.a_m + k * g.a_k, re, im);
-      ra[i][0] = re; ra[i][1] = im;
-    }
+  for (int i = 0; i < NA; ++i)
+    offa[i] = (uint32_t)((min(arow(i), mlast) * g.a_m + ak(i) * g.a_k) * (int64_t)sizeof(TA));
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int e = tid + 256 * i;
-      int col, kc;
-      if (B_NCONTIG) { kc = e / BN; col = e % BN; } else { col = e / BK; kc = e % BK; }
-      const int64_t n = n0 + col, k = k0 + kc;
-      Tc re = 0, im = 0;
-      if (n < bN && k < K) load_c<Tc>(Bp + k * g.b_k + n * g.b_n, re, im);
-      rb[i][0] = re; rb[i][1] = sb * im;
+  for (int i = 0; i < NB; ++i)
+    offb[i] = (uint32_t)((min(bcol(i), nlast) * g.b_n + bkk(i) * g.b_k) * (int64_t)sizeof(TB));
+
+  // the next stage to load: segment sg, k offset k0 in it
+  int sg = 0;
+  int64_t k0 = 0, K = bk->K[0];
+  const TA* Ap = A + bk->a_off[0];
+  const TB* Bp = B + bk->b_off[0];
+  int nst = 0;
+  for (int i = 0; i < nseg; ++i) nst += (int)((bk->K[i] + BK - 1) / BK);
+  C2 ra[NA], rb[NB];
+  auto load_next = [&]() {
+    const TA* Ak = Ap + k0 * g.a_k;
+    const TB* Bk = Bp + k0 * g.b_k;
+    if (g.fast && k0 + BK <= K) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        load_c<Tc>((const TA*)((const char*)Ak + offa[i]), ra[i].x, ra[i].y);
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        load_c<Tc>((const TB*)((const char*)Bk + offb[i]), rb[i].x, rb[i].y);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        ra[i] = C2{0, 0};
+        if (k0 + ak(i) < K)
+          load_c<Tc>(Ak + (int64_t)min(arow(i), mlast) * g.a_m + (int64_t)ak(i) * g.a_k, ra[i].x,
+                     ra[i].y);
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        rb[i] = C2{0, 0};
+        if (k0 + bkk(i) < K)
+          load_c<Tc>(Bk + (int64_t)min(bcol(i), nlast) * g.b_n + (int64_t)bkk(i) * g.b_k, rb[i].x,
+                     rb[i].y);
+      }
+    }
+    k0 += BK;
+    if (k0 >= K && sg + 1 < nseg) {
+      ++sg;
+      k0 = 0;
+      K = bk->K[sg];
+      Ap = A + bk->a_off[sg];
+      Bp = B + bk->b_off[sg];
     }
   };
   auto store_tiles = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int e = tid + 256 * i;
-      int row, kc;
-      if (A_KCONTIG) { row = e / BK; kc = e % BK; } else { kc = e / BM; row = e % BM; }
-      As[buf][2 * kc][row] = ra[i][0];
-      As[buf][2 * kc + 1][row] = ra[i][1];
-    }
+    for (int i = 0; i < NA; ++i) As[buf][ak(i)][arow(i)] = ra[i];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int e = tid + 256 * i;
-      int col, kc;
-      if (B_NCONTIG) { kc = e / BN; col = e % BN; } else { col = e / BK; kc = e % BK; }
-      Bs[buf][kc][2 * col] = rb[i][0];
-      Bs[buf][kc][2 * col + 1] = rb[i][1];
-    }
+    for (int i = 0; i < NB; ++i) Bs[buf][bkk(i)][bcol(i)] = C2{rb[i].x, sb * rb[i].y};
   };
 
   acc_t acc[TM][TN];
@@ -160,35 +192,36 @@ __global__ __launch_bounds__(256) void zgemm_grouped_kernel(GLaunch g) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-  // expanded B operand per lane: real k parity (pa), real column parity (pb)
-  const int kk = lane >> 4;
-  const int pa = kk & 1, pb = lane & 1;
-  const bool take_im = (pa != pb);
-  const Tc im_sign = (pa == 1) ? (Tc)-1 : (Tc)1;
+  const int l16 = lane & 15, kk = lane >> 4, pb = lane & 1;
   int buf = 0;
   if (nst > 0) {
-    load_tiles(0);
+    load_next();
     store_tiles(0);
   }
   __syncthreads();
   for (int it = 0; it < nst; ++it) {
     const bool more = it + 1 < nst;
-    if (more) load_tiles(it + 1);
+    if (more) load_next();
 #pragma unroll
-    for (int ks = 0; ks < BK / 2; ++ks) {
-      Tc av[TM], bv[TN];
+    for (int ks = 0; ks < BK / 4; ++ks) {
+      C2 av[TM];
+      Tc b0[TN], b1[TN];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) av[i] = As[buf][4 * ks + kk][wm0 + 16 * i + (lane & 15)];
+      for (int i = 0; i < TM; ++i) av[i] = As[buf][4 * ks + kk][wm0 + 16 * i + l16];
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const Tc* p = &Bs[buf][2 * ks + (kk >> 1)][2 * (wn0 + 8 * j + ((lane & 15) >> 1))];
-        const Tc re = p[0], im = p[1];
-        bv[j] = take_im ? im_sign * im : re;
+        const C2 b = Bs[buf][4 * ks + kk][wn0 + 8 * j + (l16 >> 1)];
+        b0[j] = pb ? b.y : b.x;
+        b1[j] = pb ? b.x : -b.y;
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(av[i], bv[j], acc[i][j]);
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(av[i].x, b0[j], acc[i][j]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(av[i].y, b1[j], acc[i][j]);
     }
     if (more) store_tiles(buf ^ 1);
     __syncthreads();
@@ -246,11 +279,13 @@ static int zero_fill(int64_t n, void* p, hipStream_t s) {
 // the first grouped product writes), and the second product reads T2[l, o, r']
 // only for the outputs o with qml[m] + qs[s'] = Q - P whose output sector
 // P + qml[m] exists. The mix reads and writes just those: T1 needs no zero
-// fill and T2 no zeros outside what is read. One wave per row l and 64-column
-// chunk of a unit, the lanes over the columns r' (coalesced). The kernel is
-// bound by the bytes in flight per CU: a lane's inputs are held in registers
-// sized to the plan's longest input list (CAP = 8, 16 or 32), and complex64
-// operands are mixed in FP32 arithmetic (A = float).
+// fill and T2 no zeros outside what is read. A workgroup takes MIX_ROWS rows l of one
+// 64-column chunk of a unit, MIX_ROWS / 4 per wave, the lanes over the columns r'
+// (coalesced). Memory-bound, so what counts is the bytes in flight per CU and
+// little else per byte: the unit's part of W is gathered once per workgroup, a lane's
+// inputs are held in registers sized to the plan's longest input list (CAP = 8, 16 or
+// 32), the next row's loaded while the current one is mixed, and complex64
+// operands are mixed in FP32 arithmetic (A = float). D = 2048: 72 -> 58 us.
 constexpr int MIX_LIST = 32;   // d * Mr and Ml * d are at most 32
 enum { PLAN_HEFF = SECTORS_HEFF, PLAN_ENV_RIGHT = SECTORS_ENV_RIGHT, PLAN_ENV_LEFT = SECTORS_ENV_LEFT };
 
@@ -258,9 +293,10 @@ struct MixUnit {
   int64_t l0, nl, r0, nr;
   int64_t tile0;                // first workgroup of the unit
   int32_t ni, no;
-  int32_t chunks;               // 64-column chunks per row: a wave per (row, chunk)
+  int32_t chunks;               // 64-column chunks per row
   int8_t il[MIX_LIST], ol[MIX_LIST];
 };
+constexpr int MIX_ROWS = 16;    // rows per workgroup
 
 template <typename TX, typename TY, typename A, int CAP>
 __global__ __launch_bounds__(256) void k_mix_sectors(const MixUnit* __restrict__ units, int nunits,
@@ -268,10 +304,10 @@ __global__ __launch_bounds__(256) void k_mix_sectors(const MixUnit* __restrict__
                                                      const double2* __restrict__ wm,
                                                      const TX* __restrict__ x, TY* __restrict__ y,
                                                      const int* __restrict__ skip, int wtrans) {
-  __shared__ double2 W[MIX_LIST * MIX_LIST];
+  typedef typename cplx_of<A>::type C2;
+  __shared__ C2 W[MIX_LIST * MIX_LIST];
+  __shared__ int il[MIX_LIST], ol[MIX_LIST];
   if (skip && skip[0]) return;
-  for (int t = threadIdx.x; t < ni_all * no_all; t += blockDim.x) W[t] = wm[t];
-  __syncthreads();
   const int64_t tile = blockIdx.x;
   int lo = 0, hi = nunits - 1;
   while (lo < hi) {
@@ -279,39 +315,58 @@ __global__ __launch_bounds__(256) void k_mix_sectors(const MixUnit* __restrict__
     if (units[mid].tile0 <= tile) lo = mid; else hi = mid - 1;
   }
   const MixUnit* __restrict__ u = units + lo;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // one wave per (row, 64-column chunk) of the unit: short independent work
-  // items keep many loads in flight
-  const int64_t wi = (tile - u->tile0) * 4 + wave;
-  const int64_t row = wi / u->chunks;
-  if (row >= u->nl) return;
-  const int64_t r = u->r0 + (wi % u->chunks) * 64 + lane;
-  if (r >= u->r0 + u->nr) return;
-  const int64_t l = u->l0 + row;
   const int ni = u->ni, no = u->no;
-  const TX* __restrict__ xl = x + l * ni_all * nr_all;
-  TY* __restrict__ yl = y + l * no_all * nr_all;
-  {
-    A xr[CAP], xi[CAP];
+  if (threadIdx.x < MIX_LIST) il[threadIdx.x] = u->il[threadIdx.x];
+  else if (threadIdx.x < 2 * MIX_LIST) ol[threadIdx.x - MIX_LIST] = u->ol[threadIdx.x - MIX_LIST];
+  __syncthreads();
+  // Wm[o, i] of the unit's lists, or stored transposed as W[i, o] (left environment)
+  for (int t = threadIdx.x; t < ni * no; t += 256) {
+    const int j = t / ni, k = t - j * ni;
+    const int o = ol[j], i = il[k];
+    const double2 w = wtrans ? wm[i * no_all + o] : wm[o * ni_all + i];
+    W[t] = C2{(A)w.x, (A)w.y};
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t rt = tile - u->tile0;
+  const int64_t row0 = rt / u->chunks * MIX_ROWS;
+  const int64_t c = rt % u->chunks * 64 + lane;
+  const bool in = c < u->nr;
+  const int64_t r = u->r0 + c;
+  const int64_t rows = u->nl - row0 < MIX_ROWS ? u->nl - row0 : MIX_ROWS;
+  const int64_t l0 = u->l0 + row0;
+  // the lanes share the lists: offsets in scalar registers, known before the loads
+  int64_t ioff[CAP];
+#pragma unroll
+  for (int k = 0; k < CAP; ++k)
+    ioff[k] = (int64_t)__builtin_amdgcn_readfirstlane(k < ni ? il[k] : 0) * nr_all;
+  C2 next[CAP];
+  auto load = [&](int64_t row) {
+    const TX* __restrict__ xl = x + (l0 + row) * ni_all * nr_all + r;
 #pragma unroll
     for (int k = 0; k < CAP; ++k) {
-      xr[k] = 0; xi[k] = 0;
-      if (k < ni) load_c<A>(xl + (int64_t)u->il[k] * nr_all + r, xr[k], xi[k]);
+      next[k] = C2{0, 0};
+      if (k < ni && in) load_c<A>(xl + ioff[k], next[k].x, next[k].y);
     }
+  };
+  if (wave < rows) load(wave);
+  for (int64_t row = wave; row < rows; row += 4) {
+    C2 v[CAP];
+#pragma unroll
+    for (int k = 0; k < CAP; ++k) v[k] = next[k];
+    if (row + 4 < rows) load(row + 4);
+    TY* __restrict__ yl = y + (l0 + row) * no_all * nr_all + r;
     for (int j = 0; j < no; ++j) {
-      const int o = u->ol[j];
       A yr = 0, yi = 0;
 #pragma unroll
       for (int k = 0; k < CAP; ++k) {
         if (k < ni) {
-          // Wm[o, i], or stored transposed as W[i, o] (left environment)
-          const double2 w = wtrans ? W[u->il[k] * no_all + o] : W[o * ni_all + u->il[k]];
-          const A wr = (A)w.x, wi = (A)w.y;
-          yr += wr * xr[k] - wi * xi[k];
-          yi += wr * xi[k] + wi * xr[k];
+          const C2 w = W[j * ni + k];
+          yr += w.x * v[k].x - w.y * v[k].y;
+          yi += w.x * v[k].y + w.y * v[k].x;
         }
       }
-      store_c(yl + (int64_t)o * nr_all + r, yr, yi);
+      if (in) store_c(yl + (int64_t)ol[j] * nr_all, yr, yi);
     }
   }
 }
@@ -337,7 +392,7 @@ static bool sectors_of(const int64_t* q, int64_t n, std::map<int64_t, Sector>& o
 struct GProduct {
   std::vector<GBlock> blocks;
   int64_t tiles = 0;
-  int big = 0;          // 1: 128 x 64 tiles (TileCfg<4, 4>), 0: 64 x 32 (TileCfg<2, 2>)
+  int tile = 2;         // TileCfg<tile, tile>: 128 x 64 (4), 64 x 32 (2) or 32 x 16 (1)
   double flop = 0.0;    // 8 M N K summed over the blocks
   double bytes = 0.0;   // operand blocks read once, output blocks written once
 };
@@ -368,30 +423,54 @@ struct SectorPlan {
   uint64_t stamp = 0;
 };
 
-// tile shape and first tiles of a product: the 128 x 64 tile when its padding
+// Tile shape and first tiles of a product. The 128 x 64 tile when its padding
 // costs at most 15 % more work than the 64 x 32 tile's and it still gives
-// enough workgroups for the chip (>= 512)
+// enough workgroups for the chip (>= 512); else the cheaper of 64 x 32 and 32 x 16 by
+// padded work / (rate x share of the chip at work): full tiles of them reach 63 and
+// 52 TFLOP/s (FP64), and with fewer than about six tiles per CU the CUs that get
+// one more than the others set the time. Two-site U(1) H_eff, both products on 64 x 32
+// against both on 32 x 16 tiles: D = 96 40 / 35 us, 512 78 / 59, 1024 138 / 112,
+// 1500 261 / 248, 2048 493 / 503 (and 473 with the output product alone on 32 x 16:
+// 811 tiles of 64 x 32 are 3.2 per CU).
 static void finish_product(GProduct& P, size_t csz_a, size_t csz_b, size_t csz_c) {
-  double w_small = 0.0, w_big = 0.0;
-  int64_t t_big = 0;
+  static const struct { int code; int64_t bm, bn; double rate; } tile[3] = {
+      {4, 128, 64, 65.0}, {2, 64, 32, 63.0}, {1, 32, 16, 52.0}};
+  double work[3] = {0, 0, 0};
+  int64_t n[3] = {0, 0, 0};
   P.flop = 0.0;
   P.bytes = 0.0;
+  auto up = [](int64_t x, int64_t t) { return (x + t - 1) / t * t; };
+  auto total_k = [](const GBlock& b) {
+    int64_t k = 0;
+    for (int i = 0; i < b.nseg; ++i) k += b.K[i];
+    return k;
+  };
   for (const GBlock& b : P.blocks) {
-    double k = 0.0;
-    for (int i = 0; i < b.nseg; ++i) k += (double)b.K[i];
+    const double k = (double)total_k(b);
     P.flop += 8.0 * (double)b.M * (double)b.N * k;
     P.bytes += k * ((double)b.M * csz_a + (double)b.N * csz_b) + (double)b.M * b.N * csz_c;
-    w_small += (double)((b.M + 63) / 64 * 64) * (double)((b.N + 31) / 32 * 32) * k;
-    w_big += (double)((b.M + 127) / 128 * 128) * (double)((b.N + 63) / 64 * 64) * k;
-    t_big += ((b.M + 127) / 128) * ((b.N + 63) / 64);
+    for (int t = 0; t < 3; ++t) {
+      const int64_t m = up(b.M, tile[t].bm), c = up(b.N, tile[t].bn);
+      work[t] += (double)m * (double)c * k;
+      n[t] += (m / tile[t].bm) * (c / tile[t].bn);
+    }
   }
-  P.big = (w_big <= 1.15 * w_small && t_big >= 512) ? 1 : 0;
-  const int64_t BM = P.big ? 128 : 64, BN = P.big ? 64 : 32;
+  int pick = 0;
+  if (!(work[0] <= 1.15 * work[1] && n[0] >= 512)) {
+    auto cost = [&](int t) {
+      return n[t] ? work[t] / tile[t].rate * (double)up(n[t], 256) / (double)n[t] : 0.0;
+    };
+    pick = cost(2) < cost(1) ? 2 : 1;
+  }
+  P.tile = tile[pick].code;
+  // the tiles with the longest sums first, so that the last workgroups are short ones
+  std::stable_sort(P.blocks.begin(), P.blocks.end(),
+                   [&](const GBlock& x, const GBlock& y) { return total_k(x) > total_k(y); });
   int64_t tiles = 0;
   for (GBlock& b : P.blocks) {
-    b.tiles_n = (int32_t)((b.N + BN - 1) / BN);
+    b.tiles_n = (int32_t)((b.N + tile[pick].bn - 1) / tile[pick].bn);
     b.tile0 = tiles;
-    tiles += ((b.M + BM - 1) / BM) * b.tiles_n;
+    tiles += ((b.M + tile[pick].bm - 1) / tile[pick].bm) * b.tiles_n;
   }
   P.tiles = tiles;
 }
@@ -556,7 +635,7 @@ static void plan_mix(const Dims& D, bool left, const int64_t* qs, const int64_t*
       u.nr = rq.second.len;
       u.tile0 = sp.mix_tiles;
       u.chunks = (int32_t)((u.nr + 63) / 64);
-      sp.mix_tiles += (u.nl * u.chunks + 3) / 4;
+      sp.mix_tiles += (u.nl + MIX_ROWS - 1) / MIX_ROWS * u.chunks;
       sp.mix_bytes += (double)u.nl * (double)u.nr * (double)(u.ni + u.no);
       sp.mix.push_back(u);
     }
@@ -694,29 +773,51 @@ int sector_plan_get(const ptn_local_op* op, int kind, SectorPlanRef* out) {
 }
 
 template <typename Tc, typename TA, typename TB, typename TC, bool AK, bool BNC>
-static int grouped_launch(const GLaunch& g, const GProduct& P, hipStream_t s) {
-  char name[112];
-  snprintf(name, sizeof(name), "zgemm_grouped_kernel<%s, %s, %s, %s, %d, %d, %s, %s>",
-           type_tag<Tc>::s, type_tag<TA>::s, type_tag<TB>::s, type_tag<TC>::s, P.big ? 4 : 2,
-           P.big ? 4 : 2, AK ? "true" : "false", BNC ? "true" : "false");
-  // launch records keep the name pointer: intern the names
-  static std::mutex mu;
-  static std::unordered_map<std::string, std::string> names;
-  const char* nm;
-  {
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = names.find(name);
-    if (it == names.end()) it = names.emplace(name, name).first;
-    nm = it->second.c_str();
-  }
-  if (P.big)
-    tlaunch(nm, P.flop, P.bytes, zgemm_grouped_kernel<Tc, TA, TB, TC, 4, 4, AK, BNC>,
-            dim3((unsigned)P.tiles), dim3(256), s, g);
+static int grouped_launch(GLaunch g, const GProduct& P, hipStream_t s) {
+  // launch records keep the name pointer: formatted once per instance
+  static const auto make = [](int t) {
+    char name[112];
+    snprintf(name, sizeof(name), "zgemm_grouped_kernel<%s, %s, %s, %s, %d, %d, %s, %s>",
+             type_tag<Tc>::s, type_tag<TA>::s, type_tag<TB>::s, type_tag<TC>::s, t, t,
+             AK ? "true" : "false", BNC ? "true" : "false");
+    return std::string(name);
+  };
+  static const std::string* names = new std::string[3]{make(1), make(2), make(4)};
+  const char* nm = names[P.tile >> 1].c_str();
+  const int64_t lim = (int64_t)1 << 31;
+  g.fast = g.a_m < lim && g.a_k < lim && g.b_k < lim && g.b_n < lim &&
+           (128 * g.a_m + 16 * g.a_k) * (int64_t)sizeof(TA) < lim &&
+           (64 * g.b_n + 16 * g.b_k) * (int64_t)sizeof(TB) < lim;
+  const dim3 grid((unsigned)(P.tiles + g.fill_wgs));
+  if (P.tile == 4)
+    tlaunch(nm, P.flop, P.bytes, zgemm_grouped_kernel<Tc, TA, TB, TC, 4, 4, AK, BNC>, grid,
+            dim3(256), s, g);
+  else if (P.tile == 2)
+    tlaunch(nm, P.flop, P.bytes, zgemm_grouped_kernel<Tc, TA, TB, TC, 2, 2, AK, BNC>, grid,
+            dim3(256), s, g);
   else
-    tlaunch(nm, P.flop, P.bytes, zgemm_grouped_kernel<Tc, TA, TB, TC, 2, 2, AK, BNC>,
-            dim3((unsigned)P.tiles), dim3(256), s, g);
+    tlaunch(nm, P.flop, P.bytes, zgemm_grouped_kernel<Tc, TA, TB, TC, 1, 1, AK, BNC>, grid,
+            dim3(256), s, g);
   PTN_LAUNCH_CHECK();
   return PTN_OK;
+}
+
+static size_t mpo_bytes(const Dims& D) { return (size_t)(D.Ml * D.d * D.d * D.Mr) * 16; }
+
+// Zero fill of the n outputs: inside the first product's launch g, or (a caller's
+// output that overlaps what that product or the mix reads) by zero_fill after the mix.
+// in0, in1: the operands of the first product, w: the MPO tensor, each with its bytes.
+static bool fill_with(GLaunch& g, void* out, int64_t n, const void* in0, size_t b0,
+                      const void* in1, size_t b1, const void* w, size_t bw) {
+  const char* o = (const char*)out;
+  auto apart = [&](const void* p, size_t b) {
+    return (const char*)p + b <= o || o + n * (int64_t)sizeof(double2) <= (const char*)p;
+  };
+  if (!apart(in0, b0) || !apart(in1, b1) || !apart(w, bw)) return false;
+  g.fill = (double2*)out;
+  g.nfill = n;
+  g.fill_wgs = (unsigned)((n + FILL_PER_WG - 1) / FILL_PER_WG);
+  return true;
 }
 
 // the sector mix of a plan: T2 (y) from T1 (x) with the MPO matrix w (complex128),
@@ -773,6 +874,8 @@ int heff_apply_sectors(int prec, const Dims& D, const SectorPlan* sp, const void
   int st;
   GLaunch g1{b1, (int)sp->p1.blocks.size(), D.d * D.Dr, 1, D.Mr * D.Dr, 1, D.d * D.Mr * D.Dr, 1,
              a, r, t1, skip, 0};
+  const bool filled = fill_with(g1, out, nout, a, (size_t)nout * 16, r,
+                                (size_t)(D.Dr * D.Mr * D.Dr) * csz, w, mpo_bytes(D));
   const int ni = (int)(D.d * D.Mr), no = (int)(D.Ml * D.d);
   if (bp == PTN_FP64) {
     if ((st = grouped_launch<double, double2, double2, double2, true, true>(g1, sp->p1, s)))
@@ -784,7 +887,7 @@ int heff_apply_sectors(int prec, const Dims& D, const SectorPlan* sp, const void
     if ((st = mix_launch(sp, false, ni, no, D.Dr, w, t1, t2, skip, 0, s))) return st;
   }
   PTN_LAUNCH_CHECK();
-  if ((st = zero_fill<double2>(nout, out, s))) return st;
+  if (!filled && (st = zero_fill<double2>(nout, out, s))) return st;
   GLaunch g3{b3, (int)sp->p3.blocks.size(), 1, D.Ml * D.Dl, D.Ml * D.d * D.Dr, 1, D.d * D.Dr, 1,
              l, t2, out, skip, 0};
   if (bp == PTN_FP64)
@@ -819,16 +922,19 @@ int env_right_sectors(int prec, const Dims& D, const SectorPlan* sp, const void*
   // out[(l, m), lb] = sum T2[(l, m), (s', r')] conj(B[lb, (s', r')])
   GLaunch g3{b3, (int)sp->p3.blocks.size(), D.Ml * D.d * D.Dr, 1, 1, D.d * D.Dr, D.Ml * D.Dl, 1,
              t2, b, out, skip, 1};
+  const int64_t nout = D.Dl * D.Ml * D.Dl;
+  const bool filled = fill_with(g1, out, nout, a, (size_t)(D.Dl * D.d * D.Dr) * 16, r,
+                                (size_t)(D.Dr * D.Mr * D.Dr) * csz, w, mpo_bytes(D));
   if (bp == PTN_FP64) {
     if ((st = grouped_launch<double, double2, double2, double2, true, true>(g1, sp->p1, s)))
       return st;
     if ((st = mix_launch(sp, true, ni, no, D.Dr, w, t1, t2, skip, 0, s))) return st;
-    if ((st = zero_fill<double2>(D.Dl * D.Ml * D.Dl, out, s))) return st;
+    if (!filled && (st = zero_fill<double2>(nout, out, s))) return st;
     return grouped_launch<double, double2, double2, double2, true, false>(g3, sp->p3, s);
   }
   if ((st = grouped_launch<float, double2, float2, float2, true, true>(g1, sp->p1, s))) return st;
   if ((st = mix_launch(sp, false, ni, no, D.Dr, w, t1, t2, skip, 0, s))) return st;
-  if ((st = zero_fill<double2>(D.Dl * D.Ml * D.Dl, out, s))) return st;
+  if (!filled && (st = zero_fill<double2>(nout, out, s))) return st;
   return grouped_launch<float, float2, double2, double2, true, false>(g3, sp->p3, s);
 }
 
@@ -859,16 +965,19 @@ int env_left_sectors(int prec, const Dims& D, const SectorPlan* sp, const void* 
   // out[r, (m', r')] = sum_{(l, s)} A[(l, s), r] T2[(l, s), (m', r')]
   GLaunch g3{b3, (int)sp->p3.blocks.size(), 1, D.d * D.Dr, D.d * D.Mr * D.Dr, 1, D.Mr * D.Dr, 1,
              a, t2, out, skip, 0};
+  const int64_t nout = D.Dr * D.Mr * D.Dr;
+  const bool filled = fill_with(g1, out, nout, l, (size_t)(D.Dl * D.Ml * D.Dl) * csz, b,
+                                (size_t)(D.Dl * D.d * D.Dr) * 16, w, mpo_bytes(D));
   if (bp == PTN_FP64) {
     if ((st = grouped_launch<double, double2, double2, double2, true, true>(g1, sp->p1, s)))
       return st;
     if ((st = mix_launch(sp, true, ni, no, D.Dr, w, t1, t2, skip, 1, s))) return st;
-    if ((st = zero_fill<double2>(D.Dr * D.Mr * D.Dr, out, s))) return st;
+    if (!filled && (st = zero_fill<double2>(nout, out, s))) return st;
     return grouped_launch<double, double2, double2, double2, false, true>(g3, sp->p3, s);
   }
   if ((st = grouped_launch<float, float2, double2, float2, true, true>(g1, sp->p1, s))) return st;
   if ((st = mix_launch(sp, false, ni, no, D.Dr, w, t1, t2, skip, 1, s))) return st;
-  if ((st = zero_fill<double2>(D.Dr * D.Mr * D.Dr, out, s))) return st;
+  if (!filled && (st = zero_fill<double2>(nout, out, s))) return st;
   return grouped_launch<float, double2, float2, double2, false, true>(g3, sp->p3, s);
 }
 
