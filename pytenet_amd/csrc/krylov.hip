@@ -9,11 +9,14 @@
 // round trip. A breakdown or a non-finite value stops the recurrence through a
 // flag that later kernels read; the host reads the status words afterwards.
 #include <float.h>
+#include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <unordered_map>
 #include "common.h"
 #include "ops.h"
+#include "wave.h"
 
 namespace ptn {
 
@@ -70,9 +73,8 @@ __device__ void block_store_partial(double v, double* out) {
   if (t == 0) out[blockIdx.x] = red[0];
 }
 
-__global__ __launch_bounds__(256) void k_state_init(LzState* st, int numiter) {
-  st += blockIdx.x;
-  int t = threadIdx.x;
+__device__ __forceinline__ void state_init(LzState* st, int numiter) {
+  const int t = threadIdx.x;
   if (t < LZ_MAX) {
     st->alpha[t] = 0; st->beta[t] = 0; st->coef_re[t] = 0; st->coef_im[t] = 0;
   }
@@ -84,7 +86,8 @@ __global__ __launch_bounds__(256) void k_state_init(LzState* st, int numiter) {
 
 __global__ __launch_bounds__(256) void k_sumsq_partial(int64_t n, const double2* __restrict__ x,
                                                        int64_t xs, double* __restrict__ part,
-                                                       int rb) {
+                                                       int rb, LzState* st, int numiter) {
+  if (blockIdx.x == 0) state_init(st + blockIdx.y, numiter);
   x += blockIdx.y * xs;
   part += blockIdx.y * rb;
   double s = 0;
@@ -211,130 +214,391 @@ __global__ __launch_bounds__(256) void k_beta_next(int64_t n, const double2* __r
   }
 }
 
-// last alpha (krylov.py:54-56); one block per problem
-__global__ __launch_bounds__(256) void k_alpha_last(int j, const double* __restrict__ part_in,
-                                                    int rb, LzState* st) {
+// Short vectors: one workgroup per problem keeps its part of the vectors in registers
+// and does all of a step at once, R elements per thread (n <= 1024 R). Such a step is bound
+// by launches and by the latency of dependent loads and sums. A Lanczos step (inner product,
+// update, normalisation) as three launches of 256-thread workgroups and as one: n = 1024 2.7 + 3.9
+// + 3.5 -> 4.5 us, 4096 -> 6.5 us, 8192 10.4 -> 11.0 us with two launches and their gaps
+// fewer; at 16384 one CU's bandwidth would cost more (the registers spill: 45 us).
+constexpr int SHORT_T = 1024;     // largest workgroup
+constexpr int64_t SHORT_MAX = 8 * SHORT_T;
+
+// barrier that orders LDS accesses only: stores to memory that only the threads which
+// made them read back stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// sum over the workgroup (up to 16 waves) in a fixed order, in every thread: the sums of
+// each wave's rows of 16 lanes through LDS, then lane l of a row adds those of wave l. red
+// is not written again until the caller's next barrier after it.
+__device__ __forceinline__ double row_sum(double v) {
+  v += dpp_rot<0x128>(v);   // row rotate right by 8, 4, 2, 1
+  v += dpp_rot<0x124>(v);
+  v += dpp_rot<0x122>(v);
+  v += dpp_rot<0x121>(v);
+  return v;
+}
+__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4]) {
+  v = row_sum(v);
+  const int t = threadIdx.x, w = t & 15;
+  if (w == 0) red[t >> 6][(t >> 4) & 3] = v;
+  lds_barrier();
+  const double s = (red[w][0] + red[w][1]) + (red[w][2] + red[w][3]);
+  return row_sum(w < (int)(blockDim.x >> 6) ? s : 0.0);
+}
+
+// x / b from inv = 1 / b with one correction (b a normal number)
+__device__ __forceinline__ double div_by(double x, double b, double inv) {
+  const double q = x * inv;
+  return fma(fma(-q, b, x), inv, q);
+}
+
+// state, norm of the start vector and v0 = x / |x|  (krylov.py:29-31)
+template <int R>
+__global__ __launch_bounds__(SHORT_T) void k_lz_start(int n, const double2* __restrict__ x,
+                                                      double2* __restrict__ v0, LzState* st,
+                                                      int numiter) {
+  __shared__ __align__(16) double red[16][4];
+  x += (int64_t)blockIdx.x * n;
+  v0 += (int64_t)blockIdx.x * n;
   st += blockIdx.x;
-  if (st->stopped) return;
-  const double a = block_sum_partials(part_in + blockIdx.x * rb, rb);
+  const int nt = blockDim.x;
+  double2 a[R];
+  double s = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = threadIdx.x + r * nt;
+    a[r] = i < n ? x[i] : make_double2(0.0, 0.0);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) s += a[r].x * a[r].x + a[r].y * a[r].y;
+  state_init(st, numiter);
+  const double nrm = sqrt(wg_sum(s, red));
+  const bool bad = !(nrm > 0.0) || !isfinite(nrm);
   if (threadIdx.x == 0) {
-    st->alpha[j] = a;
-    if (!isfinite(a)) st->nonfinite = 1;
+    st->nrm0 = nrm;
+    if (bad) {
+      if (nrm == 0.0) st->zero_start = 1; else st->nonfinite = 1;
+      st->stopped = 1;
+      st->nvalid = 0;
+    }
+  }
+  if (bad) return;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = threadIdx.x + r * nt;
+    if (i < n) v0[i] = make_double2(a[r].x / nrm, a[r].y / nrm);
   }
 }
 
-// Eigendecomposition of the nv x nv tridiagonal matrix by the implicit QL
-// method with Wilkinson shifts (one wave: every lane runs the same scalar
-// recurrence on the diagonal/off-diagonal, lane k applies the plane
-// rotations to row k of the eigenvector matrix), eigenvalues sorted
-// ascending as numpy.linalg.eigh returns them; then the coefficients:
-//   mode 0 (expm):  c = U (|v| exp(dt lambda) * U[0, :])    (krylov.py:132-136)
-//   mode 1 (eigh):  c = U[:, 0], energy = lambda_0          (krylov.py:116-119)
-__global__ __launch_bounds__(64) void k_tridiag(LzState* st, int mode, double dt_re,
-                                                double dt_im) {
+// alpha_j, the update of w, beta_j with the breakdown test and v_{j+1} = w / beta_j (the
+// formulas of k_dot_partial, k_alpha_update and k_beta_next); w is only read
+template <int R>
+__global__ __launch_bounds__(SHORT_T) void k_lz_step(int n, const double2* __restrict__ w,
+                                                     const double2* __restrict__ vj,
+                                                     const double2* __restrict__ vjm1,
+                                                     double2* __restrict__ vnext, int j,
+                                                     double thresh, double rel, LzState* st) {
+  __shared__ __align__(16) double red[2][16][4];
   st += blockIdx.x;
-  __shared__ double d[LZ_MAX], e[LZ_MAX];
-  __shared__ double Z[LZ_MAX][LZ_MAX + 1];
-  __shared__ double tre[LZ_MAX], tim[LZ_MAX];
-  const int lane = threadIdx.x;
-  const int n = st->nvalid;
-  if (n <= 0 || st->nonfinite) return;
-  d[lane] = (lane < n) ? st->alpha[lane] : 0.0;
-  e[lane] = (lane < n - 1) ? st->beta[lane] : 0.0;
-  for (int k = 0; k < LZ_MAX; ++k) Z[lane][k] = (lane == k) ? 1.0 : 0.0;
-  __syncthreads();
-  int noconv = 0;
+  if (st->stopped) return;
+  const int64_t o = (int64_t)blockIdx.x * n;
+  w += o;
+  vj += o;
+  vjm1 += o;
+  vnext += o;
+  const int nt = blockDim.x;
+  const double2 zero = make_double2(0.0, 0.0);
+  constexpr bool KEEP = R <= 4;   // v_j and v_{j-1} stay in registers from the first read on
+  double2 x[R], v[KEEP ? R : 1], u[KEEP ? R : 1];
+  double s = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = threadIdx.x + r * nt;
+    x[r] = i < n ? w[i] : zero;
+    if constexpr (KEEP) {
+      v[r] = i < n ? vj[i] : zero;
+      u[r] = j > 0 && i < n ? vjm1[i] : zero;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = threadIdx.x + r * nt;
+    const double2 b = KEEP ? v[KEEP ? r : 0] : (i < n ? vj[i] : zero);
+    s += x[r].x * b.x + x[r].y * b.y;
+    if (!KEEP && (r & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // loads of four at a time
+  }
+  const double b0 = j > 0 ? st->beta[j - 1] : 0.0;
+  const double a = wg_sum(s, red[0]);
+  if (threadIdx.x == 0) st->alpha[j] = a;
+  if (!isfinite(a)) {
+    if (threadIdx.x == 0) { st->nonfinite = 1; st->stopped = 1; st->nvalid = j + 1; }
+    return;
+  }
+  s = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = threadIdx.x + r * nt;
+    const double2 vr = KEEP ? v[KEEP ? r : 0] : (i < n ? vj[i] : zero);
+    double tr = a * vr.x, ti = a * vr.y;
+    if (j > 0) {
+      const double2 ur = KEEP ? u[KEEP ? r : 0] : (i < n ? vjm1[i] : zero);
+      tr += b0 * ur.x;
+      ti += b0 * ur.y;
+    }
+    x[r].x -= tr;
+    x[r].y -= ti;
+    s += x[r].x * x[r].x + x[r].y * x[r].y;
+    if (!KEEP && (r & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+  const double b = sqrt(wg_sum(s, red[1]));
+  const bool nf = !isfinite(b);
+  const bool brk = !nf && b < fmax(thresh, rel * sqrt(a * a + b0 * b0 + b * b));
+  if (threadIdx.x == 0) {
+    if (nf) { st->nonfinite = 1; st->stopped = 1; st->nvalid = j + 1; }
+    else if (brk) { st->breakdown = j + 1; st->stopped = 1; st->nvalid = j + 1; }
+    else st->beta[j] = b;
+  }
+  if (nf || brk) return;
+  const double inv = 1.0 / b;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = threadIdx.x + r * nt;
+    if (i < n) vnext[i] = make_double2(div_by(x[r].x, b, inv), div_by(x[r].y, b, inv));
+  }
+}
+
+// the value of the next (UP) or the previous lane of the wave, zero beyond its ends
+template <bool UP> __device__ __forceinline__ double lane_shift(double v) {
+  constexpr int CTRL = UP ? 0x130 : 0x138;   // wave shift left / right by one lane
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double wave_max(double v) {
+  v = fmax(v, dpp_rot<0x128>(v));
+  v = fmax(v, dpp_rot<0x124>(v));
+  v = fmax(v, dpp_rot<0x122>(v));
+  v = fmax(v, dpp_rot<0x121>(v));
+  return fmax(fmax(lane_value(v, 0), lane_value(v, 16)),
+              fmax(lane_value(v, 32), lane_value(v, 48)));
+}
+
+// Coefficients of the Krylov vectors from the tridiagonal matrix (alpha, beta) of n
+// rows, by one wave (lane k holds row k in registers and returns coefficient k):
+//   mode 0 (expm):  c = |v| exp(dt T) e_1                              (krylov.py:132-136)
+//   mode 1 (eigh):  c = the eigenvector of the lowest eigenvalue, its energy (krylov.py:116-119)
+// The exponential is applied to e_1 by Taylor polynomials of degree 18 in Horner's form, in
+// steps of |dt| rho <= 1 with T shifted to the centre of its Gershgorin interval of radius rho
+// (the remainder is below 2^-56): a step is 18 products with a tridiagonal matrix, neighbours
+// read across the lanes. Up to 16 steps; beyond them, and for mode 1, the
+// eigendecomposition below. Error against 50 digits, norm of the result = 1, |dt| rho =
+// 0.01 .. 16, imaginary, real and complex dt: 3e-17 .. 9e-16 in the median, largest
+// 3.2e-15; from the eigendecomposition (LAPACK) 4e-16 .. 6e-15 and 2.4e-13.
+// The last kernel of a solve at n = 10 takes 4 - 6 us with it.
+//
+// Eigendecomposition by the implicit QL method with Wilkinson shifts: every lane runs
+// the same scalar recurrence on values read as scalars, and lane k applies the plane rotations
+// to row k of the eigenvector matrix (Z, rows of ldz doubles in LDS). The chain of
+// dependent operations of the rotations (about 1.7 n sweeps of n / 2) sets its time:
+// r = sqrt(f^2 + g^2), f / r and g / r come from one reciprocal square root (hypot where
+// the squares leave the normal range): 25 - 38 us at n = 8 - 10 (40 - 58 with hypot and divisions
+// in every rotation and the matrix's diagonals in LDS).
+constexpr double TAYLOR_MAX_STEPS = 16.0;
+__device__ __forceinline__ bool tridiag_coefs(int n, const double* alpha, const double* beta,
+                                              double* Z, int ldz, int mode, double nrm,
+                                              double dt_re, double dt_im, double& cr, double& ci,
+                                              double& energy) {
+  const int lane = threadIdx.x & 63;
+  double d = lane < n ? alpha[lane] : 0.0;
+  double e = lane < n - 1 ? beta[lane] : 0.0;
+  cr = ci = 0.0;
+  if (mode == 0) {
+    const double em = lane_shift<false>(e);          // coupling to the previous row
+    const double off = fabs(e) + fabs(em);
+    const double hi = wave_max(lane < n ? d + off : -INFINITY);
+    const double lo = -wave_max(lane < n ? off - d : -INFINITY);
+    const double mid = 0.5 * (lo + hi), rho = 0.5 * (hi - lo);
+    const double steps = fmax(ceil(rho * hypot(dt_re, dt_im)), 1.0);
+    if (steps <= TAYLOR_MAX_STEPS) {
+      const double zr = dt_re / steps, zi = dt_im / steps, dc = d - mid;
+      double x = lane == 0 ? 1.0 : 0.0, y = 0.0;
+      for (int q = (int)steps; q > 0; --q) {
+        const double x0 = x, y0 = y;
+#pragma unroll
+        for (int k = 18; k > 0; --k) {
+          const double kr = zr * (1.0 / k), ki = zi * (1.0 / k);
+          const double tx = fma(dc, x, fma(e, lane_shift<true>(x), em * lane_shift<false>(x)));
+          const double ty = fma(dc, y, fma(e, lane_shift<true>(y), em * lane_shift<false>(y)));
+          x = fma(kr, tx, fma(-ki, ty, x0));
+          y = fma(kr, ty, fma(ki, tx, y0));
+        }
+      }
+      const double mag = nrm * exp(dt_re * mid), ph = dt_im * mid;
+      const double er = mag * cos(ph), ei = mag * sin(ph);
+      cr = er * x - ei * y;
+      ci = er * y + ei * x;
+      return true;
+    }
+  }
+  double* zrow = Z + (lane < n ? lane : 0) * ldz;
+  if (lane < n)
+    for (int k = 0; k < n; ++k) zrow[k] = lane == k ? 1.0 : 0.0;
+  bool conv = true;
   for (int l = 0; l < n; ++l) {
     int iter = 0;
     for (;;) {
-      int m = l;
-      while (m < n - 1) {
-        const double dd = fabs(d[m]) + fabs(d[m + 1]);
-        if (fabs(e[m]) <= DBL_EPSILON * dd) break;
-        ++m;
-      }
+      const bool tiny = lane >= l && lane < n - 1 &&
+                        fabs(e) <= DBL_EPSILON * (fabs(d) + fabs(lane_shift<true>(d)));
+      const unsigned long long at = __ballot(tiny);
+      const int m = at ? __ffsll(at) - 1 : n - 1;
       if (m == l) break;
-      if (++iter > 100) { noconv = 1; break; }
+      if (++iter > 100) { conv = false; break; }
       // shift from the leading 2 x 2 block of the unreduced part
-      double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
-      double r = hypot(g, 1.0);
-      g = d[m] - d[l] + e[l] / (g + copysign(r, g));
+      const double dl = lane_value(d, l), el = lane_value(e, l);
+      double g = (lane_value(d, l + 1) - dl) / (2.0 * el);
+      double r = fabs(g) < 1e150 ? sqrt(fma(g, g, 1.0)) : fabs(g);
+      g = lane_value(d, m) - dl + el / (g + copysign(r, g));
       double s = 1.0, c = 1.0, p = 0.0;
+      double dh = lane_value(d, m);    // d[i + 1]
+      double zh = zrow[m];             // Z[.][i + 1]
       bool split = false;
-      for (int i = m - 1; i >= l; --i) {
-        const double f = s * e[i];
-        const double b = c * e[i];
-        r = hypot(f, g);
-        e[i + 1] = r;
-        if (r == 0.0) {
-          d[i + 1] -= p;
-          e[m] = 0.0;
-          split = true;
-          break;
+      int i = m - 1;
+      for (; i >= l; --i) {
+        const double ei = lane_value(e, i), di = lane_value(d, i), z0 = zrow[i];
+        const double f = s * ei;
+        const double b = c * ei;
+        const double h = fma(f, f, g * g);
+        if (h > 1e-280 && h < 1e280) {
+          const double ri = rsq_full(h);
+          r = h * ri;
+          s = f * ri;
+          c = g * ri;
+        } else {
+          r = hypot(f, g);
+          if (r == 0.0) {
+            if (lane == i + 1) { d = dh - p; e = 0.0; }
+            if (lane == m) e = 0.0;
+            split = true;
+            break;
+          }
+          s = f / r;
+          c = g / r;
         }
-        s = f / r;
-        c = g / r;
-        g = d[i + 1] - p;
-        r = (d[i] - g) * s + 2.0 * c * b;
-        p = s * r;
-        d[i + 1] = g + p;
-        g = c * r - b;
-        const double z1 = Z[lane][i + 1], z0 = Z[lane][i];
-        Z[lane][i + 1] = s * z0 + c * z1;
-        Z[lane][i] = c * z0 - s * z1;
+        if (lane == i + 1) e = r;
+        g = dh - p;
+        const double t = fma(di - g, s, 2.0 * c * b);
+        p = s * t;
+        if (lane == i + 1) d = g + p;
+        g = fma(c, t, -b);
+        zrow[i + 1] = s * z0 + c * zh;
+        zh = c * z0 - s * zh;
+        dh = di;
       }
+      zrow[i + 1] = zh;
       if (split) continue;
-      d[l] -= p;
-      e[l] = g;
-      e[m] = 0.0;
+      if (lane == l) { d -= p; e = g; }
+      if (lane == m) e = 0.0;
     }
   }
-  // ascending order (selection sort; the permutation is identical in every lane)
-  for (int i = 0; i < n - 1; ++i) {
-    int k = i;
-    double dm = d[i];
-    for (int j = i + 1; j < n; ++j)
-      if (d[j] < dm) { dm = d[j]; k = j; }
-    if (k != i) {
-      const double t = d[i];
-      d[k] = t;
-      d[i] = dm;
-      const double zt = Z[lane][i];
-      Z[lane][i] = Z[lane][k];
-      Z[lane][k] = zt;
-    }
-  }
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
   if (mode == 0) {
-    if (lane < n) {
-      // |v| * exp(dt * lambda_j) * U[0, j]
-      const double lam = d[lane];
-      const double mag = exp(dt_re * lam);
-      const double ph = dt_im * lam;
-      const double er = st->nrm0 * (mag * cos(ph));
-      const double ei = st->nrm0 * (mag * sin(ph));
-      tre[lane] = er * Z[0][lane];
-      tim[lane] = ei * Z[0][lane];
-    }
-    __syncthreads();
-    if (lane < n) {
-      double cr = 0, ci = 0;
-      for (int j = 0; j < n; ++j) {
-        cr += Z[lane][j] * tre[j];
-        ci += Z[lane][j] * tim[j];
-      }
-      st->coef_re[lane] = cr;
-      st->coef_im[lane] = ci;
+    // |v| * exp(dt * lambda_j) * U[0, j] in lane j
+    const double mag = nrm * exp(dt_re * d), ph = dt_im * d;
+    const double z = lane < n ? Z[lane] : 0.0;
+    const double tr = mag * cos(ph) * z, ti = mag * sin(ph) * z;
+    for (int j = 0; j < n; ++j) {
+      const double u = zrow[j];
+      cr = fma(u, lane_value(tr, j), cr);
+      ci = fma(u, lane_value(ti, j), ci);
     }
   } else {
-    if (lane < n) {
-      st->coef_re[lane] = Z[lane][0];
-      st->coef_im[lane] = 0.0;
+    int k = 0;
+    energy = lane_value(d, 0);
+    for (int j = 1; j < n; ++j) {
+      const double dj = lane_value(d, j);
+      if (dj < energy) { energy = dj; k = j; }
     }
-    if (lane == 0) st->energy = d[0];
+    cr = zrow[k];
   }
-  if (lane == 0 && noconv) st->noconv = 1;
+  return conv;
 }
+
+// The end of a solve, one workgroup per problem: the last alpha (krylov.py:54-56; from
+// the rb partial sums, or for short vectors, rb = 0, straight from w and v_j), the
+// coefficients and the exported scalars.
+__global__ __launch_bounds__(SHORT_T) void k_lz_tail(int n, const double2* __restrict__ w,
+                                                     const double2* __restrict__ vj, int j,
+                                                     const double* __restrict__ part, int rb,
+                                                     LzState* st, int mode, double dt_re,
+                                                     double dt_im, int32_t* info,
+                                                     double* alpha_beta, double* energy) {
+  __shared__ __align__(16) double red[16][4], Z[LZ_MAX * (LZ_MAX + 1)];
+  const int b = blockIdx.x, t = threadIdx.x;
+  st += b;
+  const int numiter = j + 1;
+  const bool go = !st->stopped;
+  double a = 0;
+  if (go) {
+    if (rb) {
+      for (int i = t; i < rb; i += blockDim.x) a += part[(int64_t)b * rb + i];
+    } else {
+      const int64_t o = (int64_t)b * n;
+#pragma unroll 4
+      for (int i = t; i < n; i += blockDim.x) {
+        const double2 x = w[o + i], v = vj[o + i];
+        a += x.x * v.x + x.y * v.y;
+      }
+    }
+    a = wg_sum(a, red);
+  }
+  if (t >= 64) return;
+  if (go && t == 0) {
+    st->alpha[j] = a;
+    if (!isfinite(a)) st->nonfinite = 1;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  const int nv = st->nvalid;
+  double en = 0.0;
+  bool conv = true;
+  if (nv > 0 && !st->nonfinite) {
+    double cr, ci;
+    conv = tridiag_coefs(nv, st->alpha, st->beta, Z, LZ_MAX + 1, mode, st->nrm0, dt_re, dt_im, cr,
+                         ci, en);
+    if (t < nv) {
+      st->coef_re[t] = cr;
+      st->coef_im[t] = ci;
+    }
+  }
+  if (t == 0) {
+    st->energy = en;
+    st->noconv = !conv;
+    if (info) {
+      info[4 * b] = nv;
+      info[4 * b + 1] = st->breakdown;
+      info[4 * b + 2] = st->nonfinite | (conv ? 0 : 2);
+      info[4 * b + 3] = st->zero_start;
+    }
+    if (energy) energy[b] = en;
+  }
+  if (alpha_beta && t < numiter) {
+    double* ab = alpha_beta + (int64_t)2 * numiter * b;
+    ab[t] = st->alpha[t];
+    ab[numiter + t] = st->beta[t];
+  }
+}
+
+}  // namespace ptn
+
+#include "krylov_small.h"
+
+namespace ptn {
 
 // out = sum_{j < nvalid} c_j V_j  (krylov.py:118, :136)
 // V_j of problem b at V + j * js + b * Vs
@@ -360,29 +624,6 @@ __global__ __launch_bounds__(256) void k_combine(int64_t n, const double2* __res
       si += cr[j] * v.y + ci[j] * v.x;
     }
     out[i] = make_double2(sr, si);
-  }
-}
-
-__global__ void k_export(const LzState* __restrict__ st, int32_t* info, double* alpha_beta,
-                         double* energy, int numiter) {
-  const int b = blockIdx.x;
-  st += b;
-  if (info) info += 4 * b;
-  if (energy) energy += b;
-  if (alpha_beta) alpha_beta += 2 * numiter * b;
-  const int t = threadIdx.x;
-  if (t == 0) {
-    if (info) {
-      info[0] = st->nvalid;
-      info[1] = st->breakdown;
-      info[2] = st->nonfinite | (st->noconv << 1);
-      info[3] = st->zero_start;
-    }
-    if (energy) *energy = st->energy;
-  }
-  if (alpha_beta && t < numiter) {
-    alpha_beta[t] = st->alpha[t];
-    alpha_beta[numiter + t] = st->beta[t];
   }
 }
 
@@ -608,6 +849,14 @@ int krylov_run(const ptn_local_op* op, int mode, const void* v, double dt_re, do
   return PTN_OK;
 }
 
+// f with the elements per thread of the short-vector kernels as a constant
+template <typename F> static void short_r(int64_t n, F f) {
+  if (n <= SHORT_T) f(std::integral_constant<int, 1>());
+  else if (n <= 2 * SHORT_T) f(std::integral_constant<int, 2>());
+  else if (n <= 4 * SHORT_T) f(std::integral_constant<int, 4>());
+  else f(std::integral_constant<int, 8>());
+}
+
 static int krylov_enqueue(const ptn_local_op* op, int mode, const void* v, double dt_re,
                           double dt_im, int numiter, void* out, double* energy, int32_t* info,
                           double* alpha_beta, void* ws, size_t ws_bytes, hipStream_t s,
@@ -640,6 +889,35 @@ static int krylov_enqueue(const ptn_local_op* op, int mode, const void* v, doubl
                          ? 128.0 * FLT_EPSILON
                          : (bprec == PTN_BF16X3 ? 1.0 / 4096 : 0.0);
 
+  // (in a batch, a problem's output must not lie over what another workgroup still reads)
+  auto apart = [&](const void* q, int64_t elems) {
+    const char *o = (const char*)out, *x = (const char*)q;
+    return !q || x + batch * elems * 16 <= o || o + batch * n * 16 <= x;
+  };
+  LzSmall sm;
+  if (small_plan(op, numiter, batch, &sm) &&
+      (batch == 1 || ((v == out || apart(v, n)) && apart(op->l, op->Dl * op->Ml * op->Dl) &&
+                      apart(op->r, op->Dr * op->Mr * op->Dr) &&
+                      apart(op->w, op->Ml * op->d * op->d * op->Mr)))) {
+    sm.mode = mode;
+    sm.thresh = thresh;
+    sm.dt_re = dt_re;
+    sm.dt_im = dt_im;
+    sm.l = (const double2*)op->l;
+    sm.w = (const double2*)op->w;
+    sm.r = (const double2*)op->r;
+    sm.v = (const double2*)v;
+    sm.V = V;
+    sm.out = (double2*)out;
+    sm.js = js;
+    sm.info = info;
+    sm.alpha_beta = alpha_beta;
+    sm.energy = energy;
+    small_solve(sm, batch, s);
+    PTN_LAUNCH_CHECK();
+    return PTN_OK;
+  }
+
   // environment blocks in the matvec's operand precision, converted once per solve
   const void* L = op->l;
   const void* R = op->r;
@@ -671,30 +949,37 @@ static int krylov_enqueue(const ptn_local_op* op, int mode, const void* v, doubl
   // remaining matvecs of that problem do no work
   static_assert(sizeof(LzState) % sizeof(int) == 0, "LzState stride in ints");
   SkipGuard skip(&st->stopped, (int64_t)(sizeof(LzState) / sizeof(int)));
-  k_state_init<<<B, 256, 0, s>>>(st, numiter);
-  k_sumsq_partial<<<dim3(rb, B), 256, 0, s>>>(n, (const double2*)v, n, pa, rb);
-  k_start<<<dim3((unsigned)gblocks, B), 256, 0, s>>>(n, (const double2*)v, n, V, n, pa, rb, st);
+  const double2* x0 = (const double2*)v;
+  const bool shrt = n <= SHORT_MAX;
+  const int ni = (int)std::min<int64_t>(n, SHORT_MAX);
+  const dim3 nt((unsigned)std::min<int64_t>(SHORT_T, (n + 63) / 64 * 64));
+  if (shrt) {
+    short_r(n, [&](auto r) { k_lz_start<r.value><<<B, nt, 0, s>>>(ni, x0, V, st, numiter); });
+  } else {
+    k_sumsq_partial<<<dim3(rb, B), 256, 0, s>>>(n, x0, n, pa, rb, st, numiter);
+    k_start<<<dim3((unsigned)gblocks, B), 256, 0, s>>>(n, x0, n, V, n, pa, rb, st);
+  }
   PTN_LAUNCH_CHECK();
-  for (int j = 0; j < numiter - 1; ++j) {
+  for (int j = 0; j < numiter; ++j) {
     double2* vj = V + (int64_t)j * js;
+    const double2* vp = j > 0 ? vj - js : vj;
     if ((st_ = matvec(vj, w))) return st_;
-    k_dot_partial<<<dim3(rb, B), 256, 0, s>>>(n, w, n, vj, n, pa, rb);
-    k_alpha_update<<<dim3(rb, B), 256, 0, s>>>(n, w, n, vj, j > 0 ? vj - js : vj, n, j, pa, pb,
-                                                rb, st);
-    k_beta_next<<<dim3((unsigned)gblocks, B), 256, 0, s>>>(n, w, n, vj + js, n, j, pb, rb,
-                                                            thresh, rel, st);
+    if (!shrt) k_dot_partial<<<dim3(rb, B), 256, 0, s>>>(n, w, n, vj, n, pa, rb);
+    if (j == numiter - 1) {
+      k_lz_tail<<<B, shrt ? nt : dim3(512), 0, s>>>(ni, w, vj, j, pa, shrt ? 0 : rb, st, mode, dt_re,
+                                                    dt_im, info, alpha_beta, energy);
+    } else if (shrt) {
+      short_r(n, [&](auto r) {
+        k_lz_step<r.value><<<B, nt, 0, s>>>(ni, w, vj, vp, vj + js, j, thresh, rel, st);
+      });
+    } else {
+      k_alpha_update<<<dim3(rb, B), 256, 0, s>>>(n, w, n, vj, vp, n, j, pa, pb, rb, st);
+      k_beta_next<<<dim3((unsigned)gblocks, B), 256, 0, s>>>(n, w, n, vj + js, n, j, pb, rb,
+                                                              thresh, rel, st);
+    }
     PTN_LAUNCH_CHECK();
   }
-  {
-    const int j = numiter - 1;
-    double2* vj = V + (int64_t)j * js;
-    if ((st_ = matvec(vj, w))) return st_;
-    k_dot_partial<<<dim3(rb, B), 256, 0, s>>>(n, w, n, vj, n, pa, rb);
-    k_alpha_last<<<B, 256, 0, s>>>(j, pa, rb, st);
-  }
-  k_tridiag<<<B, 64, 0, s>>>(st, mode, dt_re, dt_im);
   k_combine<<<dim3((unsigned)gblocks, B), 256, 0, s>>>(n, V, js, n, st, (double2*)out, n);
-  k_export<<<B, 64, 0, s>>>(st, info, alpha_beta, energy, numiter);
   PTN_LAUNCH_CHECK();
   return PTN_OK;
 }

@@ -23,31 +23,9 @@
 // with the same three steps and T in place of T^H.
 #include <float.h>
 #include "qr.h"
+#include "wave.h"
 
 namespace ptn {
-
-// sum over the wave, in every lane: rotations inside the rows of 16 lanes (DPP), then the
-// four row sums read as scalars (an exchange through LDS per step takes several
-// times as long)
-template <int CTRL> __device__ __forceinline__ double dpp_rot(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)b, lane);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-__device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_rot<0x128>(v);   // row rotate right by 8, 4, 2, 1
-  v += dpp_rot<0x124>(v);
-  v += dpp_rot<0x122>(v);
-  v += dpp_rot<0x121>(v);
-  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
 
 // Eight sums over the wave at once: two values fold into one register per step (the
 // halves of the wave, then the rows of 16, then of 8 lanes keep one each and add the
@@ -142,16 +120,11 @@ __device__ __forceinline__ Refl make_refl(double2 alpha, double xnorm) {
   h.rd = make_double2(beta, 0.0);
   return h;
 }
-// 1 / x and 1 / sqrt(x) to full precision from the hardware's estimates (normal x)
+// 1 / x to full precision from the hardware's estimate (normal x)
 __device__ __forceinline__ double rcp_full(double x) {
   double y = __builtin_amdgcn_rcp(x);
   y = fma(y, fma(-x, y, 1.0), y);
   return fma(y, fma(-x, y, 1.0), y);
-}
-__device__ __forceinline__ double rsq_full(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 // the same reflector from the sum of squares s2 = |x|^2, with the short chain of
 // operations that the panel kernels wait for; norms far outside the usual range

@@ -40,6 +40,7 @@
 #include <float.h>
 #include "common.h"
 #include "qr.h"
+#include "wave.h"
 
 namespace ptn {
 
@@ -187,16 +188,6 @@ __global__ __launch_bounds__(256) void k_jac_gram(int64_t p, int nblk, int r,
       out[i * JP + j] = C2{re, im};
     }
   }
-}
-
-// 1 / sqrt(x) to full double precision for normal positive x: the hardware's estimate
-// (relative error about 2^-24) and one third-order step. The rotations' chain of
-// dependent operations sets the speed of the solves; the library's rsqrt, sqrt and
-// division take several times as many.
-__device__ __forceinline__ double rsq_full(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 // rotation parameters of the index pair (i, j) of a Hermitian Gram matrix with
