@@ -223,24 +223,9 @@ __global__ __launch_bounds__(256) void k_beta_next(int64_t n, const double2* __r
 constexpr int SHORT_T = 1024;     // largest workgroup
 constexpr int64_t SHORT_MAX = 8 * SHORT_T;
 
-// barrier that orders LDS accesses only: stores to memory that only the threads which
-// made them read back stay in flight across it
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // sum over the workgroup (up to 16 waves) in a fixed order, in every thread: the sums of
 // each wave's rows of 16 lanes through LDS, then lane l of a row adds those of wave l. red
 // is not written again until the caller's next barrier after it.
-__device__ __forceinline__ double row_sum(double v) {
-  v += dpp_rot<0x128>(v);   // row rotate right by 8, 4, 2, 1
-  v += dpp_rot<0x124>(v);
-  v += dpp_rot<0x122>(v);
-  v += dpp_rot<0x121>(v);
-  return v;
-}
 __device__ __forceinline__ double wg_sum(double v, double (&red)[16][4]) {
   v = row_sum(v);
   const int t = threadIdx.x, w = t & 15;

@@ -38,6 +38,7 @@
 //   cs = 1 / sqrt(1 + t^2), s = cs t e^{i phi},
 //   x' = cs x - conj(s) y,   y' = s x + cs y.
 #include <float.h>
+#include <type_traits>
 #include "common.h"
 #include "qr.h"
 #include "wave.h"
@@ -76,7 +77,12 @@ __global__ void k_eye(int64_t q, double2* __restrict__ V) {
 __device__ __forceinline__ void round_pair(int ne, int r, int k, int& p, int& q) {
   const int cyc = ne - 1;
   if (k == 0) { p = r; q = cyc; }
-  else { p = (r + k) % cyc; q = (r - k + cyc) % cyc; }
+  else {   // r + k and r - k modulo cyc (0 <= r, k < cyc)
+    p = r + k;
+    if (p >= cyc) p -= cyc;
+    q = r - k;
+    if (q < 0) q += cyc;
+  }
   if (p > q) { int t = p; p = q; q = t; }
 }
 
@@ -792,11 +798,12 @@ __global__ void k_set_ints(int* p, int n, int v) {
   if ((int)threadIdx.x < n) p[threadIdx.x] = v;
 }
 
+// sweeps < 0: they and the unconverged flag are on the device
 __global__ void k_svd_info(int32_t* info, int sweeps, int notconv, const int* counters,
                            int sweeps32) {
   if (threadIdx.x == 0) {
-    info[0] = sweeps;
-    info[1] = notconv;
+    info[0] = sweeps < 0 ? counters[2] : sweeps;
+    info[1] = sweeps < 0 ? counters[3] : notconv;
     info[2] = counters[1];
     info[3] = sweeps32;
   }
@@ -860,10 +867,13 @@ __global__ void k_ns_update(int64_t n, const double2* __restrict__ Q, const doub
 
 static inline size_t al(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// pinned word for the per-sweep rotation count, allocated once per process
+// pinned words for the rotation count, flags and the singular values of small splits,
+// allocated once per thread
+constexpr int PINNED_INTS = 4;
 static int* pinned_counter() {
   static thread_local int* p = nullptr;
-  if (!p && hipHostMalloc((void**)&p, sizeof(int), hipHostMallocDefault) != hipSuccess) p = nullptr;
+  if (!p && hipHostMalloc((void**)&p, PINNED_INTS * sizeof(int), hipHostMallocDefault) != hipSuccess)
+    p = nullptr;
   return p;
 }
 
@@ -929,6 +939,163 @@ static inline unsigned gs_blocks(int64_t total) {
   return (unsigned)(b < 1 ? 1 : (b > 1024 ? 1024 : b));
 }
 
+// Small matrices: the whole Jacobi phase of a problem in one launch and one workgroup,
+// without Gram matrices. The columns (and V) stay in LDS; a group of 16 lanes takes a column
+// pair per step of the round-robin over single columns (q - 1 steps a sweep), R = q / 16 rows
+// per lane: |x|^2, |y|^2 and x^H y straight from the columns, summed across the group in
+// registers (DPP), then the rotation. The sweeps stop per problem on the device (same
+// tolerances and stopping rule as the blocked form), and the column norms, their order and
+// the singular values follow in the same launch. Bound by the chain load - sums - rotation -
+// store of a step for small q (0.66 us at q = 32), by LDS bandwidth from q = 64 on (the columns
+// are read and written once a step). Blocked sweeps are three launches per round and a wait of
+// the host per sweep whatever the size. A whole split (QRs and products included), blocked and
+// here: q = 8 302 -> 170 us, 32 455 -> 295, 48 848 -> 540, 64 899 -> 713, 80 1316 -> 1087, 96
+// 1333 -> 1368; a thin SVD, with V: q = 32 483 -> 315, 48 881 -> 591, 64 922 -> 835, 400 of
+// 64 at once 2293 -> 1779.
+template <int R, bool WANT_V>
+__global__ __launch_bounds__(128 * R) void k_jac_small(
+    int q, int qp, double2* __restrict__ X, double2* __restrict__ V, double tol, double big,
+    int max_sweeps, double* __restrict__ nrm, int64_t* __restrict__ perm,
+    double* __restrict__ s_out, int64_t ss, const double* __restrict__ scl,
+    const double* __restrict__ scl2, int* __restrict__ counters) {
+  constexpr int Q = 16 * R;               // rows and columns in LDS, zeros beyond q
+  __shared__ __align__(16) double2 sx[Q * Q];
+  __shared__ __align__(16) double2 sv[WANT_V ? Q * Q : 1];
+  __shared__ double key[Q];
+  __shared__ int more[2];
+  const int t = threadIdx.x, nt = blockDim.x, l16 = t & 15, grp = t >> 4;
+  X += (int64_t)blockIdx.x * q * qp;
+  if (WANT_V) V += (int64_t)blockIdx.x * qp * qp;
+  nrm += (int64_t)blockIdx.x * qp;
+  perm += (int64_t)blockIdx.x * qp;
+  s_out += (int64_t)blockIdx.x * ss;
+  const double scale = scl2 ? *scl * *scl2 : scl[blockIdx.x];
+  for (int i = t; i < Q * Q; i += nt) {
+    const int c = i / Q, r = i % Q;
+    sx[i] = c < q && r < q ? X[(int64_t)c * q + r] : make_double2(0.0, 0.0);
+    if (WANT_V) sv[i] = make_double2(c == r ? 1.0 : 0.0, 0.0);
+  }
+  if (t < 2) more[t] = 0;
+  __syncthreads();
+  const int ne = (q + 1) & ~1;            // a column of zeros makes the number even
+  int sweeps = 0;
+  bool done = q < 2;
+  while (!done && sweeps < max_sweeps) {
+    bool any = false;
+    for (int r = 0; r < ne - 1; ++r) {
+      for (int k = grp; k < ne / 2; k += nt >> 4) {
+        int ci, cj;
+        round_pair(ne, r, k, ci, cj);
+        double2* px = sx + ci * Q + l16;
+        double2* py = sx + cj * Q + l16;
+        double2 x[R], y[R];
+        double a = 0.0, b = 0.0, cr = 0.0, cim = 0.0;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          x[u] = px[16 * u];
+          y[u] = py[16 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+          a = fma(x[u].x, x[u].x, fma(x[u].y, x[u].y, a));
+          b = fma(y[u].x, y[u].x, fma(y[u].y, y[u].y, b));
+          cr = fma(x[u].x, y[u].x, fma(x[u].y, y[u].y, cr));
+          cim = fma(x[u].x, y[u].y, fma(-x[u].y, y[u].x, cim));
+        }
+        a = row_sum(a);
+        b = row_sum(b);
+        cr = row_sum(cr);
+        cim = row_sum(cim);
+        double cs, sr, si;
+        bool rot, rbig;
+        jac_rotation(a, b, make_double2(cr, cim), tol, big, cs, sr, si, rot, rbig);
+        any |= rbig;
+        if (rot) {
+          auto turn = [&](double2* gx, double2* gy, double2 xv, double2 yv) {
+            // x' = cs x - conj(s) y, y' = s x + cs y
+            *gx = make_double2(fma(cs, xv.x, -fma(sr, yv.x, si * yv.y)),
+                               fma(cs, xv.y, -fma(sr, yv.y, -(si * yv.x))));
+            *gy = make_double2(fma(cs, yv.x, fma(sr, xv.x, -(si * xv.y))),
+                               fma(cs, yv.y, fma(sr, xv.y, si * xv.x)));
+          };
+#pragma unroll
+          for (int u = 0; u < R; ++u) turn(px + 16 * u, py + 16 * u, x[u], y[u]);
+          if (WANT_V) {
+            double2* vx = sv + ci * Q + l16;
+            double2* vy = sv + cj * Q + l16;
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+              turn(vx + 16 * u, vy + 16 * u, vx[16 * u], vy[16 * u]);
+          }
+        }
+      }
+      lds_barrier();
+    }
+    if (any) more[sweeps & 1] = 1;
+    __syncthreads();
+    done = !more[sweeps & 1];
+    if (t == 0) more[~sweeps & 1] = 0;
+    ++sweeps;
+  }
+  __syncthreads();
+  // column norms, X and V back, the order of the norms (as k_colnorms and k_rank)
+  for (int c = grp; c < q; c += nt >> 4) {
+    double n2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const double2 x = sx[c * Q + 16 * u + l16];
+      n2 = fma(x.x, x.x, fma(x.y, x.y, n2));
+    }
+    n2 = row_sum(n2);
+    if (l16 == 0) key[c] = sqrt(n2);
+  }
+  for (int i = t; i < q * q; i += nt) {
+    const int c = i / q, r = i % q;
+    X[i] = sx[c * Q + r];
+    if (WANT_V) V[(int64_t)c * qp + r] = sv[c * Q + r];
+  }
+  __syncthreads();
+  for (int j = t; j < q; j += nt) {
+    const double sj = key[j], kj = isfinite(sj) ? sj : -1.0;
+    if (!isfinite(sj)) atomicOr(counters + 1, 1);
+    int rank = 0;
+    for (int i = 0; i < q; ++i) {
+      const double ki = isfinite(key[i]) ? key[i] : -1.0;
+      rank += ki > kj || (ki == kj && i < j);
+    }
+    nrm[j] = sj;
+    perm[rank] = j;
+    s_out[rank] = sj / scale;
+  }
+  if (t == 0) {
+    atomicMax(counters + 2, sweeps);
+    if (!done) atomicOr(counters + 3, 1);
+  }
+}
+
+constexpr int64_t SMALL_Q = 80;      // largest q of k_jac_small without V
+constexpr int64_t SMALL_QV = 64;     // the same with V
+
+template <bool WANT_V>
+static void jac_small_launch(const SvdLayout& L, char* base, double2* X, double2* V, double tol,
+                             double big, int max_sweeps, double* s, int64_t ss, const double* scl,
+                             const double* scl2, int* counters, hipStream_t st) {
+  auto go = [&](auto r) {
+    constexpr int R = decltype(r)::value;
+    tlaunch("k_jac_small", 0.0, 0.0, k_jac_small<R, WANT_V>, dim3((unsigned)L.batch),
+            dim3(128 * R), st, (int)L.q, (int)L.qp, X, V, tol, big, max_sweeps,
+            (double*)(base + L.nrm), (int64_t*)(base + L.perm), s, ss, scl, scl2, counters);
+  };
+  const int64_t r = (L.q + 15) / 16;
+  if (r == 1) go(std::integral_constant<int, 1>());
+  else if (r == 2) go(std::integral_constant<int, 2>());
+  else if (r == 3) go(std::integral_constant<int, 3>());
+  else if (r == 4) go(std::integral_constant<int, 4>());
+  if constexpr (!WANT_V) {
+    if (r == 5) go(std::integral_constant<int, 5>());
+  }
+}
+
 // One Jacobi sweep (every round of the block tournament) over the columns of X, the
 // rotations accumulated in V if want_v; counters[0] receives the number of
 // pairs that needed a rotation above `big`. The algorithmic work per launch for the live timing:
@@ -983,7 +1150,7 @@ static void jacobi_sweep(const SvdLayout& L, char* base, typename JacT<T>::c2* X
 // Thin SVD of `batch` m x n matrices of identical shape (problem b at a + b sa,
 // u + b su, s + b ss, vh + b svh). The Jacobi sweeps run on all problems at
 // once and stop together, after the first sweep in which no problem needed a
-// rotation above `big` (relative). info (if given) receives the number of
+// rotation above `big` (relative); those of k_jac_small stop each by itself. info (if given) receives the number of
 // sweeps, whether the sweep limit was hit, and whether any singular value was
 // not finite.
 // With `precond32` (and at least PRE32_MIN_Q columns) the Jacobi phase starts
@@ -1001,8 +1168,12 @@ static void jacobi_sweep(const SvdLayout& L, char* base, typename JacT<T>::c2* X
 // of the workspace after FP32 preconditioning).
 struct JacobiResult {
   int sweeps = 0, sweeps32 = 0, converged = 0;
+  bool ranked = false;   // k_jac_small: norms, order and singular values are done, and the
+                         // sweeps (maximum over the batch) and the unconverged flag are in
+                         // counters[2] and [3]
 };
 static int jacobi_core(const SvdLayout& L, char* base, double2*& X, double2* V, bool want_v,
+                       double* s, int64_t ss, const double* scl, const double* scl2,
                        hipStream_t st, JacobiResult& res) {
   const unsigned NB = (unsigned)L.batch;
   double* nrm = (double*)(base + L.nrm);
@@ -1012,7 +1183,21 @@ static int jacobi_core(const SvdLayout& L, char* base, double2*& X, double2* V, 
   int stt;
   int* host_rot = pinned_counter();
   if (!host_rot) return PTN_ERR_HIP;
-  k_set_ints<<<1, 64, 0, st>>>(counters, 2, 0);
+  k_set_ints<<<1, 64, 0, st>>>(counters, 4, 0);
+  const double tol = DBL_EPSILON * sqrt((double)L.q);
+  // the iteration stops after a sweep in which no pair needed a rotation above
+  // this relative size: convergence is quadratic, so the couplings left after
+  // such a sweep are of order big^2 (n big^2 at most), and a further sweep
+  // would only rotate by rounding-level angles
+  const double big = 1e-8;
+  const int max_sweeps = 60;
+  if (L.q <= (want_v ? SMALL_QV : SMALL_Q)) {
+    if (want_v) jac_small_launch<true>(L, base, X, V, tol, big, max_sweeps, s, ss, scl, scl2, counters, st);
+    else jac_small_launch<false>(L, base, X, V, tol, big, max_sweeps, s, ss, scl, scl2, counters, st);
+    PTN_LAUNCH_CHECK();
+    res.ranked = true;
+    return PTN_OK;
+  }
   if (L.pre32) {
     float2* X32 = (float2*)(base + L.x32);
     float2* V32 = (float2*)(base + L.v32);
@@ -1060,13 +1245,6 @@ static int jacobi_core(const SvdLayout& L, char* base, double2*& X, double2* V, 
     k_eye<<<dim3(gs_blocks(L.qp * L.qp), NB), 256, 0, st>>>(L.qp, V);
     PTN_LAUNCH_CHECK();
   }
-  const double tol = DBL_EPSILON * sqrt((double)L.q);
-  // the iteration stops after a sweep in which no pair needed a rotation above
-  // this relative size: convergence is quadratic, so the couplings left after
-  // such a sweep are of order big^2 (n big^2 at most), and a further sweep
-  // would only rotate by rounding-level angles
-  const double big = 1e-8;
-  const int max_sweeps = 60;
   res.converged = (L.q < 2);
   while (!res.converged && res.sweeps < max_sweeps) {
     jacobi_sweep<double>(L, base, X, V, want_v, tol, big, counters, st);
@@ -1082,7 +1260,7 @@ static int jacobi_core(const SvdLayout& L, char* base, double2*& X, double2* V, 
 // Thin SVD of `batch` m x n matrices of identical shape (problem b at a + b sa,
 // u + b su, s + b ss, vh + b svh). The Jacobi sweeps run on all problems at
 // once and stop together, after the first sweep in which no problem needed a
-// rotation above `big` (relative). info (if given) receives the number of
+// rotation above `big` (relative); those of k_jac_small stop each by itself. info (if given) receives the number of
 // sweeps, whether the sweep limit was hit, and whether any singular value was
 // not finite.
 // With `precond32` (and at least PRE32_MIN_Q columns) the Jacobi phase starts
@@ -1143,22 +1321,24 @@ int svd_run(int64_t m, int64_t n, const void* a, int64_t lda, void* u, int64_t l
                                                         f2.bs.W, f2.bs.k);
   PTN_LAUNCH_CHECK();
   JacobiResult jr;
-  if ((stt = jacobi_core(L, base, X, V, true, st, jr))) return stt;
+  if ((stt = jacobi_core(L, base, X, V, true, s, ss, f.scl, nullptr, st, jr))) return stt;
   // 3. B = Q1 R2^H Q2^H = (Q1 [U_X; 0]) diag(sigma) (Q2 V)^H with U_X = X / sigma
-  k_colnorms<<<dim3((unsigned)L.q, NB), 256, 0, st>>>(L.q, X, nrm, sx, L.qp);
+  if (!jr.ranked) k_colnorms<<<dim3((unsigned)L.q, NB), 256, 0, st>>>(L.q, X, nrm, sx, L.qp);
   k_embed_u<<<dim3(gs_blocks(L.p * L.q), NB), 256, 0, st>>>(L.p, L.q, X, nrm, UB, sx, L.qp);
   k_copy_v<<<dim3(gs_blocks(L.q * L.q), NB), 256, 0, st>>>(L.q, L.qp, V, VB);
   PTN_LAUNCH_CHECK();
   if ((stt = qr_apply_q(f, UB, L.p, L.q, false, st, L.p * L.q))) return stt;
   if ((stt = qr_apply_q(f2, VB, L.q, L.q, false, st, L.q * L.q))) return stt;
-  k_rank<<<dim3((unsigned)((L.q + 255) / 256), NB), 256, 0, st>>>(L.q, nrm, perm, s, counters + 1,
-                                                                   L.qp, ss, f.scl);
+  if (!jr.ranked)
+    k_rank<<<dim3((unsigned)((L.q + 255) / 256), NB), 256, 0, st>>>(L.q, nrm, perm, s,
+                                                                     counters + 1, L.qp, ss, f.scl);
   const int64_t tot = (m * k > k * n) ? m * k : k * n;
   k_svd_out<<<dim3((unsigned)((tot + 255) / 256), NB), 256, 0, st>>>(
       m, n, k, adjoint, L.p, L.q, UB, VB, perm, (double2*)u, ldu, (double2*)vh, ldvh, L.qp, su,
       svh);
   if (info)
-    k_svd_info<<<1, 64, 0, st>>>(info, jr.sweeps, jr.converged ? 0 : 1, counters, jr.sweeps32);
+    k_svd_info<<<1, 64, 0, st>>>(info, jr.ranked ? -1 : jr.sweeps, jr.converged ? 0 : 1, counters,
+                                 jr.sweeps32);
   PTN_LAUNCH_CHECK();
   return PTN_OK;
 }
@@ -1338,33 +1518,35 @@ int svd_split_run(int64_t m, int64_t n, const void* theta, int64_t lda, int dist
   k_rh<<<dim3(gs_blocks(L.q * L.qp), 1), 256, 0, st>>>(L.q, L.q, L.q, L.qp, 1, f2.W, f2.rdiag, X,
                                                        f2.bs.W, f2.bs.k);
   PTN_LAUNCH_CHECK();
-  JacobiResult jr;
-  if ((stt = jacobi_core(L, base, X, V, false, st, jr))) return stt;
   // the singular values carry the power-of-two input scales of the QR(s)
-  double* scl = f.scl;
-  if (S.wide) {
-    scl = (double*)(wsb + S.inner - 16);
-    k_mul_scale<<<1, 64, 0, st>>>(f.scl, f0.scl, scl);
+  JacobiResult jr;
+  const double* scl0 = S.wide ? f0.scl : nullptr;
+  if ((stt = jacobi_core(L, base, X, V, false, sdev, L.q, f.scl, scl0, st, jr))) return stt;
+  if (!jr.ranked) {
+    double* scl = f.scl;
+    if (S.wide) {
+      scl = (double*)(wsb + S.inner - 16);
+      k_mul_scale<<<1, 64, 0, st>>>(f.scl, f0.scl, scl);
+    }
+    k_colnorms<<<dim3((unsigned)L.q, 1), 256, 0, st>>>(L.q, X, nrm, sx, L.qp);
+    k_rank<<<dim3((unsigned)((L.q + 255) / 256), 1), 256, 0, st>>>(
+        L.q, nrm, perm, sdev, counters + 1, L.qp, L.q, scl);
   }
-  k_colnorms<<<dim3((unsigned)L.q, 1), 256, 0, st>>>(L.q, X, nrm, sx, L.qp);
-  k_rank<<<dim3((unsigned)((L.q + 255) / 256), 1), 256, 0, st>>>(L.q, nrm, perm, sdev,
-                                                                  counters + 1, L.qp, L.q, scl);
   PTN_LAUNCH_CHECK();
-  // the singular values and the non-finite flag on the host (the kept count
-  // sizes the outputs)
+  // the singular values and the flags on the host (the kept count sizes the outputs)
   int* host_rot = pinned_counter();
   if (!host_rot) return PTN_ERR_HIP;
+  PTN_HIP_CHECK(hipMemcpyAsync(host_rot, counters, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
   PTN_HIP_CHECK(hipMemcpyAsync(s_host, sdev, (size_t)L.q * sizeof(double), hipMemcpyDeviceToHost,
                                st));
-  PTN_HIP_CHECK(hipMemcpyAsync(host_rot, counters + 1, sizeof(int), hipMemcpyDeviceToHost, st));
   PTN_HIP_CHECK(hipStreamSynchronize(st));
   if (info_host) {
-    info_host[0] = jr.sweeps;
-    info_host[1] = jr.converged ? 0 : 1;
-    info_host[2] = *host_rot;
+    info_host[0] = jr.ranked ? host_rot[2] : jr.sweeps;
+    info_host[1] = jr.ranked ? host_rot[3] : !jr.converged;
+    info_host[2] = host_rot[1];
     info_host[3] = jr.sweeps32;
   }
-  if (*host_rot) { *k_out = 0; return PTN_ERR_NONFINITE; }
+  if (host_rot[1]) { *k_out = 0; return PTN_ERR_NONFINITE; }
   const int64_t k = kept_count(s_host, L.q, tol, max_bond);
   *k_out = k;
   if (k == 0) return PTN_OK;

@@ -38,4 +38,20 @@ __device__ __forceinline__ double rsq_full(double x) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+// sum over each row of 16 lanes, in every lane of it
+__device__ __forceinline__ double row_sum(double v) {
+  v += dpp_rot<0x128>(v);   // row rotate right by 8, 4, 2, 1
+  v += dpp_rot<0x124>(v);
+  v += dpp_rot<0x122>(v);
+  v += dpp_rot<0x121>(v);
+  return v;
+}
+// barrier that orders LDS accesses only: stores to memory that only the threads which
+// made them read back stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 }  // namespace ptn
