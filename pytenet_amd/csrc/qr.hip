@@ -210,6 +210,40 @@ __global__ void k_to_colmajor(int64_t m, int64_t n, const double2* __restrict__ 
   w[j * m + i] = make_double2(x.x * sc, x.y * sc);
 }
 
+// The three launches above in one for a matrix of at most QR_IN_MAX entries: one workgroup
+// per matrix holds it in registers between the maximum and the copy.
+constexpr int64_t QR_IN_MAX = 8192;
+__global__ __launch_bounds__(1024) void k_qr_in(int m, int n, const double2* __restrict__ a,
+                                                int64_t lda, double2* __restrict__ w, int64_t sa,
+                                                int64_t sw, double* __restrict__ scl) {
+  constexpr int E = QR_IN_MAX / 1024;
+  __shared__ double wmax[16];
+  a += blockIdx.x * sa;
+  w += blockIdx.x * sw;
+  const int t = threadIdx.x, nw = blockDim.x >> 6;
+  double2 x[E];
+  double v = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int at = t + e * (int)blockDim.x;
+    x[e] = at < m * n ? a[(int64_t)(at / n) * lda + at % n] : make_double2(0.0, 0.0);
+    v = fmax(v, fmax(fabs(x[e].x), fabs(x[e].y)));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+  if ((t & 63) == 0) wmax[t >> 6] = v;
+  __syncthreads();
+  v = 0.0;
+  for (int k = 0; k < nw; ++k) v = fmax(v, wmax[k]);
+  const double sc = qr_scale_of((unsigned long long)__double_as_longlong(v));
+  if (t == 0) scl[blockIdx.x] = sc;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int at = t + e * (int)blockDim.x;
+    if (at < m * n) w[(int64_t)(at % n) * m + at / n] = make_double2(x[e].x * sc, x[e].y * sc);
+  }
+}
+
 // reflector j, applied to column c = j + blockIdx.x (< pe) of the panel.
 // Workgroup 0 stores v_j (with the unit and the zeros above), tau_j and R[j, j];
 // column j of W itself is left as it is (rows > j are not read again).
@@ -534,6 +568,155 @@ __global__ __launch_bounds__(256) void k_qr_col2r(int64_t m, int64_t j, double2*
   }
 }
 
+// G[a][b] = v_a^H v_b (a <= b in steps of 16) of the panel's reflectors over the rows
+// first .. end - 1: FP64 MFMA on 16 x 16 tiles, the operands loaded as in the
+// cross Gram kernel of the Jacobi iteration (a lane holds rows 2 kk, 2 kk + 1 of every 8
+// of column l16); columns >= nbp count as zero. Thread t (of 256) ends with entry (t / 16,
+// t % 16) of the tiles (0, 0), (0, 16) and (16, 16). No __restrict__ here: k_qr_panel reads
+// what its own waves have just stored.
+typedef double2 VtvRed[4][3][4][64];
+__device__ __forceinline__ void vtv_block(int64_t m, int64_t j0, int nbp, int64_t first,
+                                          int64_t end, const double2* Vf,
+                                          VtvRed& red, double2 (&g)[3]) {
+  static_assert(QR_NB == 32, "two 16-column tiles");
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int l16 = lane & 15, kk = lane >> 4;
+  d4_t re[3], im[3];
+#pragma unroll
+  for (int h = 0; h < 3; ++h) re[h] = im[h] = d4_t{0, 0, 0, 0};
+  const double2* V0 = Vf + (j0 + l16) * m;
+  const double2* V1 = V0 + 16 * m;
+  const bool in0 = l16 < nbp, in1 = 16 + l16 < nbp;
+  for (int64_t r0 = first + 32 * wave; r0 < end; r0 += 128) {
+    double2 a[4][2], b[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int64_t i = r0 + 8 * u + 2 * kk + h;
+        a[u][h] = (in0 && i < end) ? V0[i] : make_double2(0.0, 0.0);
+        b[u][h] = (in1 && i < end) ? V1[i] : make_double2(0.0, 0.0);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double2 x[3] = {a[u][h], a[u][h], b[u][h]}, y[3] = {a[u][h], b[u][h], b[u][h]};
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+          re[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].x, y[e].x, re[e], 0, 0, 0);
+          im[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].x, y[e].y, im[e], 0, 0, 0);
+          re[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].y, y[e].y, re[e], 0, 0, 0);
+          im[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[e].y, y[e].x, im[e], 0, 0, 0);
+        }
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][e][v][lane] = make_double2(re[e][v], im[e][v]);
+  __syncthreads();
+  const int i = t >> 4, j = t & 15, src = 16 * (i & 3) + j;
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    g[e] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const double2 v = red[w][e][i >> 2][src];
+      g[e].x += v.x;
+      g[e].y += v.y;
+    }
+  }
+}
+
+// compact WY factor (forward, columnwise; zero padded to QR_NB x QR_NB): T of a
+// single reflector is tau, and two neighbouring blocks combine to
+//   T = [[T1, -T1 (V1^H V2) T2], [0, T2]],
+// so five levels of doubling build the factor with all threads at work (a column by
+// column recurrence in one wave took 19 us). Gs holds V^H V above the diagonal and zeros
+// elsewhere.
+typedef double2 QrTile[QR_NB][QR_NB + 1];
+__device__ __forceinline__ void tmat_block(int nbp, const QrTile& Gs, QrTile& Ts, QrTile& Ms,
+                                           const double2* tau, double2* T) {
+  const int t = threadIdx.x;
+#pragma unroll
+  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
+    const int e = t + 256 * u, a = e / QR_NB, b = e % QR_NB;
+    Ts[a][b] = (a == b && a < nbp) ? tau[a] : make_double2(0.0, 0.0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 1; h < QR_NB; h *= 2) {
+    // output (i, j) of block pair b: 16 h outputs in all
+    const int b = t / (h * h), i = (t / h) % h, j = t % h;
+    const int r0 = 2 * h * b, c0 = r0 + h;
+    const bool on = t < 16 * h;
+    if (on) {   // M = (V1^H V2) T2
+      double2 m = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int k = 0; k < h; ++k) {
+        const double2 x = cmul2(Gs[r0 + i][c0 + k], Ts[c0 + k][c0 + j]);
+        m.x += x.x;
+        m.y += x.y;
+      }
+      Ms[r0 + i][c0 + j] = m;
+    }
+    __syncthreads();
+    if (on) {
+      double2 m = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int k = 0; k < h; ++k) {
+        const double2 x = cmul2(Ts[r0 + i][r0 + k], Ms[r0 + k][c0 + j]);
+        m.x -= x.x;
+        m.y -= x.y;
+      }
+      Ts[r0 + i][c0 + j] = m;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
+    const int e = t + 256 * u;
+    T[e] = Ts[e / QR_NB][e % QR_NB];
+  }
+}
+
+// V^H V over the rows j0 + rows blockIdx.x .. (rows a multiple of 128) as a partial G, and
+// T from the sum of the partials: panels of more than 256 rows (shorter ones: k_qr_panel)
+__global__ __launch_bounds__(256) void k_qr_vtv(int64_t m, int64_t j0, int nbp, int rows,
+                                                const double2* __restrict__ Vf,
+                                                double2* __restrict__ G, QrStrides bs) {
+  __shared__ VtvRed red;
+  Vf += blockIdx.y * bs.V;
+  G += blockIdx.y * bs.G + (int64_t)blockIdx.x * QR_NB * QR_NB;
+  const int64_t first = j0 + (int64_t)blockIdx.x * rows;
+  double2 g[3];
+  vtv_block(m, j0, nbp, first, first + rows < m ? first + rows : m, Vf, red, g);
+  const int i = threadIdx.x >> 4, j = threadIdx.x & 15;
+#pragma unroll
+  for (int e = 0; e < 3; ++e)
+    G[((e == 2 ? 16 : 0) + i) * QR_NB + (e == 0 ? 0 : 16) + j] = g[e];
+}
+__global__ __launch_bounds__(256) void k_qr_tmat(int nbp, int nparts, const double2* __restrict__ G,
+                                                 const double2* __restrict__ tau,
+                                                 double2* __restrict__ T, QrStrides bs) {
+  __shared__ QrTile Gs, Ts, Ms;
+  G += blockIdx.x * bs.G;
+#pragma unroll
+  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
+    const int e = threadIdx.x + 256 * u, a = e / QR_NB, b = e % QR_NB;
+    double2 g = make_double2(0.0, 0.0);
+    if (a < b && b < nbp)
+      for (int p = 0; p < nparts; ++p) {
+        const double2 v = G[(int64_t)p * QR_NB * QR_NB + e];
+        g.x += v.x;
+        g.y += v.y;
+      }
+    Gs[a][b] = g;
+  }
+  tmat_block(nbp, Gs, Ts, Ms, tau + blockIdx.x * bs.k, T + blockIdx.x * bs.T);
+}
+
 // A whole panel of at most 64 R rows factored by one workgroup with its columns
 // j0 .. j0+nbp-1 (nbp <= C NW) in registers: column j0 + q NW + w in element q of
 // wave w, row j0 + lane + 64 u in element u. The current column y is read from
@@ -544,14 +727,26 @@ __global__ __launch_bounds__(256) void k_qr_col2r(int64_t m, int64_t j, double2*
 // so the chain per column is one pass, one sum and one update. Bound by the
 // instructions of one CU: 32 columns of 256 rows take 48 us (95 with two columns
 // per launch), of 128 rows 40 us.
-// Writes v_j (rows >= j0), tau_j, R[j][j] and the rows j0 .. j-1 of R above it.
+// Writes v_j (rows >= j0), tau_j, R[j][j], the rows j0 .. j-1 of R above it, and the panel's
+// T (with its products V^H V as launches of their own 9.4 us more per panel).
 template <int R, int C, int NW>
 __global__ __launch_bounds__(64 * NW) void k_qr_panel(int64_t m, int64_t j0, int nbp,
                                                       double2* __restrict__ W,
                                                       double2* __restrict__ Vf,
                                                       double2* __restrict__ tau,
-                                                      double2* __restrict__ rdiag, QrStrides bs) {
-  __shared__ double2 Ys[2][64 * R];
+                                                      double2* __restrict__ rdiag,
+                                                      double2* __restrict__ T, QrStrides bs) {
+  static_assert(NW == 4, "256 threads");
+  struct TPart {
+    QrTile Ts, Ms;
+  };
+  __shared__ __align__(16) union {
+    double2 Ys[2][64 * R];
+    VtvRed red;
+    TPart tp;
+  } sm;
+  __shared__ QrTile Gs;
+  auto& Ys = sm.Ys;
   W += blockIdx.x * bs.W;
   Vf += blockIdx.x * bs.V;
   tau += blockIdx.x * bs.k;
@@ -661,6 +856,17 @@ __global__ __launch_bounds__(64 * NW) void k_qr_panel(int64_t m, int64_t j0, int
       __syncthreads();
     }
   }
+  // V^H V and T (the barrier above orders the stores of V and tau with these loads)
+  double2 g[3];
+  vtv_block(m, j0, nbp, j0, m, Vf, sm.red, g);
+  const int gi = threadIdx.x >> 4, gj = threadIdx.x & 15;
+  const double2 zero = make_double2(0.0, 0.0);
+  Gs[gi][gj] = gi < gj && gj < nbp ? g[0] : zero;
+  Gs[gi][16 + gj] = 16 + gj < nbp ? g[1] : zero;
+  Gs[16 + gi][gj] = zero;
+  Gs[16 + gi][16 + gj] = gi < gj && 16 + gj < nbp ? g[2] : zero;
+  __syncthreads();
+  tmat_block(nbp, Gs, sm.tp.Ts, sm.tp.Ms, tau + j0, T + blockIdx.x * bs.T);
 }
 
 // Columns j .. j+nc-1 (nc <= 4) of a panel that starts at j0, at most 256 R rows below j,
@@ -815,134 +1021,6 @@ __global__ void k_qr_fixsup(int64_t m, int64_t j0, int64_t pe, const double2* __
   if (jj + 1 < pe) W[(jj + 1) * m + jj] = rsup[jj];
 }
 
-// partial G[a][b] = v_a^H v_b (a <= b in steps of 16) of the panel's reflectors over the
-// rows j0 + rows blockIdx.x ..: FP64 MFMA on 16 x 16 tiles, the operands loaded as in the
-// cross Gram kernel of the Jacobi iteration (a lane holds rows 2 kk, 2 kk + 1 of every 8
-// of column l16); columns >= nbp count as zero. rows is a multiple of 128.
-__global__ __launch_bounds__(256) void k_qr_vtv(int64_t m, int64_t j0, int nbp, int rows,
-                                                const double2* __restrict__ Vf,
-                                                double2* __restrict__ G, QrStrides bs) {
-  static_assert(QR_NB == 32, "two 16-column tiles");
-  __shared__ double2 red[4][3][4][64];
-  Vf += blockIdx.y * bs.V;
-  G += blockIdx.y * bs.G + (int64_t)blockIdx.x * QR_NB * QR_NB;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int l16 = lane & 15, kk = lane >> 4;
-  const int64_t end = j0 + (int64_t)(blockIdx.x + 1) * rows < m
-                          ? j0 + (int64_t)(blockIdx.x + 1) * rows : m;
-  d4_t re[3], im[3];
-#pragma unroll
-  for (int h = 0; h < 3; ++h) re[h] = im[h] = d4_t{0, 0, 0, 0};
-  const double2* __restrict__ V0 = Vf + (j0 + l16) * m;
-  const double2* __restrict__ V1 = V0 + 16 * m;
-  const bool in0 = l16 < nbp, in1 = 16 + l16 < nbp;
-  for (int64_t r0 = j0 + (int64_t)blockIdx.x * rows + 32 * wave; r0 < end; r0 += 128) {
-    double2 a[4][2], b[4][2];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int64_t i = r0 + 8 * u + 2 * kk + h;
-        a[u][h] = (in0 && i < end) ? V0[i] : make_double2(0.0, 0.0);
-        b[u][h] = (in1 && i < end) ? V1[i] : make_double2(0.0, 0.0);
-      }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const double2 x[3] = {a[u][h], a[u][h], b[u][h]}, y[3] = {a[u][h], b[u][h], b[u][h]};
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-          re[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].x, y[e].x, re[e], 0, 0, 0);
-          im[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].x, y[e].y, im[e], 0, 0, 0);
-          re[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[e].y, y[e].y, re[e], 0, 0, 0);
-          im[e] = __builtin_amdgcn_mfma_f64_16x16x4f64(-x[e].y, y[e].x, im[e], 0, 0, 0);
-        }
-      }
-  }
-#pragma unroll
-  for (int e = 0; e < 3; ++e)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) red[wave][e][v][lane] = make_double2(re[e][v], im[e][v]);
-  __syncthreads();
-  const int i = t >> 4, j = t & 15, src = 16 * (i & 3) + j;
-#pragma unroll
-  for (int e = 0; e < 3; ++e) {
-    double2 sum = make_double2(0.0, 0.0);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const double2 v = red[w][e][i >> 2][src];
-      sum.x += v.x;
-      sum.y += v.y;
-    }
-    const int a0 = e == 2 ? 16 : 0, b0 = e == 0 ? 0 : 16;
-    G[(a0 + i) * QR_NB + b0 + j] = sum;
-  }
-}
-
-// compact WY factor (forward, columnwise; zero padded to QR_NB x QR_NB): T of a
-// single reflector is tau, and two neighbouring blocks combine to
-//   T = [[T1, -T1 (V1^H V2) T2], [0, T2]],
-// so five levels of doubling build the factor with all threads at work (a column by
-// column recurrence in one wave took 19 us). Sums the nparts partial G first.
-__global__ __launch_bounds__(256) void k_qr_tmat(int nbp, int nparts, const double2* __restrict__ G,
-                                                 const double2* __restrict__ tau,
-                                                 double2* __restrict__ T, QrStrides bs) {
-  G += blockIdx.x * bs.G;
-  tau += blockIdx.x * bs.k;
-  T += blockIdx.x * bs.T;
-  __shared__ double2 Gs[QR_NB][QR_NB + 1], Ts[QR_NB][QR_NB + 1], Ms[QR_NB][QR_NB + 1];
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
-    const int e = t + 256 * u, a = e / QR_NB, b = e % QR_NB;
-    double2 g = make_double2(0.0, 0.0);
-    if (a < b && b < nbp)
-      for (int p = 0; p < nparts; ++p) {
-        const double2 v = G[(int64_t)p * QR_NB * QR_NB + e];
-        g.x += v.x;
-        g.y += v.y;
-      }
-    Gs[a][b] = g;
-    Ts[a][b] = (a == b && a < nbp) ? tau[a] : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int h = 1; h < QR_NB; h *= 2) {
-    // output (i, j) of block pair b: 16 h outputs in all
-    const int b = t / (h * h), i = (t / h) % h, j = t % h;
-    const int r0 = 2 * h * b, c0 = r0 + h;
-    const bool on = t < 16 * h;
-    if (on) {   // M = (V1^H V2) T2
-      double2 m = make_double2(0.0, 0.0);
-#pragma unroll
-      for (int k = 0; k < h; ++k) {
-        const double2 x = cmul2(Gs[r0 + i][c0 + k], Ts[c0 + k][c0 + j]);
-        m.x += x.x;
-        m.y += x.y;
-      }
-      Ms[r0 + i][c0 + j] = m;
-    }
-    __syncthreads();
-    if (on) {
-      double2 m = make_double2(0.0, 0.0);
-#pragma unroll
-      for (int k = 0; k < h; ++k) {
-        const double2 x = cmul2(Ts[r0 + i][r0 + k], Ms[r0 + k][c0 + j]);
-        m.x -= x.x;
-        m.y -= x.y;
-      }
-      Ts[r0 + i][c0 + j] = m;
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
-    const int e = t + 256 * u;
-    T[e] = Ts[e / QR_NB][e % QR_NB];
-  }
-}
-
 // Y = sum of the nparts partial products P[s] (QR_NB x nc, rows < nbp used);
 // Z = -T^H Y (adjoint = 1) or Z = -T Y (adjoint = 0). A workgroup handles 8
 // columns; thread (r, cl) sums row r of column cl, then forms row r of Z.
@@ -1043,6 +1121,112 @@ QrFact qr_fact_layout(int64_t m, int64_t n, int64_t ncmax, void* ws, int64_t bat
   return f;
 }
 
+// C <- (I - V op(T) V^H) C, op(T) = T^H (ADJ) or T, on 8 columns of C (mr rows) per workgroup:
+// the product V^H C, its reduction with T and the update in one launch, for panels whose rows
+// one workgroup covers in a few steps. Y = V^H C: wave w takes rows 16 (w % 2) .. of Y and
+// every fourth part of the rows of C; the update goes over tiles of 16 rows. FP64 MFMA with
+// the real embedding of the products (gemm_impl.h), operands straight from memory.
+// Up to 256 rows (512 in a batch, whose three products fill the chip no better): QR of
+// 64 x 32 67 -> 60 us, 128 x 64 152 -> 136, 256 x 128 359 -> 340, 8 of 512 x 256 1020 -> 911; one
+// of 512 x 256 807 -> 815, of 1024 x 512 1927 -> 2232 without the limit.
+constexpr int64_t QR_APPLY_ROWS = 256;
+constexpr int QA_T = 512, QA_PARTS = QA_T / 128;
+template <bool ADJ>
+__global__ __launch_bounds__(QA_T) void k_qr_apply(int64_t ldv, int mr, int nbp,
+                                                   const double2* __restrict__ V,
+                                                   const double2* __restrict__ T,
+                                                   double2* __restrict__ C, int64_t ldc, int nc,
+                                                   QrStrides bs, int64_t sc) {
+  constexpr int U = 4;
+  __shared__ QrTile Ts;
+  __shared__ __align__(16) double2 Yp[QA_PARTS][QR_NB][8], Ys[QR_NB][9], Zs[QR_NB][8];
+  V += blockIdx.y * bs.V;
+  T += blockIdx.y * bs.T;
+  C += blockIdx.y * sc + (int64_t)blockIdx.x * 8 * ldc;
+  nc -= 8 * (int)blockIdx.x;
+  const int t = threadIdx.x, lane = t & 63, l16 = lane & 15, kk = lane >> 4, pb = lane & 1;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int col = min(l16 >> 1, nc - 1);
+  for (int e = t; e < QR_NB * QR_NB; e += QA_T) Ts[e / QR_NB][e % QR_NB] = T[e];
+  {
+    const int vc = 16 * (wave & 1) + l16, part = wave >> 1;
+    const bool on = vc < nbp;
+    const double2* pv = V + (int64_t)(on ? vc : 0) * ldv;
+    const double2* pc = C + (int64_t)col * ldc;
+    const int steps = (mr + 3) / 4, per = (steps + QA_PARTS - 1) / QA_PARTS;
+    const int s1 = min((part + 1) * per, steps);
+    d4_t acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+    for (int s = part * per; s < s1; s += U) {
+      double2 a[U], b[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int r = 4 * (s + u) + kk;
+        const bool in = s + u < s1 && r < mr;
+        a[u] = in && on ? pv[r] : make_double2(0.0, 0.0);
+        b[u] = in ? pc[r] : make_double2(0.0, 0.0);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {   // conj(a) b
+        const double br = pb ? b[u].y : b[u].x, bi = pb ? -b[u].x : b[u].y;
+        acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u].x, br, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u].y, bi, acc1, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      double* y = (double*)&Yp[part][16 * (wave & 1) + kk + 4 * v][l16 >> 1];
+      y[pb] = acc0[v] + acc1[v];
+    }
+  }
+  __syncthreads();
+  const int r = t >> 3, c = t & 7;
+  if (r < QR_NB) {
+    double2 y = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int p = 0; p < QA_PARTS; ++p) {
+      y.x += Yp[p][r][c].x;
+      y.y += Yp[p][r][c].y;
+    }
+    Ys[r][c] = y;
+  }
+  __syncthreads();
+  if (r < QR_NB) {   // Z = -op(T) Y (T is zero below the diagonal and beyond nbp)
+    double zr = 0.0, zi = 0.0;
+#pragma unroll 8
+    for (int q = 0; q < QR_NB; ++q) {
+      const double2 a = ADJ ? conj2(Ts[q][r]) : Ts[r][q], y = Ys[q][c];
+      zr = fma(-a.x, y.x, fma(a.y, y.y, zr));
+      zi = fma(-a.x, y.y, fma(-a.y, y.x, zi));
+    }
+    Zs[r][c] = make_double2(zr, zi);
+  }
+  __syncthreads();
+  double2 z[QR_NB / 4];
+#pragma unroll
+  for (int u = 0; u < QR_NB / 4; ++u) z[u] = Zs[4 * u + kk][l16 >> 1];
+  for (int m0 = 16 * wave; m0 < mr; m0 += 16 * (QA_T / 64)) {
+    const double2* pv = V + min(m0 + l16, mr - 1);
+    d4_t acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+    double2 a[QR_NB / 4];
+#pragma unroll
+    for (int u = 0; u < QR_NB / 4; ++u)
+      a[u] = 4 * u + kk < nbp ? pv[(int64_t)(4 * u + kk) * ldv] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < QR_NB / 4; ++u) {
+      acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u].x, pb ? z[u].y : z[u].x, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u].y, pb ? z[u].x : -z[u].y, acc1, 0, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = m0 + kk + 4 * v;
+      if (row < mr && (l16 >> 1) < nc) {
+        double* o = (double*)(C + (int64_t)col * ldc + row) + pb;
+        *o += acc0[v] + acc1[v];
+      }
+    }
+  }
+}
+
 // C[j0:m, c0:c0+nc] += V_panel Z with Z = -T^(H) V_panel^H C[j0:m, c0:c0+nc]
 // (C column-major with leading dimension ldc; panel columns j0 .. j0+nbp-1;
 // matrix b of a batch at C + b * sc). A single matrix splits the K = m - j0
@@ -1055,6 +1239,15 @@ static int apply_block(const QrFact& f, int64_t j0, int nbp, const double2* Tp, 
   if (nc <= 0 || mr <= 0) return PTN_OK;
   const double2* V = f.Vf + j0 * m + j0;
   double2* Cs = C + c0 * ldc + j0;
+  if (mr <= (f.batch > 1 ? 2 * QR_APPLY_ROWS : QR_APPLY_ROWS)) {
+    const dim3 g((unsigned)((nc + 7) / 8), (unsigned)f.batch);
+    if (adjoint)
+      k_qr_apply<true><<<g, QA_T, 0, s>>>(m, (int)mr, nbp, V, Tp, Cs, ldc, (int)nc, f.bs, sc);
+    else
+      k_qr_apply<false><<<g, QA_T, 0, s>>>(m, (int)mr, nbp, V, Tp, Cs, ldc, (int)nc, f.bs, sc);
+    PTN_LAUNCH_CHECK();
+    return PTN_OK;
+  }
   int st;
   int nparts;
   if (f.batch == 1) {
@@ -1092,9 +1285,11 @@ static int apply_block(const QrFact& f, int64_t j0, int nbp, const double2* Tp, 
 // workgroup of its own (512 rows: 45 us per panel against 66 in one workgroup; the
 // sub-panels of 16 and 8 columns that one CU can hold at 1024 and 2048 rows are bound by
 // that CU's FP64 and LDS rates: 90 and 200 us per panel against 52 and 63).
-template <int R> static void panel_one(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
+constexpr int64_t QR_ONE_ROWS = 256;
+template <int R>
+static void panel_one(const QrFact& f, int64_t j0, int64_t pe, double2* Tp, hipStream_t s) {
   k_qr_panel<R, 8, 4><<<(unsigned)f.batch, 256, 0, s>>>(f.m, j0, (int)(pe - j0), f.W, f.Vf, f.tau,
-                                                       f.rdiag, f.bs);
+                                                       f.rdiag, Tp, f.bs);
 }
 template <int R> static void panel_col4(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
   const unsigned B = (unsigned)f.batch;
@@ -1103,11 +1298,11 @@ template <int R> static void panel_col4(const QrFact& f, int64_t j0, int64_t pe,
         f.m, j0, j, (int)(pe - j < 4 ? pe - j : 4), f.W, f.Vf, f.tau, f.rdiag, f.G, f.bs);
   k_qr_fixup4<<<B, 256, 0, s>>>(f.m, j0, (int)(pe - j0), f.G, f.W, f.bs);
 }
-static void panel(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
+static void panel(const QrFact& f, int64_t j0, int64_t pe, double2* Tp, hipStream_t s) {
   const int64_t rows = f.m - j0;
-  if (rows <= 64) panel_one<1>(f, j0, pe, s);
-  else if (rows <= 128) panel_one<2>(f, j0, pe, s);
-  else if (rows <= 256) panel_one<4>(f, j0, pe, s);
+  if (rows <= 64) panel_one<1>(f, j0, pe, Tp, s);
+  else if (rows <= 128) panel_one<2>(f, j0, pe, Tp, s);
+  else if (rows <= QR_ONE_ROWS) panel_one<4>(f, j0, pe, Tp, s);
   else if (rows <= 512) panel_col4<2>(f, j0, pe, s);
   else if (rows <= 1024) panel_col4<4>(f, j0, pe, s);
   else panel_col4<8>(f, j0, pe, s);
@@ -1118,22 +1313,29 @@ int qr_factor(QrFact& f, const double2* a, int64_t lda, hipStream_t s, int64_t s
   if (m == 0 || n == 0) return PTN_OK;
   if (f.batch < 1 || f.batch > 65535) return PTN_ERR_ARG;
   const unsigned B = (unsigned)f.batch;
-  k_zero_u64<<<(unsigned)((f.batch + 255) / 256), 256, 0, s>>>(f.batch, f.mxb);
-  {
-    int64_t nb = (m * n + 255) / 256;
-    const int64_t cap = f.batch > 16 ? 16 : 256;   // workgroups per matrix (one atomic each)
-    if (nb > cap) nb = cap;
-    k_maxabs<<<dim3((unsigned)nb, B), 256, 0, s>>>(m, n, a, lda, sa, f.mxb);
+  if (m * n <= QR_IN_MAX) {
+    const int64_t nt = (m * n + 63) / 64 * 64;
+    k_qr_in<<<B, (unsigned)(nt < 1024 ? nt : 1024), 0, s>>>((int)m, (int)n, a, lda, f.W, sa, f.bs.W,
+                                                           f.scl);
+  } else {
+    k_zero_u64<<<(unsigned)((f.batch + 255) / 256), 256, 0, s>>>(f.batch, f.mxb);
+    {
+      int64_t nb = (m * n + 255) / 256;
+      const int64_t cap = f.batch > 16 ? 16 : 256;   // workgroups per matrix (one atomic each)
+      if (nb > cap) nb = cap;
+      k_maxabs<<<dim3((unsigned)nb, B), 256, 0, s>>>(m, n, a, lda, sa, f.mxb);
+    }
+    k_to_colmajor<<<dim3((unsigned)((m * n + 255) / 256), B), 256, 0, s>>>(m, n, a, lda, f.W, sa,
+                                                                             f.bs.W, f.mxb, f.scl);
   }
-  k_to_colmajor<<<dim3((unsigned)((m * n + 255) / 256), B), 256, 0, s>>>(m, n, a, lda, f.W, sa,
-                                                                           f.bs.W, f.mxb, f.scl);
   PTN_LAUNCH_CHECK();
   for (int64_t p = 0; p < f.npan; ++p) {
     const int64_t j0 = p * QR_NB;
     const int64_t pe = (j0 + QR_NB < k) ? j0 + QR_NB : k;
     const int nbp = (int)(pe - j0);
+    double2* Tp = f.T + p * QR_NB * QR_NB;
     if (m - j0 <= 2048) {
-      panel(f, j0, pe, s);
+      panel(f, j0, pe, Tp, s);
     } else {
       int64_t j = j0;
       for (; j + 1 < pe; j += 2) {
@@ -1147,13 +1349,13 @@ int qr_factor(QrFact& f, const double2* a, int64_t lda, hipStream_t s, int64_t s
         k_qr_col<<<dim3((unsigned)(pe - j), B), 256, 0, s>>>(m, j, f.W, f.Vf, f.tau, f.rdiag, f.bs);
       if (pe - j0 >= 2) k_qr_fixsup<<<dim3(1, B), QR_NB / 2, 0, s>>>(m, j0, pe, f.rsup, f.W, f.bs);
     }
-    PTN_LAUNCH_CHECK();
-    double2* Tp = f.T + p * QR_NB * QR_NB;
-    const int64_t np = vtv_parts(m - j0);
-    const int64_t rows = ((m - j0 + np - 1) / np + 127) / 128 * 128;
-    const int parts = (int)((m - j0 + rows - 1) / rows);
-    k_qr_vtv<<<dim3((unsigned)parts, B), 256, 0, s>>>(m, j0, nbp, (int)rows, f.Vf, f.G, f.bs);
-    k_qr_tmat<<<B, 256, 0, s>>>(nbp, parts, f.G, f.tau + j0, Tp, f.bs);
+    if (m - j0 > QR_ONE_ROWS) {
+      const int64_t np = vtv_parts(m - j0);
+      const int64_t rows = ((m - j0 + np - 1) / np + 127) / 128 * 128;
+      const int parts = (int)((m - j0 + rows - 1) / rows);
+      k_qr_vtv<<<dim3((unsigned)parts, B), 256, 0, s>>>(m, j0, nbp, (int)rows, f.Vf, f.G, f.bs);
+      k_qr_tmat<<<B, 256, 0, s>>>(nbp, parts, f.G, f.tau + j0, Tp, f.bs);
+    }
     PTN_LAUNCH_CHECK();
     int st;
     if (pe < n && (st = apply_block(f, j0, nbp, Tp, 1, f.W, m, pe, n - pe, s, f.bs.W))) return st;
