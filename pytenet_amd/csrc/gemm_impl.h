@@ -16,6 +16,7 @@
 #include <stdio.h>
 #include <string.h>
 #include <string>
+#include <type_traits>
 #include <unordered_map>
 #include "common.h"
 
@@ -424,6 +425,257 @@ __global__ __launch_bounds__(256 * WK) void zgemm_kernel(GemmKArgs g) {
   }
 }
 
+// FP64 products of complex128 operands on the 128 x 64 and 64 x 32 tiles: the loop of
+// zgemm_kernel with its stages loaded straight into LDS (global_load_lds of 16 bytes), three
+// deep, and the fragments of the next half stage read before the MFMAs of the current one.
+// Loads then need no registers and no LDS stores, stay in flight for two stages, and neither they
+// nor the LDS reads are waited for between the MFMAs; one barrier per stage is placed between
+// its halves. A wave's load writes 64 consecutive elements of LDS, so the layout follows from
+// which element a lane fetches: [k][row] for operands contiguous in rows, else [row][k] with k
+// exchanged by k ^ (row % 8), which keeps the 128-byte runs of the global reads and spreads the
+// 16 rows that a fragment read touches over all banks. The sums are those of zgemm_kernel, in
+// the same order. One array per stage and operand: the compiler then knows that a read does
+// not wait for the loads in flight to the other stages.
+// Bound by MFMA issue (84 % of the cycles busy before): 4096 x 5120 x 1024 64.6 -> 69.5 TFLOP/s,
+// 2048^3 60.8 -> 68.8 (128 x 64); 1024 x 2560 x 512 54.7 -> 62.6 (64 x 32, two groups), 512 x
+// 1024 x 2560 55.0 -> 62.9 (four groups).
+template <int N, bool LGKM = false> __device__ __forceinline__ void wait_vm() {
+  // s_waitcnt vmcnt(N), with LGKM also lgkmcnt(0)
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 0x70 | (LGKM ? 0 : 0xF00));
+}
+__device__ __forceinline__ void wg_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+template <int WK_> struct LdsRing {
+  static constexpr int WK = WK_;
+};
+template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, typename Ring,
+          bool A_KCONTIG, bool B_NCONTIG>
+__global__ __launch_bounds__(256 * Ring::WK) void zgemm_kernel(GemmKArgs g) {
+  constexpr int WK = Ring::WK;
+  static_assert(sizeof(Tc) == 8 && sizeof(TA) == 16 && sizeof(TB) == 16 && sizeof(TC) == 16,
+                "FP64 products of complex128 operands");
+  typedef TileCfg<TM, TN, 8> T;
+  constexpr int BM = T::BM, BN = T::BN, BK = 8, NA = T::NA, NB = T::NB;
+  __shared__ __align__(16) double2 A0[WK][BM * BK], A1[WK][BM * BK], A2[WK][BM * BK];
+  __shared__ __align__(16) double2 B0[WK][BN * BK], B1[WK][BN * BK], B2[WK][BN * BK];
+  if (g.skip && g.skip[blockIdx.z * g.skip_stride]) return;
+  const int grp = WK == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int tid = threadIdx.x & 255, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm0 = (wave >> 1) * T::WM, wn0 = (wave & 1) * T::WN;
+  int tm, tn;
+  tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN, bz = blockIdx.z;
+  const char* A = (const char*)((const double2*)g.A + bz * g.bz_a + m0 * g.a_m);
+  const char* B = (const char*)((const double2*)g.B + bz * g.bz_b + n0 * g.b_n);
+  double2* __restrict__ C = (double2*)g.C + bz * g.bz_c;
+  const int mlast = (int)(g.M - m0 < BM ? g.M - m0 : BM) - 1;
+  const int nlast = (int)(g.N - n0 < BN ? g.N - n0 : BN) - 1;
+  // element `lane` of chunk c (64 elements) of a stage: row / column and k
+  auto arow = [&](int c) { return A_KCONTIG ? 8 * c + (lane >> 3) : 64 * (c % (BM / 64)) + lane; };
+  auto ak = [&](int c) { return A_KCONTIG ? (lane & 7) ^ (lane >> 3) : c / (BM / 64); };
+  auto bcol = [&](int c) { return B_NCONTIG ? (64 * c + lane) % BN : 8 * c + (lane >> 3); };
+  auto bk = [&](int c) { return B_NCONTIG ? (64 * c + lane) / BN : (lane & 7) ^ (lane >> 3); };
+  uint32_t offa[NA], offb[NB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+    offa[i] = (uint32_t)((min(arow(wave * NA + i), mlast) * g.a_m + ak(wave * NA + i) * g.a_k) * 16);
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    offb[i] = (uint32_t)((min(bcol(wave * NB + i), nlast) * g.b_n + bk(wave * NB + i) * g.b_k) * 16);
+  const int nst = (int)(g.K / BK);                 // whole stages, `per` at most to a group
+  const int per = (nst + WK - 1) / WK, least = max(0, nst - (WK - 1) * per);
+  const int mine = WK == 1 ? per : min(per, max(0, nst - grp * per));
+  const int64_t sta = g.a_k * (BK * 16), stb = g.b_k * (BK * 16);
+  const char* Ag = A + (int64_t)(mine ? grp * per : 0) * sta;
+  const char* Bg = B + (int64_t)(mine ? grp * per : 0) * stb;
+  typedef const __attribute__((address_space(1))) void* gp_t;
+  typedef __attribute__((address_space(3))) void* lp_t;
+  auto dma = [&](double2 (&As)[WK][BM * BK], double2 (&Bs)[WK][BN * BK], int st) {
+    const int sc = max(min(st, mine - 1), 0);   // beyond the end: loaded again, not used
+    const char* a = Ag + sc * sta;
+    const char* b = Bg + sc * stb;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      __builtin_amdgcn_global_load_lds((gp_t)(a + offa[i]), (lp_t)&As[grp][(wave * NA + i) * 64],
+                                       16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      __builtin_amdgcn_global_load_lds((gp_t)(b + offb[i]), (lp_t)&Bs[grp][(wave * NB + i) * 64],
+                                       16, 0, 0);
+  };
+  const int l16 = lane & 15, kk = lane >> 4, pb = lane & 1;
+  // signs of the expanded B: conjugation of B in both, of A in the second one
+  const uint32_t S = 0x80000000u;
+  const uint32_t x0 = pb && g.conjB ? S : 0u, x1 = (pb || g.conjB ? 0u : S) ^ (g.conjA ? S : 0u);
+  // fragments of the first half stage; the second half: k + 4 (k ^ 4 where k is exchanged)
+  const int fa = A_KCONTIG ? (wm0 + l16) * 8 + (kk ^ (l16 & 7)) : kk * BM + wm0 + l16;
+  const int nb = l16 >> 1;
+  const int fb = B_NCONTIG ? kk * BN + wn0 + nb : (wn0 + nb) * 8 + (kk ^ nb);
+  const int fa1 = A_KCONTIG ? fa ^ 4 : fa + 4 * BM, fb1 = B_NCONTIG ? fb + 4 * BN : fb ^ 4;
+  constexpr int SA = A_KCONTIG ? 128 : 16, SB = B_NCONTIG ? 8 : 64;
+  struct Frag {
+    double2 a[TM], b[TN];
+  };
+  auto read = [&](const double2 (&As)[WK][BM * BK], const double2 (&Bs)[WK][BN * BK], int h,
+                  Frag& f) {
+    const double2* pa = &As[grp][h ? fa1 : fa];
+    const double2* pbb = &Bs[grp][h ? fb1 : fb];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) f.a[i] = pa[i * SA];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) f.b[j] = pbb[j * SB];
+  };
+  d4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = d4_t{0, 0, 0, 0};
+  auto flip = [](double v, uint32_t m) {
+    const long long b = __double_as_longlong(v);
+    return __longlong_as_double(((long long)((uint32_t)(b >> 32) ^ m) << 32) | (uint32_t)b);
+  };
+  auto mul = [&](const Frag& f) {
+    double b0[TN], b1[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      b0[j] = flip(pb ? f.b[j].y : f.b[j].x, x0);
+      b1[j] = flip(pb ? f.b[j].x : f.b[j].y, x1);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(f.a[i].x, b0[j], acc[i][j]);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma16(f.a[i].y, b1[j], acc[i][j]);
+  };
+  constexpr int VM = NA + NB;                      // loads of a stage
+  auto sync = [&]() {
+    wait_vm<VM, true>();
+    wg_barrier();
+  };
+  Frag cur, nxt;
+  auto step = [&](double2 (&As)[WK][BM * BK], double2 (&Bs)[WK][BN * BK],
+                  double2 (&An)[WK][BM * BK], double2 (&Bn)[WK][BN * BK], int st, bool on) {
+    read(As, Bs, 1, nxt);
+    if (on) mul(cur);
+    sync();             // stage st + 1 has landed and every wave has read stage st
+    dma(As, Bs, st + 3);
+    read(An, Bn, 0, cur);
+    if (on) mul(nxt);
+  };
+  if (per > 0) {
+    dma(A0, B0, 0);
+    dma(A1, B1, 1);
+    dma(A2, B2, 2);
+    wait_vm<2 * VM>();
+    wg_barrier();
+    read(A0, B0, 0, cur);
+    int st = 0;
+    for (; st + 3 <= least; st += 3) {
+      step(A0, B0, A1, B1, st, true);
+      step(A1, B1, A2, B2, st + 1, true);
+      step(A2, B2, A0, B0, st + 2, true);
+    }
+    for (; st < per; st += 3) {
+      step(A0, B0, A1, B1, st, st < mine);
+      if (st + 1 < per) step(A1, B1, A2, B2, st + 1, st + 1 < mine);
+      if (st + 2 < per) step(A2, B2, A0, B0, st + 2, st + 2 < mine);
+    }
+    __builtin_amdgcn_s_waitcnt(0x70);   // no load may land in LDS from here on
+  }
+  __syncthreads();
+  const int rem = (int)(g.K - (int64_t)nst * BK);
+  if (rem) {   // the last, partial stage through registers, by the last group
+    const int64_t k0 = (int64_t)nst * BK;
+    if (grp == WK - 1) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const int c = wave * NA + i;
+        double2 v = make_double2(0.0, 0.0);
+        if (ak(c) < rem)
+          v = *(const double2*)(A + ((int64_t)min(arow(c), mlast) * g.a_m + (k0 + ak(c)) * g.a_k) * 16);
+        A0[grp][c * 64 + lane] = v;
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int c = wave * NB + i;
+        double2 v = make_double2(0.0, 0.0);
+        if (bk(c) < rem)
+          v = *(const double2*)(B + ((int64_t)min(bcol(c), nlast) * g.b_n + (k0 + bk(c)) * g.b_k) * 16);
+        B0[grp][c * 64 + lane] = v;
+      }
+    }
+    __syncthreads();
+    if (grp == WK - 1) {
+      read(A0, B0, 0, cur);
+      read(A0, B0, 1, nxt);
+      mul(cur);
+      mul(nxt);
+    }
+    __syncthreads();
+  }
+  if constexpr (WK > 1) {
+    constexpr int ROW = TN * 4 * 256;
+    static_assert(ROW * 8 <= sizeof(A0), "a group's sums fit an operand buffer");
+    double* pool[3] = {(double*)&A0[0][0], (double*)&A1[0][0], (double*)&A2[0][0]};
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int w = 1; w < WK; ++w)
+        if (grp == w) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) pool[w - 1][(j * 4 + v) * 256 + tid] = acc[i][j][v];
+        }
+      __syncthreads();
+      if (grp == 0) {
+#pragma unroll
+        for (int w = 1; w < WK; ++w)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[i][j][v] += pool[w - 1][(j * 4 + v) * 256 + tid];
+      }
+      __syncthreads();
+    }
+    if (grp > 0) return;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      double mine_[4], other[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        mine_[v] = acc[i][j][v];
+        other[v] = __shfl_xor(mine_[v], 1);
+      }
+      const int64_t n = n0 + wn0 + 8 * j + (l16 >> 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int v = 2 * pb + h;
+        const int64_t m = m0 + wm0 + 16 * i + acc4<double>::row(kk, v);
+        double re = pb ? other[2 + h] : mine_[h];
+        double im = pb ? mine_[2 + h] : other[h];
+        if (m < g.M && n < g.N) {
+          double2* p = C + m * g.c_m + n * g.c_n;
+          if (g.accumulate) {
+            re += p->x;
+            im += p->y;
+          }
+          *p = make_double2(re, im);
+        }
+      }
+    }
+}
+
 // The smallest products. A workgroup of WK waves owns 16 rows x (8*TN) complex
 // columns and every wave takes its part of k: a product of a few thousand
 // outputs then reaches all CUs, which the 2 x 2-wave tiles above do not (64 x 256
@@ -643,6 +895,32 @@ inline bool fill_args(const ZGemm& z, GemmKArgs& g, int BM, int BN) {
     return PTN_OK;                                                                              \
   } while (0)
 
+// loads of 16 bytes into LDS need operands on 16-byte boundaries
+inline bool dma_operands(const ZGemm& z) { return (((uintptr_t)z.A | (uintptr_t)z.B) & 15) == 0; }
+template <int TM, int TN, int WK>
+inline int launch_dma(const ZGemm& z, const GemmKArgs& g, hipStream_t s) {
+  const bool ak = (z.a_k == 1) || (z.a_m != 1), bn = (z.b_n == 1) || (z.b_k != 1);
+  const dim3 grid((unsigned)((int64_t)g.tiles_m * g.tiles_n), 1, (unsigned)z.batch);
+  const double fl = gemm_flop(z), by = gemm_bytes<double2, double2, double2>(z);
+  auto go = [&](auto a, auto b) {
+    static const std::string nm =
+        "zgemm_kernel<double, c128, c128, c128, " + std::to_string(TM) + ", " +
+        std::to_string(TN) + ", LdsRing<" + std::to_string(WK) + ">, " +
+        (a.value ? "true" : "false") + ", " + (b.value ? "true" : "false") + ">";
+    tlaunch(nm.c_str(), fl, by,
+            zgemm_kernel<double, double2, double2, double2, TM, TN, LdsRing<WK>, a.value, b.value>,
+            grid, dim3(256 * WK), s, g);
+  };
+  using Y = std::true_type;
+  using N = std::false_type;
+  if (ak && bn) go(Y(), Y());
+  else if (ak) go(Y(), N());
+  else if (bn) go(N(), Y());
+  else go(N(), N());
+  PTN_LAUNCH_CHECK();
+  return PTN_OK;
+}
+
 template <typename Tc, typename TA, typename TB, typename TC, int TM, int TN, int WK = 1>
 inline int launch_cfg(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t mws_bytes = 0) {
   typedef TileCfg<TM, TN, StageK<Tc, TM>::value> T;
@@ -655,6 +933,10 @@ inline int launch_cfg(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t
            (T::BN * z.b_n + T::BK * z.b_k) * (int64_t)sizeof(TB) < lim;
   int st = build_masks<TA, TB>(z, g, T::BM, T::BN, T::BK, mws, mws_bytes, s);
   if (st) return st;
+  if constexpr (sizeof(Tc) == 8 && TM >= 2) {
+    static_assert(sizeof(TA) == 16 && sizeof(TB) == 16 && sizeof(TC) == 16, "complex128 operands");
+    if (g.fast && !g.maskA && dma_operands(z)) return launch_dma<TM, TN, WK>(z, g, s);
+  }
   auto nm = [](bool ak, bool bn) {   // formatted once per instance
     static const char* const n[4] = {gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(false, false),
                                      gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(false, true),
@@ -691,13 +973,16 @@ bool autotune_enabled();
 //    against 11.3 of the next best; 128 x 256 x 640: 9.1 against 18.5; equal at
 //    200 x 400 x 1000 = 650 tiles); below K = 192 four waves have work enough.
 //  * large tiles (128 x 64; FP32 also 128 x 128) where their number fills whole waves
-//    of two workgroups per CU: full waves 65.4 TFLOP/s against 63.0 of 64 x 32 tiles
+//    of two workgroups per CU: full waves 69.2 TFLOP/s against 67.0 of 64 x 32 tiles
 //    (1024 x 4096 x 5120), but 53.6 against 62.3 with 640 tiles in 512 slots
-//    (5120 x 1024 x 2048). FP32: 128 x 128 down to 0.8 of a wave's slots.
+//    (5120 x 1024 x 2048, without the loads into LDS). FP32: 128 x 128 down to 0.8 of a wave's
+//    slots.
 //  * 64 x 32 tiles from 192 up. Fewer than about two per CU leave the matrix cores
 //    waiting for operands: then k is split over two or four groups of the workgroup
-//    (256 tiles, 512 x 1024 x 2560: 44.4 / 49.6 / 55.0 TFLOP/s with 1 / 2 / 4 groups;
-//    1280 tiles, 1024 x 2560 x 512: 59.0 / 55.9 / 51.2).
+//    (256 tiles, 512 x 1024 x 2560: 50.1 / 61.8 / 62.9 TFLOP/s with 1 / 2 / 4 groups).
+//    With loads into LDS two groups pay up to 2048 tiles (1280 tiles, 1024 x 2560 x 512: 59.7 /
+//    62.6 / 56.9; 2048, 2048^3: 66.0 / 66.4; 10240: 67.2 / 66.5), staged through registers
+//    one group does from 600 on (1280 tiles: 59.0 / 55.9 / 51.2).
 //  * tile-skipping products (mask workspace given) never take the large tiles: the
 //    small one skips the zero blocks of sector-structured operands at finer
 //    granularity, which outweighs its lower efficiency per flop (U(1) two-site DMRG
@@ -726,11 +1011,13 @@ inline int launch_heuristic(const ZGemm& z, hipStream_t s, void* mws, size_t mws
       return launch_cfg<Tc, TA, TB, TC, 4, 8>(z, s);
   }
   const int64_t t44 = tiles_of(z, 128, 64), t22 = tiles_of(z, 64, 32), t11 = tiles_of(z, 32, 16);
-  if (!masked && t44 >= 512 && wave_fill(t44, 512) >= 0.95)
+  const bool dma = sizeof(Tc) == 8 && !masked && dma_operands(z);
+  if (!masked && t44 >= 512 && wave_fill(t44, 512) >= 0.96)
     return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s);
   if (t22 >= 192 && 3 * t22 <= t11) {   // t11 / t22 is 4 without padding
-    if (t22 >= 600 || z.K < 64) return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
-    if (z.K < 256) return launch_cfg<Tc, TA, TB, TC, 2, 2, 2>(z, s, mws, mws_bytes);
+    if (t22 >= (dma ? 2048 : 600) || z.K < 64)
+      return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
+    if (z.K < 256 || t22 >= 600) return launch_cfg<Tc, TA, TB, TC, 2, 2, 2>(z, s, mws, mws_bytes);
     return launch_cfg<Tc, TA, TB, TC, 2, 2, 4>(z, s, mws, mws_bytes);
   }
   if (z.K < 64 || t11 >= 512) return launch_cfg<Tc, TA, TB, TC, 1, 1>(z, s, mws, mws_bytes);
