@@ -13,6 +13,8 @@
 // CU. expm with 10 steps, MPO bond 5, one launch against the launches per step: two sites
 // D = 8 168 -> 65 us, 14 193 -> 127; one site D = 16 178 -> 90, 16 x 24 (1.2 MFLOP per
 // matvec) 192 -> 125; the two meet near 2 MFLOP.
+#include "wave_product.h"
+
 namespace ptn {
 
 constexpr double SMALL_FLOP = 1.6e6;
@@ -21,69 +23,6 @@ constexpr int64_t SMALL_N = 2048;        // longest vector
 constexpr int SMALL_LDS = 148 * 1024;
 constexpr int SMALL_MIX = 32;            // largest row or column count of the MPO matrix (as mode_mix)
 constexpr int SMALL_W = 1024;            // largest number of its entries
-
-// C = A . B with M x N outputs and K terms in ks parts: A(m, k) at a[m * am + k * ak],
-// B(k, n) at b[k * bk + n]; part p of output (m, n) goes to c[p * cp + m * cm + n]. A wave
-// takes tiles of 16 x 8 (tn of them per row of tiles, tk = tn ks with the parts); rows and
-// columns beyond the ends repeat the last ones, terms beyond K are zero.
-struct SmallProduct {
-  int M, N, K, am, ak, bk, cm, ks, cp, per, tk, tn, tiles;
-  float rk, rn;                           // 1 / tk, 1 / tn: exact quotients below 2^14
-};
-template <typename PA, typename PB>
-__device__ __forceinline__ void small_product(const SmallProduct& g, PA a, PB b, double2* c) {
-  constexpr int U = 2;                    // steps per batch of loads
-  const int lane = threadIdx.x & 63, l16 = lane & 15, kk = lane >> 4, pb = lane & 1;
-  const int nw = blockDim.x >> 6, whole = g.K >> 2;
-  for (int t = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); t < g.tiles; t += nw) {
-    const int mt = __builtin_amdgcn_readfirstlane((int)(((float)t + 0.5f) * g.rk));
-    const int q = t - mt * g.tk;
-    const int p = __builtin_amdgcn_readfirstlane((int)(((float)q + 0.5f) * g.rn));
-    const int m0 = 16 * mt, n0 = 8 * (q - p * g.tn);
-    const int s0 = p * g.per, s1 = min(s0 + g.per, whole);   // whole steps of four k
-    const int col = n0 + (l16 >> 1);
-    const PA ra = a + min(m0 + l16, g.M - 1) * g.am + kk * g.ak;
-    const PB rb = b + min(col, g.N - 1) + kk * g.bk;
-    d4_t acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
-    double2 xa[U], xb[U], ya[U], yb[U];
-    auto load = [&](int s, double2 (&fa)[U], double2 (&fb)[U]) {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (s + u < s1) {
-          fa[u] = ra[4 * (s + u) * g.ak];
-          fb[u] = rb[4 * (s + u) * g.bk];
-        }
-    };
-    auto step = [&](double2 fa, double2 fb) {
-      acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa.x, pb ? fb.y : fb.x, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa.y, pb ? fb.x : -fb.y, acc1, 0, 0, 0);
-    };
-    auto multiply = [&](int s, const double2 (&fa)[U], const double2 (&fb)[U]) {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (s + u < s1) step(fa[u], fb[u]);
-    };
-    load(s0, xa, xb);
-    for (int s = s0; s < s1; s += 2 * U) {
-      load(s + U, ya, yb);
-      multiply(s, xa, xb);
-      load(s + 2 * U, xa, xb);
-      multiply(s + U, ya, yb);
-    }
-    if ((g.K & 3) && p == g.ks - 1) {     // the last terms
-      const bool in = 4 * whole + kk < g.K;
-      const double2 z = make_double2(0.0, 0.0);
-      step(in ? ra[4 * whole * g.ak] : z, in ? rb[4 * whole * g.bk] : z);
-    }
-    // result element v: row lane / 16 + 4 v, column lane % 16 (real and imaginary parts)
-    double* o = (double*)(c + p * g.cp + col) + pb;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = m0 + kk + 4 * v;
-      if (row < g.M && col < g.N) o[2 * row * g.cm] = acc0[v] + acc1[v];
-    }
-  }
-}
 
 struct LzSmall {
   int heff, Dl, d, Dr, Ml, Mr, n, numiter, mode;
@@ -187,7 +126,14 @@ __global__ __launch_bounds__(SHORT_T) void k_lz_solve(LzSmall g) {
     double b0 = 0.0;
     for (int j = 0; j < g.numiter; ++j) {
       // T1[(l, s), (m', r')] = A R, T2 = W T1, w = L^T T2
-      small_product(g.g1, (const double2*)v, R, t1);
+      const auto same = [](int n_) { return n_; };
+      const int wcols = g.g3.N;
+      const auto out_at = [&](int p, int m_, int n_, int part) {
+        return (double*)&wv[p * n + m_ * wcols + n_] + part;
+      };
+      small_product<false>(g.g1, (const double2*)v, R, same, [&](int, int m_, int n_, int part) {
+        return (double*)&t1[m_ * g.ld1 + n_] + part;
+      });
       lds_barrier();
       if (g.heff) {
         // a thread takes a unit (l, r') and a part of the rows' entries
@@ -224,9 +170,9 @@ __global__ __launch_bounds__(SHORT_T) void k_lz_solve(LzSmall g) {
           }
         }
         lds_barrier();
-        small_product(g.g3, L, (const double2*)t2, wv);
+        small_product<false>(g.g3, L, (const double2*)t2, same, out_at);
       } else {
-        small_product(g.g3, L, (const double2*)t1, wv);
+        small_product<false>(g.g3, L, (const double2*)t1, same, out_at);
       }
       lds_barrier();
       // alpha_j, the update of w, beta_j with the breakdown test, v_{j+1} (k_lz_step)
@@ -356,28 +302,8 @@ static bool small_plan(const ptn_local_op* op, int numiter, int64_t batch, LzSma
   const int64_t tiles = (op->Dl + 15) / 16 * ((n2 + 7) / 8), steps = (op->Dl * op->Ml + 3) / 4;
   int ks = 1;
   while (ks < 4 && tiles * ks * 2 <= SHORT_T / 64 && steps >= 4 * ks && (!heff || 2 * ks * n <= s1)) ks *= 2;
-  auto product = [](int64_t M, int64_t N, int64_t K, int64_t am, int64_t ak, int64_t bk, int64_t cm,
-                    int ks, int64_t cp) {
-    SmallProduct p{};
-    p.M = (int)M;
-    p.N = (int)N;
-    p.K = (int)K;
-    p.am = (int)am;
-    p.ak = (int)ak;
-    p.bk = (int)bk;
-    p.cm = (int)cm;
-    p.ks = ks;
-    p.cp = (int)cp;
-    p.per = (int)((K + 4 * ks - 1) / (4 * ks));
-    p.tn = (int)((N + 7) / 8);
-    p.tk = p.tn * ks;
-    p.tiles = (int)((M + 15) / 16) * p.tk;
-    p.rk = 1.0f / (float)p.tk;
-    p.rn = 1.0f / (float)p.tn;
-    return p;
-  };
-  g->g1 = product(op->Dl * d, n1, op->Dr, op->Dr, 1, n1, g->ld1, 1, 0);
-  g->g3 = product(op->Dl, n2, op->Dl * op->Ml, 1, op->Dl, heff ? g->ld2 : n2, n2, ks, n);
+  g->g1 = small_product_of(op->Dl * d, n1, op->Dr, op->Dr, 1, n1, 1);
+  g->g3 = small_product_of(op->Dl, n2, op->Dl * op->Ml, 1, op->Dl, heff ? g->ld2 : n2, ks);
   g->rdr = 1.0f / (float)op->Dr;
   const int64_t up = (op->Dl * op->Dr + 63) / 64 * 64;
   g->parts = (int)std::max<int64_t>(1, std::min<int64_t>(SHORT_T / up, no));

@@ -23,6 +23,10 @@ int env_right(int prec, const Dims& D, const void* a, const void* b, const void*
               int tr, void* out, void* ws, size_t ws_bytes, hipStream_t s, int64_t batch = 1);
 int env_left(int prec, const Dims& D, const void* a, const void* b, const void* w, const void* l,
              int tl, void* out, void* ws, size_t ws_bytes, hipStream_t s, int64_t batch = 1);
+// the contractions of small bonds in one launch (fused.hip); *done = false: not applicable
+enum { FUSED_HEFF = 0, FUSED_ENV_LEFT = 1, FUSED_ENV_RIGHT = 2 };
+int fused_apply(int kind, const Dims& D, const void* a, const void* b, const void* w, const void* f,
+                void* out, hipStream_t s, int64_t batch, bool* done);
 int convert_c128_c64(int64_t n, const void* x, void* y, hipStream_t s);
 
 // sector-grouped H_eff (U(1) quantum numbers, batch 1): the plan of an

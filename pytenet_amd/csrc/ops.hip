@@ -115,6 +115,12 @@ int heff_apply(int prec, const Dims& D, const void* l, int tl, const void* w, co
   if (!dims_ok(D) || batch < 1) return PTN_ERR_ARG;
   const size_t wtot = heff_ws_bytes(prec, D, batch);
   if (ws_bytes < wtot) return PTN_ERR_WORKSPACE;
+  if (prec == PTN_FP64 && tl == PTN_T_C128 && tr == PTN_T_C128 && ta == PTN_T_C128 &&
+      tout == PTN_T_C128) {
+    bool done;
+    const int e = fused_apply(FUSED_HEFF, D, a, r, w, l, out, s, batch, &done);
+    if (e || done) return e;
+  }
   const size_t spb = split2(prec, batch, D.Dl * D.d, D.Mr * D.Dr, D.Dr, D.Dl, D.d * D.Dr,
                             D.Dl * D.Ml);
   void* sws = spb ? (char*)ws + (wtot - spb) : nullptr;
@@ -160,6 +166,11 @@ int env_right(int prec, const Dims& D, const void* a, const void* b, const void*
   if (!dims_ok(D) || batch < 1) return PTN_ERR_ARG;
   const size_t wtot = env_ws_bytes(prec, D, batch);
   if (ws_bytes < wtot) return PTN_ERR_WORKSPACE;
+  if (prec == PTN_FP64 && tr == PTN_T_C128) {
+    bool done;
+    const int e = fused_apply(FUSED_ENV_RIGHT, D, a, r, w, b, out, s, batch, &done);
+    if (e || done) return e;
+  }
   const size_t spb = split2(prec, batch, D.Dl * D.d, D.Mr * D.Dr, D.Dr, D.Dl * D.Ml, D.Dl,
                             D.d * D.Dr);
   void* sws = spb ? (char*)ws + (wtot - spb) : nullptr;
@@ -198,6 +209,11 @@ int env_left(int prec, const Dims& D, const void* a, const void* b, const void* 
   if (!dims_ok(D) || batch < 1) return PTN_ERR_ARG;
   const size_t wtot = env_ws_bytes(prec, D, batch);
   if (ws_bytes < wtot) return PTN_ERR_WORKSPACE;
+  if (prec == PTN_FP64 && tl == PTN_T_C128) {
+    bool done;
+    const int e = fused_apply(FUSED_ENV_LEFT, D, l, b, w, a, out, s, batch, &done);
+    if (e || done) return e;
+  }
   const size_t spb = split2(prec, batch, D.Dl * D.Ml, D.d * D.Dr, D.Dl, D.Dr, D.Mr * D.Dr,
                             D.Dl * D.d);
   void* sws = spb ? (char*)ws + (wtot - spb) : nullptr;
