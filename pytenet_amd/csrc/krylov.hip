@@ -226,13 +226,21 @@ constexpr int64_t SHORT_MAX = 8 * SHORT_T;
 // sum over the workgroup (up to 16 waves) in a fixed order, in every thread: the sums of
 // each wave's rows of 16 lanes through LDS, then lane l of a row adds those of wave l. red
 // is not written again until the caller's next barrier after it.
-__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4]) {
-  v = row_sum(v);
+// Of the first `waves` waves; the others only take part in the barrier (result 0).
+__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4], int waves) {
   const int t = threadIdx.x, w = t & 15;
-  if (w == 0) red[t >> 6][(t >> 4) & 3] = v;
+  const bool on = t >> 6 < waves;
+  if (on) {
+    v = row_sum(v);
+    if (w == 0) red[t >> 6][(t >> 4) & 3] = v;
+  }
   lds_barrier();
+  if (!on) return 0.0;
   const double s = (red[w][0] + red[w][1]) + (red[w][2] + red[w][3]);
-  return row_sum(w < (int)(blockDim.x >> 6) ? s : 0.0);
+  return row_sum(w < waves ? s : 0.0);
+}
+__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4]) {
+  return wg_sum(v, red, (int)(blockDim.x >> 6));
 }
 
 // x / b from inv = 1 / b with one correction (b a normal number)

@@ -11,8 +11,8 @@
 // One CU has 1/256 of the chip's matrix rate (0.28 TFLOP/s) and every phase of a
 // matvec waits for LDS and L2, so this pays up to SMALL_FLOP per matvec and one workgroup per
 // CU. expm with 10 steps, MPO bond 5, one launch against the launches per step: two sites
-// D = 8 168 -> 65 us, 14 193 -> 127; one site D = 16 178 -> 90, 16 x 24 (1.2 MFLOP per
-// matvec) 192 -> 125; the two meet near 2 MFLOP.
+// D = 8 168 -> 58 us, 14 193 -> 127; one site D = 16 178 -> 86, 16 x 24 (1.2 MFLOP per
+// matvec) 192 -> 123; the two meet near 2 MFLOP.
 #include "wave_product.h"
 
 namespace ptn {
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(SHORT_T) void k_lz_solve(LzSmall g) {
   __shared__ int part_end[SMALL_MIX + 1], used[SMALL_MIX];
   __shared__ short src[SMALL_W], dst[SMALL_W], row[SMALL_W];
   __shared__ int count[SMALL_W / 64];
-  __shared__ int conv_s;
+  __shared__ int conv_s, st[4];
   __shared__ double en_s;
   const int t = threadIdx.x, b = blockIdx.x, n = g.n;
   const double2* L = g.l + (int64_t)b * g.Dl * g.Ml * g.Dl;
@@ -111,11 +111,17 @@ __global__ __launch_bounds__(SHORT_T) void k_lz_solve(LzSmall g) {
       part_end[t] = c;
     }
   }
-  int nvalid = g.numiter, breakdown = 0, nonfinite = 0, zero = 0;
-  if (!(nrm > 0.0) || !isfinite(nrm)) {
-    if (nrm == 0.0) zero = 1; else nonfinite = 1;
-    nvalid = 0;
-  } else {
+  // vectors in use, breakdown step + 1, non-finite value, zero start: uniform through LDS
+  const bool bad = !(nrm > 0.0) || !isfinite(nrm);
+  if (t == 0) {
+    st[0] = bad ? 0 : g.numiter;
+    st[1] = 0;
+    st[2] = bad && nrm != 0.0;
+    st[3] = nrm == 0.0;
+  }
+  const int waves = min(NT, (n + 63) & ~63) >> 6;   // waves that hold elements
+  const bool mine = t >> 6 < waves;
+  if (!bad) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int i = t + e * NT;
@@ -175,56 +181,68 @@ __global__ __launch_bounds__(SHORT_T) void k_lz_solve(LzSmall g) {
         small_product<false>(g.g3, L, (const double2*)t1, same, out_at);
       }
       lds_barrier();
-      // alpha_j, the update of w, beta_j with the breakdown test, v_{j+1} (k_lz_step)
+      // alpha_j, the update of w, beta_j with the breakdown test, v_{j+1} (k_lz_step), by the
+      // waves that hold elements: the others would only take issue slots from them
       s = 0;
+      if (mine) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int i = t + e * NT;
-        x[e] = make_double2(0.0, 0.0);
-        if (i < n) {
-          x[e] = wv[i];
-          for (int p = 1; p < g.g3.ks; ++p) {
-            const double2 z = wv[p * n + i];
-            x[e].x += z.x;
-            x[e].y += z.y;
+        for (int e = 0; e < E; ++e) {
+          const int i = t + e * NT;
+          x[e] = make_double2(0.0, 0.0);
+          if (i < n) {
+            x[e] = wv[i];
+            for (int p = 1; p < g.g3.ks; ++p) {
+              const double2 z = wv[p * n + i];
+              x[e].x += z.x;
+              x[e].y += z.y;
+            }
+          }
+          s += x[e].x * vc[e].x + x[e].y * vc[e].y;
+        }
+      }
+      const double a = wg_sum(s, red[1], waves);
+      const bool last = j + 1 == g.numiter, nfa = !isfinite(a);
+      if (t == 0) {
+        al[j] = a;
+        if (nfa) { st[0] = last ? g.numiter : j + 1; st[2] = 1; }
+      }
+      if (last) break;
+      s = 0;
+      if (mine) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          x[e].x -= a * vc[e].x + b0 * vp[e].x;
+          x[e].y -= a * vc[e].y + b0 * vp[e].y;
+          s += x[e].x * x[e].x + x[e].y * x[e].y;
+        }
+      }
+      s = wg_sum(s, red[2], waves);
+      if (mine && !nfa) {
+        const bool mid = s > 1e-280 && s < 1e280;
+        const double inv = mid ? rsq_full(s) : 1.0 / sqrt(s), bn = mid ? s * inv : sqrt(s);
+        const bool nfb = !isfinite(bn), brk = !nfb && bn < g.thresh;
+        if (t == 0) {
+          if (nfb) { st[0] = j + 1; st[2] = 1; }
+          else if (brk) st[0] = st[1] = j + 1;
+          else be[j] = bn;
+        }
+        if (!nfb && !brk) {
+          b0 = bn;
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const int i = t + e * NT;
+            vp[e] = vc[e];
+            vc[e] = make_double2(div_by(x[e].x, bn, inv), div_by(x[e].y, bn, inv));
+            if (i < n) v[i] = V[(int64_t)(j + 1) * g.js + i] = vc[e];
           }
         }
-        s += x[e].x * vc[e].x + x[e].y * vc[e].y;
-      }
-      const double a = wg_sum(s, red[1]);
-      if (t == 0) al[j] = a;
-      if (!isfinite(a)) {
-        nonfinite = 1;
-        if (j + 1 < g.numiter) nvalid = j + 1;
-        break;
-      }
-      if (j + 1 == g.numiter) break;
-      s = 0;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        x[e].x -= a * vc[e].x + b0 * vp[e].x;
-        x[e].y -= a * vc[e].y + b0 * vp[e].y;
-        s += x[e].x * x[e].x + x[e].y * x[e].y;
-      }
-      s = wg_sum(s, red[2]);
-      const bool mid = s > 1e-280 && s < 1e280;
-      const double inv = mid ? rsq_full(s) : 1.0 / sqrt(s), bn = mid ? s * inv : sqrt(s);
-      if (!isfinite(bn)) { nonfinite = 1; nvalid = j + 1; break; }
-      if (bn < g.thresh) { breakdown = j + 1; nvalid = j + 1; break; }
-      if (t == 0) be[j] = bn;
-      b0 = bn;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int i = t + e * NT;
-        vp[e] = vc[e];
-        vc[e] = make_double2(div_by(x[e].x, bn, inv), div_by(x[e].y, bn, inv));
-        if (i < n) v[i] = V[(int64_t)(j + 1) * g.js + i] = vc[e];
       }
       lds_barrier();
+      if (st[1] | st[2]) break;
     }
   }
   __syncthreads();
-  const int nv = nonfinite ? 0 : nvalid;
+  const int nvalid = st[0], nv = st[2] ? 0 : nvalid;
   if (t < 64) {
     double cr = 0.0, ci = 0.0, en = 0.0;
     bool conv = true;
@@ -253,9 +271,9 @@ __global__ __launch_bounds__(SHORT_T) void k_lz_solve(LzSmall g) {
     if (g.info) {
       int32_t* o = g.info + 4 * b;
       o[0] = nvalid;
-      o[1] = breakdown;
-      o[2] = nonfinite | (conv_s ? 0 : 2);
-      o[3] = zero;
+      o[1] = st[1];
+      o[2] = st[2] | (conv_s ? 0 : 2);
+      o[3] = st[3];
     }
     if (g.energy) g.energy[b] = en_s;
   }
