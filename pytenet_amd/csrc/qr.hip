@@ -725,10 +725,11 @@ __global__ __launch_bounds__(256) void k_qr_tmat(int nbp, int nparts, const doub
 // same pass, sums them inside the wave and derives the reflector itself,
 //   v = [1, sc y],  x_j -= f,  x -= f sc y  with  f = conj(tau) (x_j + conj(sc) y^H x),
 // so the chain per column is one pass, one sum and one update. Bound by the
-// instructions of one CU: 32 columns of 256 rows take 48 us (95 with two columns
-// per launch), of 128 rows 40 us.
+// instructions of one CU: 32 columns of 256 rows take 60 us with T (48 before, 95 with two
+// columns per launch), of 128 rows 48, of 64 rows 43; up to 16 columns of 64 rows 16 us with four
+// columns per wave (22 with eight, half of them empty).
 // Writes v_j (rows >= j0), tau_j, R[j][j], the rows j0 .. j-1 of R above it, and the panel's
-// T (with its products V^H V as launches of their own 9.4 us more per panel).
+// T (about 12 us, as long as the two launches that form it for longer panels, without the gaps).
 template <int R, int C, int NW>
 __global__ __launch_bounds__(64 * NW) void k_qr_panel(int64_t m, int64_t j0, int nbp,
                                                       double2* __restrict__ W,
@@ -1288,8 +1289,13 @@ static int apply_block(const QrFact& f, int64_t j0, int nbp, const double2* Tp, 
 constexpr int64_t QR_ONE_ROWS = 256;
 template <int R>
 static void panel_one(const QrFact& f, int64_t j0, int64_t pe, double2* Tp, hipStream_t s) {
-  k_qr_panel<R, 8, 4><<<(unsigned)f.batch, 256, 0, s>>>(f.m, j0, (int)(pe - j0), f.W, f.Vf, f.tau,
-                                                       f.rdiag, Tp, f.bs);
+  const int nbp = (int)(pe - j0);
+  if (nbp <= 16)   // four columns per wave: half of the products and sums per reflector
+    k_qr_panel<R, 4, 4><<<(unsigned)f.batch, 256, 0, s>>>(f.m, j0, nbp, f.W, f.Vf, f.tau, f.rdiag,
+                                                         Tp, f.bs);
+  else
+    k_qr_panel<R, 8, 4><<<(unsigned)f.batch, 256, 0, s>>>(f.m, j0, nbp, f.W, f.Vf, f.tau, f.rdiag,
+                                                         Tp, f.bs);
 }
 template <int R> static void panel_col4(const QrFact& f, int64_t j0, int64_t pe, hipStream_t s) {
   const unsigned B = (unsigned)f.batch;
