@@ -118,8 +118,8 @@ def run_leg(H, psi0, prec, warmup, steps, D, numiter, svd_precond32=None, decide
 def _kernel_bound(name):
     """(bound, peak, unit) of a timed kernel instance: the complex products
     and the Jacobi Gram kernel are MFMA-bound (8 flops per complex
-    multiply-add, the peak of their arithmetic), the Jacobi apply kernel
-    streams the rotated columns (HBM); the rotation solve is latency-bound and
+    multiply-add, the peak of their arithmetic), the Jacobi apply and cross
+    Gram kernels stream the columns (HBM); the rotation solve is latency-bound and
     has no roofline."""
     if name.startswith("zgemm_bf16x3") or name.startswith("zgemm_bf16x6"):
         return "mfma", PEAK_TFLOPS["bf16x3"], "TFLOP/s"
@@ -129,7 +129,7 @@ def _kernel_bound(name):
     if (name.startswith("zgemm_kernel<double") or name.startswith("zgemm_grouped_kernel<double")
             or name == "k_jac_gram<double>"):
         return "mfma", PEAK_TFLOPS["fp64"], "TFLOP/s"
-    if name.startswith("k_jac_apply") or name.startswith("k_mix_sectors"):
+    if name.startswith(("k_jac_apply", "k_jac_gram_cross", "k_mix_sectors")):
         return "hbm", HBM_PEAK_GBS, "GB/s"
     return None, None, None
 
@@ -710,8 +710,8 @@ def main():
         "higher_is_better": False,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": f"{MIXED_DTYPE.get(args.mixed, args.mixed)} contractions, f64 Krylov/QR, "
-                 "SVD: f32 Jacobi preconditioning sweeps finished by f64 sweeps (f64 accuracy)",
+        "dtype": f"{MIXED_DTYPE.get(args.mixed, args.mixed)} contractions, "
+                 "f64 Krylov/QR/SVD",
         "data": "synthetic (seeded random MPS, XXZ MPO)",
         "config": {"workload": "two-site TDVP sweep, XXZ L=%d J=1 Delta=0.8 h=-0.1, fixed D=%d "
                                "(tapered), dt=-0.05j, numiter=%d, tol_split=1e-10"
