@@ -43,34 +43,41 @@ struct LzState {
 // indexed by problem. `rb` partial sums per reduction (rb = min(512,
 // ceil(n / 256)), a function of n only, so every sum has a fixed order).
 
-// sum of the rb partials in a fixed order; every block of a kernel computes
-// the identical value (256 threads)
-__device__ double block_sum_partials(const double* __restrict__ part, int rb) {
-  __shared__ double red[256];
-  const int t = threadIdx.x;
-  double v = 0;
-  for (int i = t; i < rb; i += 256) v += part[i];
-  red[t] = v;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) red[t] += red[t + w];
-    __syncthreads();
+// sum over the workgroup (up to 16 waves) in a fixed order, in every thread: the sums of
+// each wave's rows of 16 lanes through LDS, then lane l of a row adds those of wave l. red
+// is not written again until the caller's next barrier after it.
+// Of the first `waves` waves; the others only take part in the barrier (result 0).
+__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4], int waves) {
+  const int t = threadIdx.x, w = t & 15;
+  const bool on = t >> 6 < waves;
+  if (on) {
+    v = row_sum(v);
+    if (w == 0) red[t >> 6][(t >> 4) & 3] = v;
   }
-  double s = red[0];
-  __syncthreads();
-  return s;
+  lds_barrier();
+  if (!on) return 0.0;
+  const double s = (red[w][0] + red[w][1]) + (red[w][2] + red[w][3]);
+  return row_sum(w < waves ? s : 0.0);
+}
+__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4]) {
+  return wg_sum(v, red, (int)(blockDim.x >> 6));
 }
 
-__device__ void block_store_partial(double v, double* out) {
-  __shared__ double red[256];
-  const int t = threadIdx.x;
-  red[t] = v;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) red[t] += red[t + w];
-    __syncthreads();
-  }
-  if (t == 0) out[blockIdx.x] = red[0];
+// (the three vector kernels at n = 16384 with sums by halving in LDS 2.9 + 4.3 + 3.9 us, with
+// wg_sum 2.5 + 3.3 + 3.3)
+// sum of the rb partials in a fixed order; every block of a kernel computes the identical
+// value (256 threads)
+__device__ __forceinline__ double block_sum_partials(const double* __restrict__ part, int rb) {
+  __shared__ __align__(16) double red[16][4];
+  double v = 0;
+  for (int i = threadIdx.x; i < rb; i += 256) v += part[i];
+  return wg_sum(v, red);
+}
+
+__device__ __forceinline__ void block_store_partial(double v, double* out) {
+  __shared__ __align__(16) double red[16][4];
+  const double s = wg_sum(v, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 __device__ __forceinline__ void state_init(LzState* st, int numiter) {
@@ -222,26 +229,6 @@ __global__ __launch_bounds__(256) void k_beta_next(int64_t n, const double2* __r
 // fewer; at 16384 one CU's bandwidth would cost more (the registers spill: 45 us).
 constexpr int SHORT_T = 1024;     // largest workgroup
 constexpr int64_t SHORT_MAX = 8 * SHORT_T;
-
-// sum over the workgroup (up to 16 waves) in a fixed order, in every thread: the sums of
-// each wave's rows of 16 lanes through LDS, then lane l of a row adds those of wave l. red
-// is not written again until the caller's next barrier after it.
-// Of the first `waves` waves; the others only take part in the barrier (result 0).
-__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4], int waves) {
-  const int t = threadIdx.x, w = t & 15;
-  const bool on = t >> 6 < waves;
-  if (on) {
-    v = row_sum(v);
-    if (w == 0) red[t >> 6][(t >> 4) & 3] = v;
-  }
-  lds_barrier();
-  if (!on) return 0.0;
-  const double s = (red[w][0] + red[w][1]) + (red[w][2] + red[w][3]);
-  return row_sum(w < waves ? s : 0.0);
-}
-__device__ __forceinline__ double wg_sum(double v, double (&red)[16][4]) {
-  return wg_sum(v, red, (int)(blockDim.x >> 6));
-}
 
 // x / b from inv = 1 / b with one correction (b a normal number)
 __device__ __forceinline__ double div_by(double x, double b, double inv) {
