@@ -639,7 +639,7 @@ inline size_t v3_split_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {
   const int64_t Mp = v2_round(M, V2_BM), N2p = v2_round(2 * N, V2_BN), K2p = v3_kpad(K);
   const int sk = v2_splitk(M, N, K, batch);
   const size_t part = sk > 1 ? (size_t)sk * (size_t)Mp * (size_t)N2p * sizeof(float) + 256 : 0;
-  return (size_t)batch * (size_t)(Mp + N2p) * (size_t)K2p * V3_NT * sizeof(__bf16) + 512 + part;
+  return (size_t)batch * (size_t)(Mp + N2p / 2) * (size_t)K2p * V3_NT * sizeof(__bf16) + 512 + part;
 }
 
 __device__ __forceinline__ void split3(float x, __bf16& hi, __bf16& mid, __bf16& lo) {
@@ -673,9 +673,13 @@ __device__ __forceinline__ int64_t v3_chunk(int64_t row, int64_t kb, int term, i
   return row * (V3_NT * K2p) + kb * (V3_NT * V3_BK) + term * V3_BK + 8 * half;
 }
 
-// A (M x K complex, as k_split_a) -> interleaved hi / mid / lo terms of A_r
+// A (M x K complex, as k_split_a) -> interleaved hi / mid / lo terms of A_r;
+// B the same way, its columns as the rows: one row per complex column, not the
+// two of the real embedding, since the pass is bound by the bytes that it
+// moves, at the copy rate (20 M complex64 values of B: 74 us, 126 us with both
+// rows written)
 template <typename TA>
-__global__ __launch_bounds__(256) void k_split3_a(int64_t M, int64_t K, const TA* __restrict__ A,
+__global__ __launch_bounds__(256) void k_split3(int64_t M, int64_t K, const TA* __restrict__ A,
                                                   int64_t a_m, int64_t a_k, int conj, int64_t bz,
                                                   int64_t K2p, int64_t pz, __bf16* __restrict__ P) {
   __shared__ float2 t[64][33];
@@ -708,52 +712,29 @@ __global__ __launch_bounds__(256) void k_split3_a(int64_t M, int64_t K, const TA
   }
 }
 
-// B (K x N complex, as k_split_b) -> interleaved terms of the real embedding
-// B_e: row 2n holds (Re, -Im), row 2n + 1 holds (Im, Re) per complex k
-template <typename TB>
-__global__ __launch_bounds__(256) void k_split3_b(int64_t K, int64_t N, const TB* __restrict__ B,
-                                                  int64_t b_k, int64_t b_n, int conj, int64_t bz,
-                                                  int64_t K2p, int64_t pz, __bf16* __restrict__ P) {
-  __shared__ float2 t[64][33];
-  const int64_t n0 = (int64_t)blockIdx.y * 64, k0 = (int64_t)blockIdx.x * 32;
-  B += blockIdx.z * bz;
-  P += blockIdx.z * pz;
-  const bool kc = (b_k == 1) || (b_n != 1);
-  for (int e = threadIdx.x; e < 64 * 32; e += 256) {
-    const int r = kc ? e / 32 : e % 64, c = kc ? e % 32 : e / 64;
-    const int64_t n = n0 + r, k = k0 + c;
-    float re = 0.f, im = 0.f;
-    if (n < N && k < K) load_c<float>(B + k * b_k + n * b_n, re, im);
-    t[r][c] = make_float2(re, conj ? -im : im);
-  }
-  __syncthreads();
-  // real rows 2 n (Re, -Im per complex k) and 2 n + 1 (Im, Re)
-  for (int q = threadIdx.x; q < 128 * V3_CHUNKS; q += 256) {
-    const int rr = q / V3_CHUNKS, w = q % V3_CHUNKS;
-    const int kb = w / (2 * V3_NT), term = (w % (2 * V3_NT)) >> 1, half = w & 1;
-    const int64_t kbg = 2 * k0 / V3_BK + kb;
-    if (kbg * V3_BK >= K2p) continue;
-    const int r = rr >> 1;
-    const bool odd = rr & 1;
-    float x[8];
+// 256 x 256 real tiles, 8 waves (2 x 4) of 128 x 64 as in zgemm_bf16x3_v2,
+// 16-deep k-stages double buffered in LDS (term planes of 256 rows of A and
+// 128 of B x 24 bf16 per stage = 54 KiB; the 48-byte row pitch keeps the
+// 16-byte fragment reads of 16 consecutive rows on distinct banks). The operand
+// pointers of V2Args are used as: ahi = A terms, bhi = B terms (alo, blo
+// unused). The real embedding of B, (Re, -Im) in the even and (Im, Re) in the
+// odd real columns, is formed from the fragments (v3_embed): two vector
+// instructions per register, in the shadow of the 48 MFMAs of a stage, for half
+// the bytes of B from memory and into LDS. The stream of operands and the power
+// that it takes, not the MFMA issue rate, bound the kernel: the two products of
+// a two-site H_eff at D = 1024 (M = 5, d = 4) take 1007 and 880 us, with both
+// rows of a column streamed 1097 and 926.
+__device__ __forceinline__ bf16x8_t v3_embed(const __bf16* p, unsigned sel, unsigned sign) {
+  u32x4_t w = *(const u32x4_t*)p;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float2 v = t[r][8 * kb + 4 * half + j];
-      x[2 * j] = odd ? v.y : v.x;
-      x[2 * j + 1] = odd ? v.x : -v.y;
-    }
-    *(bf16x8_t*)(P + v3_chunk(2 * n0 + rr, kbg, term, half, K2p)) = term8(x, term);
-  }
+  for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_perm(w[e], w[e], sel) ^ sign;
+  return __builtin_bit_cast(bf16x8_t, w);
 }
 
-// 256 x 256 real tiles, 8 waves (2 x 4) of 128 x 64 as in zgemm_bf16x3_v2,
-// 16-deep k-stages double buffered in LDS (6 term planes x 256 rows x 24 bf16
-// per stage = 72 KiB; the 48-byte row pitch keeps the 16-byte fragment reads
-// of 16 consecutive rows on distinct banks). The operand pointers of V2Args
-// are used as: ahi = A terms, bhi = B terms (alo, blo unused).
 template <typename TC>
 __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
-  __shared__ __align__(16) __bf16 sm[2][2 * V3_NT][V2_BM][V3_LD];
+  __shared__ __align__(16) __bf16 sma[2][V3_NT][V2_BM][V3_LD];
+  __shared__ __align__(16) __bf16 smb[2][V3_NT][V2_BN / 2][V3_LD];
   if (g.skip && g.skip[(g.part ? 0 : blockIdx.z) * g.skip_stride]) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 2, wn = wave & 3;
@@ -764,17 +745,18 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
   const int64_t kbeg = g.part ? (int64_t)blockIdx.z * g.kchunk : 0;
   const int64_t pitch = V3_NT * g.K2p;   // bf16 per row
   const __bf16* srcA = g.ahi + z * g.pza + m0 * pitch + V3_NT * kbeg;
-  const __bf16* srcB = g.bhi + z * g.pzb + c0 * pitch + V3_NT * kbeg;
-  // global -> register staging: per operand and stage 256 rows x 96 bytes =
-  // 1536 chunks of 16 bytes, three per thread (six consecutive threads per row)
-  u32x4_t pa[3], pb[3];
+  const __bf16* srcB = g.bhi + z * g.pzb + (c0 >> 1) * pitch + V3_NT * kbeg;
+  // global -> register staging: per stage 256 rows of A and 128 of B x 96
+  // bytes = 1536 and 768 chunks of 16 bytes (six consecutive threads per row):
+  // three of A per thread, and of B one more in the first four waves
+  u32x4_t pa[3], pb[2];
   auto gload = [&](int64_t k0) {
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       const int c = tid + 512 * u, row = c / 6, part = c % 6;
       const int64_t o = (int64_t)row * pitch + V3_NT * k0 + 8 * part;
       pa[u] = *(const u32x4_t*)(srcA + o);
-      pb[u] = *(const u32x4_t*)(srcB + o);
+      if (u == 0 || (u == 1 && tid < 256)) pb[u] = *(const u32x4_t*)(srcB + o);
     }
   };
   auto lstore = [&](int buf) {
@@ -782,8 +764,8 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
     for (int u = 0; u < 3; ++u) {
       const int c = tid + 512 * u, row = c / 6, part = c % 6;
       const int term = part >> 1, half = 8 * (part & 1);
-      *(u32x4_t*)&sm[buf][term][row][half] = pa[u];
-      *(u32x4_t*)&sm[buf][V3_NT + term][row][half] = pb[u];
+      *(u32x4_t*)&sma[buf][term][row][half] = pa[u];
+      if (u == 0 || (u == 1 && tid < 256)) *(u32x4_t*)&smb[buf][term][row][half] = pb[u];
     }
   };
   f16v_t acc[4][2];
@@ -796,6 +778,8 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
   const int64_t klen = g.part ? (g.K2p - kbeg < g.kchunk ? g.K2p - kbeg : g.kchunk) : g.K2p;
   const int nst = (int)(klen / V3_BK);
   const int r32 = lane & 31, kg = 8 * (lane >> 5);
+  const unsigned sel = lane & 1 ? 0x01000302u : 0x03020100u;   // odd: (Im, Re)
+  const unsigned sign = lane & 1 ? 0u : 0x80000000u;           // even: (Re, -Im)
   gload(0);
   lstore(0);
   __syncthreads();
@@ -807,16 +791,16 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 128 * wm + 32 * i + r32;
-      ah[i] = *(const bf16x8_t*)&sm[buf][0][row][kg];
-      am[i] = *(const bf16x8_t*)&sm[buf][1][row][kg];
-      al[i] = *(const bf16x8_t*)&sm[buf][2][row][kg];
+      ah[i] = *(const bf16x8_t*)&sma[buf][0][row][kg];
+      am[i] = *(const bf16x8_t*)&sma[buf][1][row][kg];
+      al[i] = *(const bf16x8_t*)&sma[buf][2][row][kg];
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int col = 64 * wn + 32 * j + r32;
-      bh[j] = *(const bf16x8_t*)&sm[buf][V3_NT][col][kg];
-      bm[j] = *(const bf16x8_t*)&sm[buf][V3_NT + 1][col][kg];
-      bl[j] = *(const bf16x8_t*)&sm[buf][V3_NT + 2][col][kg];
+      const int col = 32 * wn + 16 * j + (r32 >> 1);
+      bh[j] = v3_embed(&smb[buf][0][col][kg], sel, sign);
+      bm[j] = v3_embed(&smb[buf][1][col][kg], sel, sign);
+      bl[j] = v3_embed(&smb[buf][2][col][kg], sel, sign);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -877,16 +861,16 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
 template <typename TA, typename TB, typename TC>
 inline int launch_bf16_v3(const ZGemm& z, hipStream_t s) {
   const int64_t Mp = v2_round(z.M, V2_BM), N2p = v2_round(2 * z.N, V2_BN), K2p = v3_kpad(z.K);
-  const int64_t pza = Mp * K2p * V3_NT, pzb = N2p * K2p * V3_NT;
+  const int64_t pza = Mp * K2p * V3_NT, pzb = N2p / 2 * K2p * V3_NT;
   char* base = (char*)(((uintptr_t)z.sws + 255) & ~(uintptr_t)255);
   __bf16* pa = (__bf16*)base;
   __bf16* pb = pa + z.batch * pza;
   const unsigned bt = (unsigned)z.batch;
   const unsigned kblk = (unsigned)((K2p + 63) / 64);   // 32 complex k per block
-  k_split3_a<TA><<<dim3(kblk, (unsigned)(Mp / 64), bt), 256, 0, s>>>(
+  k_split3<TA><<<dim3(kblk, (unsigned)(Mp / 64), bt), 256, 0, s>>>(
       z.M, z.K, (const TA*)z.A, z.a_m, z.a_k, z.conjA, z.bz_a, K2p, pza, pa);
-  k_split3_b<TB><<<dim3(kblk, (unsigned)(N2p / 128), bt), 256, 0, s>>>(
-      z.K, z.N, (const TB*)z.B, z.b_k, z.b_n, z.conjB, z.bz_b, K2p, pzb, pb);
+  k_split3<TB><<<dim3(kblk, (unsigned)(N2p / 128), bt), 256, 0, s>>>(
+      z.N, z.K, (const TB*)z.B, z.b_n, z.b_k, z.conjB, z.bz_b, K2p, pzb, pb);
   PTN_LAUNCH_CHECK();
   const int sk = v2_splitk(z.M, z.N, z.K, z.batch);
   V2Args g;
