@@ -631,7 +631,8 @@ size_t bf16x3_split_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {
 // ([row][k / 16][term][k % 16]), so that one k-stage of a row is one
 // contiguous 96-byte read. Products too small for the pre-split kernel run on
 // the FP32 MFMA (the same accuracy).
-constexpr int V3_BK = 16, V3_LD = 24, V3_NT = 3;
+constexpr int V3_BK = 16, V3_NT = 3;
+constexpr int V3_SA = V2_BM * V3_NT * V3_BK, V3_SB = V3_SA / 2;   // a stage of A and of B in LDS
 
 inline int64_t v3_kpad(int64_t K) { return v2_round(2 * K, V3_BK); }
 
@@ -712,18 +713,24 @@ __global__ __launch_bounds__(256) void k_split3(int64_t M, int64_t K, const TA* 
   }
 }
 
-// 256 x 256 real tiles, 8 waves (2 x 4) of 128 x 64 as in zgemm_bf16x3_v2,
-// 16-deep k-stages double buffered in LDS (term planes of 256 rows of A and
-// 128 of B x 24 bf16 per stage = 54 KiB; the 48-byte row pitch keeps the
-// 16-byte fragment reads of 16 consecutive rows on distinct banks). The operand
-// pointers of V2Args are used as: ahi = A terms, bhi = B terms (alo, blo
-// unused). The real embedding of B, (Re, -Im) in the even and (Im, Re) in the
-// odd real columns, is formed from the fragments (v3_embed): two vector
-// instructions per register, in the shadow of the 48 MFMAs of a stage, for half
-// the bytes of B from memory and into LDS. The stream of operands and the power
-// that it takes, not the MFMA issue rate, bound the kernel: the two products of
-// a two-site H_eff at D = 1024 (M = 5, d = 4) take 1007 and 880 us, with both
-// rows of a column streamed 1097 and 926.
+// 256 x 256 real tiles, 8 waves (2 x 4) of 128 x 64 as in zgemm_bf16x3_v2. The
+// 16-deep k-stages (256 rows of A and 128 of B, 96 bytes each: 36 KiB) are
+// loaded straight into LDS, three deep, with one barrier per stage: no
+// registers and no LDS stores between memory and the fragments. A wave's load
+// fills 1 KiB of LDS in lane order, so rows cannot be padded; the two 16-byte
+// halves of a term are exchanged in every second group of eight rows instead,
+// which puts the fragment reads of 16 consecutive rows on distinct banks. One
+// array per stage and operand: the compiler then knows that a read does not
+// wait for the loads in flight to the others. The operand pointers of V2Args
+// are used as: ahi = A terms, bhi = B terms (alo, blo unused). The real
+// embedding of B, (Re, -Im) in the even and (Im, Re) in the odd real columns,
+// is formed from the fragments (v3_embed): two vector instructions per
+// register, in the shadow of the 48 MFMAs of a stage, for half the bytes of B
+// from memory and into LDS. The stream of operands and the power that it takes,
+// not the MFMA issue rate, bound the kernel: the two products of a two-site
+// H_eff at D = 1024 (M = 5, d = 4) take 975 and 839 us; 1007 and 880 with the
+// stages staged through registers, 1097 and 926 with both rows of a column
+// streamed as well.
 __device__ __forceinline__ bf16x8_t v3_embed(const __bf16* p, unsigned sel, unsigned sign) {
   u32x4_t w = *(const u32x4_t*)p;
 #pragma unroll
@@ -733,10 +740,11 @@ __device__ __forceinline__ bf16x8_t v3_embed(const __bf16* p, unsigned sel, unsi
 
 template <typename TC>
 __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
-  __shared__ __align__(16) __bf16 sma[2][V3_NT][V2_BM][V3_LD];
-  __shared__ __align__(16) __bf16 smb[2][V3_NT][V2_BN / 2][V3_LD];
+  __shared__ __align__(16) __bf16 A0[V3_SA], A1[V3_SA], A2[V3_SA];
+  __shared__ __align__(16) __bf16 B0[V3_SB], B1[V3_SB], B2[V3_SB];
   if (g.skip && g.skip[(g.part ? 0 : blockIdx.z) * g.skip_stride]) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
   int tm, tn;
   tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
@@ -746,27 +754,31 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
   const int64_t pitch = V3_NT * g.K2p;   // bf16 per row
   const __bf16* srcA = g.ahi + z * g.pza + m0 * pitch + V3_NT * kbeg;
   const __bf16* srcB = g.bhi + z * g.pzb + (c0 >> 1) * pitch + V3_NT * kbeg;
-  // global -> register staging: per stage 256 rows of A and 128 of B x 96
-  // bytes = 1536 and 768 chunks of 16 bytes (six consecutive threads per row):
-  // three of A per thread, and of B one more in the first four waves
-  u32x4_t pa[3], pb[2];
-  auto gload = [&](int64_t k0) {
+  // A stage is 1536 chunks of 16 bytes of A and 768 of B, six to a row; a wave
+  // loads 64 at a time into consecutive chunks of LDS: 24 of A, three to a
+  // wave, and 12 of B, two to the first four waves and one to the others
+  const bool two = wave < 4;
+  int64_t off[3];
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      const int c = tid + 512 * u, row = c / 6, part = c % 6;
-      const int64_t o = (int64_t)row * pitch + V3_NT * k0 + 8 * part;
-      pa[u] = *(const u32x4_t*)(srcA + o);
-      if (u == 0 || (u == 1 && tid < 256)) pb[u] = *(const u32x4_t*)(srcB + o);
-    }
-  };
-  auto lstore = [&](int buf) {
+  for (int u = 0; u < 3; ++u) {
+    const int c = 64 * (wave + 8 * u) + lane, row = c / 6, part = c % 6;
+    off[u] = (int64_t)row * pitch + 8 * (part ^ ((row >> 3) & 1));
+  }
+  const int64_t klen = g.part ? (g.K2p - kbeg < g.kchunk ? g.K2p - kbeg : g.kchunk) : g.K2p;
+  const int nst = (int)(klen / V3_BK);
+  typedef const __attribute__((address_space(1))) void* gp_t;
+  typedef __attribute__((address_space(3))) void* lp_t;
+  auto dma = [&](__bf16 (&As)[V3_SA], __bf16 (&Bs)[V3_SB], int st) {
+    // beyond the end: the last stage again, not used
+    const int64_t o = (int64_t)(V3_NT * V3_BK) * (st < nst ? st : nst - 1);
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      const int c = tid + 512 * u, row = c / 6, part = c % 6;
-      const int term = part >> 1, half = 8 * (part & 1);
-      *(u32x4_t*)&sma[buf][term][row][half] = pa[u];
-      if (u == 0 || (u == 1 && tid < 256)) *(u32x4_t*)&smb[buf][term][row][half] = pb[u];
-    }
+    for (int u = 0; u < 3; ++u)
+      __builtin_amdgcn_global_load_lds((gp_t)(srcA + o + off[u]),
+                                       (lp_t)&As[512 * (wave + 8 * u)], 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((gp_t)(srcB + o + off[0]), (lp_t)&Bs[512 * wave], 16, 0, 0);
+    if (two)
+      __builtin_amdgcn_global_load_lds((gp_t)(srcB + o + off[1]), (lp_t)&Bs[512 * (wave + 8)], 16,
+                                       0, 0);
   };
   f16v_t acc[4][2];
 #pragma unroll
@@ -775,32 +787,34 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  const int64_t klen = g.part ? (g.K2p - kbeg < g.kchunk ? g.K2p - kbeg : g.kchunk) : g.K2p;
-  const int nst = (int)(klen / V3_BK);
-  const int r32 = lane & 31, kg = 8 * (lane >> 5);
+  const int r32 = lane & 31, half = lane >> 5;
   const unsigned sel = lane & 1 ? 0x01000302u : 0x03020100u;   // odd: (Im, Re)
   const unsigned sign = lane & 1 ? 0u : 0x80000000u;           // even: (Re, -Im)
-  gload(0);
-  lstore(0);
-  __syncthreads();
-  for (int st = 0; st < nst; ++st) {
-    const int buf = st & 1;
-    const bool more = st + 1 < nst;
-    if (more) gload((int64_t)(st + 1) * V3_BK);
+  // fragment of row / column r: term t at + 16 t
+  const int ra = 128 * wm + r32, rb = 32 * wn + (r32 >> 1);
+  const int fa = 48 * ra + 8 * (half ^ ((ra >> 3) & 1));
+  const int fb = 48 * rb + 8 * (half ^ ((rb >> 3) & 1));
+  auto step = [&](const __bf16 (&As)[V3_SA], const __bf16 (&Bs)[V3_SB], __bf16 (&An)[V3_SA],
+                  __bf16 (&Bn)[V3_SB], int st) {
+    // stage st has landed, and every wave has read stage st - 1
+    if (two) wait_vm<5, true>();
+    else wait_vm<4, true>();
+    wg_barrier();
+    dma(An, Bn, st + 2);
     bf16x8_t ah[4], am[4], al[4], bh[2], bm[2], bl[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 128 * wm + 32 * i + r32;
-      ah[i] = *(const bf16x8_t*)&sma[buf][0][row][kg];
-      am[i] = *(const bf16x8_t*)&sma[buf][1][row][kg];
-      al[i] = *(const bf16x8_t*)&sma[buf][2][row][kg];
+    for (int j = 0; j < 2; ++j) {
+      const __bf16* p = &Bs[fb + 48 * 16 * j];
+      bh[j] = v3_embed(p, sel, sign);
+      bm[j] = v3_embed(p + 16, sel, sign);
+      bl[j] = v3_embed(p + 32, sel, sign);
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = 32 * wn + 16 * j + (r32 >> 1);
-      bh[j] = v3_embed(&smb[buf][0][col][kg], sel, sign);
-      bm[j] = v3_embed(&smb[buf][1][col][kg], sel, sign);
-      bl[j] = v3_embed(&smb[buf][2][col][kg], sel, sign);
+    for (int i = 0; i < 4; ++i) {
+      const __bf16* p = &As[fa + 48 * 32 * i];
+      ah[i] = *(const bf16x8_t*)p;
+      am[i] = *(const bf16x8_t*)(p + 16);
+      al[i] = *(const bf16x8_t*)(p + 32);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -813,9 +827,15 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bm[j], acc[i][j], 0, 0, 0);
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
       }
-    if (more) lstore(buf ^ 1);
-    __syncthreads();
+  };
+  dma(A0, B0, 0);
+  dma(A1, B1, 1);
+  for (int st = 0; st < nst; st += 3) {
+    step(A0, B0, A2, B2, st);
+    if (st + 1 < nst) step(A1, B1, A0, B0, st + 1);
+    if (st + 2 < nst) step(A2, B2, A1, B1, st + 2);
   }
+  wait_vm<0>();   // no load may land in LDS from here on
   // epilogue of zgemm_bf16x3_v2 (the same accumulator layout)
   if (g.part) {
     float* P = g.part + (int64_t)blockIdx.z * (int64_t)g.tiles_m * V2_BM * g.N2p;
