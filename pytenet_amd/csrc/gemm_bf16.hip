@@ -715,7 +715,7 @@ __global__ __launch_bounds__(256) void k_split3(int64_t M, int64_t K, const TA* 
 
 // 256 x 256 real tiles, 8 waves (2 x 4) of 128 x 64 as in zgemm_bf16x3_v2. The
 // 16-deep k-stages (256 rows of A and 128 of B, 96 bytes each: 36 KiB) are
-// loaded straight into LDS, three deep, with one barrier per stage: no
+// loaded straight into LDS, four buffers deep, with one barrier per stage: no
 // registers and no LDS stores between memory and the fragments. A wave's load
 // fills 1 KiB of LDS in lane order, so rows cannot be padded; the two 16-byte
 // halves of a term are exchanged in every second group of eight rows instead,
@@ -728,9 +728,10 @@ __global__ __launch_bounds__(256) void k_split3(int64_t M, int64_t K, const TA* 
 // register, in the shadow of the 48 MFMAs of a stage, for half the bytes of B
 // from memory and into LDS. The stream of operands and the power that it takes,
 // not the MFMA issue rate, bound the kernel: the two products of a two-site
-// H_eff at D = 1024 (M = 5, d = 4) take 975 and 839 us; 1007 and 880 with the
-// stages staged through registers, 1097 and 926 with both rows of a column
-// streamed as well.
+// H_eff at D = 1024 take 952 and 812 us; 975 and 839 with three buffers, 1007
+// and 880 with the stages staged through registers, 1097 and 926 with both
+// rows of a column streamed as well. Fragments of the next stage read between
+// the MFMAs of this one were slower (H_eff 1846 us against 1815).
 __device__ __forceinline__ bf16x8_t v3_embed(const __bf16* p, unsigned sel, unsigned sign) {
   u32x4_t w = *(const u32x4_t*)p;
 #pragma unroll
@@ -740,8 +741,8 @@ __device__ __forceinline__ bf16x8_t v3_embed(const __bf16* p, unsigned sel, unsi
 
 template <typename TC>
 __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
-  __shared__ __align__(16) __bf16 A0[V3_SA], A1[V3_SA], A2[V3_SA];
-  __shared__ __align__(16) __bf16 B0[V3_SB], B1[V3_SB], B2[V3_SB];
+  __shared__ __align__(16) __bf16 A0[V3_SA], A1[V3_SA], A2[V3_SA], A3[V3_SA];
+  __shared__ __align__(16) __bf16 B0[V3_SB], B1[V3_SB], B2[V3_SB], B3[V3_SB];
   if (g.skip && g.skip[(g.part ? 0 : blockIdx.z) * g.skip_stride]) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -797,10 +798,10 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
   auto step = [&](const __bf16 (&As)[V3_SA], const __bf16 (&Bs)[V3_SB], __bf16 (&An)[V3_SA],
                   __bf16 (&Bn)[V3_SB], int st) {
     // stage st has landed, and every wave has read stage st - 1
-    if (two) wait_vm<5, true>();
-    else wait_vm<4, true>();
+    if (two) wait_vm<10, true>();
+    else wait_vm<8, true>();
     wg_barrier();
-    dma(An, Bn, st + 2);
+    dma(An, Bn, st + 3);
     bf16x8_t ah[4], am[4], al[4], bh[2], bm[2], bl[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -830,10 +831,12 @@ __global__ __launch_bounds__(512) void zgemm_bf16x6_v3(V2Args g) {
   };
   dma(A0, B0, 0);
   dma(A1, B1, 1);
-  for (int st = 0; st < nst; st += 3) {
-    step(A0, B0, A2, B2, st);
+  dma(A2, B2, 2);
+  for (int st = 0; st < nst; st += 4) {
+    step(A0, B0, A3, B3, st);
     if (st + 1 < nst) step(A1, B1, A0, B0, st + 1);
     if (st + 2 < nst) step(A2, B2, A1, B1, st + 2);
+    if (st + 3 < nst) step(A3, B3, A2, B2, st + 3);
   }
   wait_vm<0>();   // no load may land in LDS from here on
   // epilogue of zgemm_bf16x3_v2 (the same accumulator layout)
