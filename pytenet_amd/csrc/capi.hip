@@ -110,10 +110,32 @@ const char* ptn_last_hip_error(void) { return hipGetErrorString(g_last_hip); }
 
 // In the FP32 and split-bf16 modes the environment blocks are converted to
 // complex64 once per call (one pass), as the Krylov solver does once per
-// local solve: the products then stream half the operand bytes.
+// local solve: the products then stream half the operand bytes (once_operand:
+// except where a product reads the block only once).
 static inline bool lowp(int p) { return (p & ~PTN_BLOCK_SPARSE) != PTN_FP64; }
 static inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 static inline size_t env64_bytes(int64_t D, int64_t M) { return al256((size_t)(D * M * D) * 8); }
+
+// An environment operand (n values) of an M x N x K product that is computed once
+// with it, as that product reads it best. Most kernels of the low-precision modes
+// read an element once per tile: complex64, converted into `buf`. The three-term
+// pre-split product reads it once, in its split pass, which rounds the same way:
+// as it is. At 5.2 M values the conversion takes 23 us and the split 29 us from
+// complex64; two-site H_eff at D = 1024 (both operands) 1812 -> 1780 us.
+// Not for the local solves, whose products read the operand in every iteration.
+static int once_operand(int precision, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t n,
+                        char* buf, const void** x, int* tx, hipStream_t s) {
+  *tx = PTN_T_C128;
+  if (!lowp(precision)) return PTN_OK;
+  // (the block-sparse flag asks for tile masks, which batches do not have)
+  const bool masked = (precision & PTN_BLOCK_SPARSE) && batch == 1;
+  if ((precision & ~PTN_BLOCK_SPARSE) == PTN_BF16X6 && !masked && bf16x6_presplits(M, N, K, batch))
+    return PTN_OK;
+  const int st = convert_c128_c64(n, *x, buf, s);
+  *x = buf;
+  *tx = PTN_T_C64;
+  return st;
+}
 
 size_t ptn_heff_workspace(int precision, int64_t Dl, int64_t d, int64_t Dr, int64_t Ml,
                           int64_t Mr) {
@@ -132,16 +154,14 @@ int ptn_heff_apply(int precision, int64_t Dl, int64_t d, int64_t Dr, int64_t Ml,
   if (ws_bytes < ptn_heff_workspace(precision, Dl, d, Dr, Ml, Mr)) return PTN_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   const size_t base = al256(heff_ws_bytes(precision, D));
-  if (!lowp(precision))
-    return heff_apply(precision, D, l, PTN_T_C128, w, r, PTN_T_C128, a, PTN_T_C128, out,
-                      PTN_T_C128, ws, base, s);
   char* l64 = (char*)ws + base;
   char* r64 = l64 + env64_bytes(Dl, Ml);
-  int st;
-  if ((st = convert_c128_c64(Dl * Ml * Dl, l, l64, s))) return st;
-  if ((st = convert_c128_c64(Dr * Mr * Dr, r, r64, s))) return st;
-  return heff_apply(precision, D, l64, PTN_T_C64, w, r64, PTN_T_C64, a, PTN_T_C128, out,
-                    PTN_T_C128, ws, base, s);
+  int st, tl, tr;
+  if ((st = once_operand(precision, Dl, d * Dr, Dl * Ml, 1, Dl * Ml * Dl, l64, &l, &tl, s)))
+    return st;
+  if ((st = once_operand(precision, Dl * d, Mr * Dr, Dr, 1, Dr * Mr * Dr, r64, &r, &tr, s)))
+    return st;
+  return heff_apply(precision, D, l, tl, w, r, tr, a, PTN_T_C128, out, PTN_T_C128, ws, base, s);
 }
 
 size_t ptn_bond_workspace(int precision, int64_t Dl, int64_t Dr, int64_t M) {
@@ -157,16 +177,13 @@ int ptn_bond_apply(int precision, int64_t Dl, int64_t Dr, int64_t M, const void*
   if (ws_bytes < ptn_bond_workspace(precision, Dl, Dr, M)) return PTN_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   const size_t base = al256(bond_ws_bytes(precision, Dl, Dr, M));
-  if (!lowp(precision))
-    return bond_apply(precision, Dl, Dr, M, l, PTN_T_C128, r, PTN_T_C128, c, PTN_T_C128, out,
-                      PTN_T_C128, ws, base, s);
   char* l64 = (char*)ws + base;
   char* r64 = l64 + env64_bytes(Dl, M);
-  int st;
-  if ((st = convert_c128_c64(Dl * M * Dl, l, l64, s))) return st;
-  if ((st = convert_c128_c64(Dr * M * Dr, r, r64, s))) return st;
-  return bond_apply(precision, Dl, Dr, M, l64, PTN_T_C64, r64, PTN_T_C64, c, PTN_T_C128, out,
-                    PTN_T_C128, ws, base, s);
+  int st, tl, tr;
+  if ((st = once_operand(precision, Dl, Dr, Dl * M, 1, Dl * M * Dl, l64, &l, &tl, s))) return st;
+  if ((st = once_operand(precision, Dl, M * Dr, Dr, 1, Dr * M * Dr, r64, &r, &tr, s))) return st;
+  return bond_apply(precision, Dl, Dr, M, l, tl, r, tr, c, PTN_T_C128, out, PTN_T_C128, ws, base,
+                    s);
 }
 
 int ptn_local_apply(const ptn_local_op* op, const void* a, void* out, int32_t* grouped, void* ws,
@@ -231,15 +248,15 @@ static int env_step_b(int left, int precision, int64_t batch, int64_t Dl, int64_
   if (ws_bytes < env_workspace_b(precision, batch, Dl, d, Dr, Ml, Mr)) return PTN_ERR_WORKSPACE;
   const size_t base = al256(env_ws_bytes(precision, D, batch));
   const void* e = blk;
-  int te = PTN_T_C128, st;
-  if (lowp(precision)) {
-    // the environment block stack in complex64, converted once (contiguous)
-    char* e64 = (char*)ws + base;
-    const int64_t ne = left ? Dl * Ml * Dl : Dr * Mr * Dr;
-    if ((st = convert_c128_c64(batch * ne, blk, e64, s))) return st;
-    e = e64;
-    te = PTN_T_C64;
-  }
+  char* e64 = (char*)ws + base;
+  int te;
+  // the block stack of a batch is contiguous
+  const int st =
+      left ? once_operand(precision, Dl * Ml, d * Dr, Dl, batch, batch * Dl * Ml * Dl, e64, &e,
+                          &te, s)
+           : once_operand(precision, Dl * d, Mr * Dr, Dr, batch, batch * Dr * Mr * Dr, e64, &e,
+                          &te, s);
+  if (st) return st;
   if (left) return env_left(precision, D, a, b, w, e, te, out, ws, base, s, batch);
   return env_right(precision, D, a, b, w, e, te, out, ws, base, s, batch);
 }

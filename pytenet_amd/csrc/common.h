@@ -118,6 +118,8 @@ struct ZGemm {
 size_t bf16x3_split_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
 // the same for the three-term split (PTN_BF16X6)
 size_t bf16x6_split_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
+// whether a product with that scratch and without tile masks takes the pre-split kernel
+bool bf16x6_presplits(int64_t M, int64_t N, int64_t K, int64_t batch);
 
 // element type codes for the GEMM / mix operands
 enum { PTN_T_C128 = 0, PTN_T_C64 = 1 };

@@ -922,11 +922,14 @@ inline int launch_bf16_v3(const ZGemm& z, hipStream_t s) {
   return PTN_OK;
 }
 
+bool bf16x6_presplits(int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const int64_t tiles = ((M + V2_BM - 1) / V2_BM) * ((2 * N + V2_BN - 1) / V2_BN) * batch;
+  return tiles * v2_splitk(M, N, K, batch) >= 128 && K >= 16 && batch <= 65535;
+}
+
 inline bool use_bf16_v3(const ZGemm& z, void* mws) {
-  if (mws || !z.sws) return false;
-  const int64_t tiles = ((z.M + V2_BM - 1) / V2_BM) * ((2 * z.N + V2_BN - 1) / V2_BN) * z.batch;
-  if (tiles * v2_splitk(z.M, z.N, z.K, z.batch) < 128 || z.K < 16 || z.batch > 65535) return false;
-  return z.sws_bytes >= v3_split_bytes(z.M, z.N, z.K, z.batch);
+  return !mws && z.sws && bf16x6_presplits(z.M, z.N, z.K, z.batch) &&
+         z.sws_bytes >= v3_split_bytes(z.M, z.N, z.K, z.batch);
 }
 
 size_t bf16x6_split_bytes(int64_t M, int64_t N, int64_t K, int64_t batch) {
