@@ -113,6 +113,7 @@ struct ZGemm {
   // (bf16x3_split_bytes); without it the split happens in the product kernel
   void* sws = nullptr;
   size_t sws_bytes = 0;
+  bool b_terms = false;   // the three-term pre-split: B's terms are there already
 };
 // scratch bytes of the pre-split split-bf16 product of an M x N x K (batched) product
 size_t bf16x3_split_bytes(int64_t M, int64_t N, int64_t K, int64_t batch);
@@ -134,5 +135,12 @@ int zgemm(const ZGemm& g, int compute, int ta, int tb, int tc,
 int mode_mix(int64_t nl, int64_t ni, int64_t no, int64_t nr, const void* wm, const void* x, int tx,
              void* y, int ty, hipStream_t s, int64_t batch = 1, int64_t bw = 0,
              bool wtrans = false);
+
+// The mix of complex64 values into the B operand of the three-term product z (row
+// l kp + m, column s nr + r of the outputs (m, s)), straight into its terms; *done = false:
+// z does not take the pre-split kernel, or the mix does not fit
+int mode_mix_split3(ZGemm& z, int64_t nl, int64_t ni, int64_t no, int64_t kp, int64_t nr,
+                    const void* wm, int64_t bw, bool wtrans, const void* x, void* mws,
+                    hipStream_t s, bool* done);
 
 }  // namespace ptn

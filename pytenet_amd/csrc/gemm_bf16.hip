@@ -713,6 +713,128 @@ __global__ __launch_bounds__(256) void k_split3(int64_t M, int64_t K, const TA* 
   }
 }
 
+// Mode mix (mix.hip) of complex64 values whose result is the B operand of a pre-split
+// product, written as its terms: Y[l, (m, s), r] is row k = l kp + m and column s nr + r of B.
+// Both passes are bound by the bytes that they move, and the mixed values need not go
+// through memory between them. A workgroup takes units of 8 l x 16 r: 128-byte runs of the
+// input, and kp whole k-blocks of 16 real k per column, a run of 96 kp bytes of the terms.
+// Sums as in mode_mix_kernel. The columns beyond N that fill up the last tile are not
+// written: they reach no output. Two-site H_eff at D = 1024 (20 x 20): mix and split
+// 59 + 77 -> 128 us, H_eff 1768 -> 1755 us; the splits' arithmetic and two workgroups' worth of
+// phases per CU keep it below the copy rate (3.3 TB/s).
+constexpr int MS_L = 8, MS_R = 16, MS_C = MS_L * MS_R, MS_MAX = 32;
+
+__global__ __launch_bounds__(256) void k_mix_split3(
+    int64_t nl, int ni, int no, int kp, int64_t nr, int nunits, const double2* __restrict__ wm,
+    int wtrans, const float2* __restrict__ x, int64_t bw, int64_t K2p, int64_t pz,
+    __bf16* __restrict__ P, const int* __restrict__ skip, int64_t skip_stride) {
+  extern __shared__ __align__(16) float2 ms_lds[];
+  __shared__ unsigned int nz[MS_MAX];
+  if (skip && skip[blockIdx.y * skip_stride]) return;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int ns = no / kp, ys = MS_L * kp + 1;   // columns per r; row of Y in LDS
+  float2* X = ms_lds;                           // [ni][MS_C]
+  float2* Y = X + ni * MS_C;                    // [ns * MS_R][ys]
+  float2* W = Y + ns * MS_R * ys;               // [no][ni]
+  wm += blockIdx.y * bw;
+  x += blockIdx.y * (nl * ni * nr);
+  P += blockIdx.y * pz;
+  const int chunks = (int)((nr + MS_R - 1) / MS_R);
+  float2 pre[MS_MAX / 2];
+  auto load = [&](int u) {
+    const int row = u / chunks, c = t & (MS_C - 1);
+    const int64_t l = (int64_t)row * MS_L + c / MS_R;
+    const int64_t r = (int64_t)(u - row * chunks) * MS_R + c % MS_R;
+    const bool in = l < nl && r < nr;
+#pragma unroll
+    for (int k = 0; k < MS_MAX / 2; ++k) {
+      const int i = (t >> 7) + 2 * k;
+      pre[k] = make_float2(0.f, 0.f);
+      if (in && i < ni) pre[k] = x[(l * ni + i) * nr + r];
+    }
+  };
+  int u = blockIdx.x;
+  load(u);
+  if (t < no) nz[t] = 0;
+  __syncthreads();
+  for (int e = t; e < ni * no; e += 256) {
+    const int o = e / ni, i = e - o * ni;
+    const double2 w = wm[wtrans ? i * no + o : e];
+    W[e] = make_float2((float)w.x, (float)w.y);
+    if (w.x != 0.0 || w.y != 0.0) atomicOr(&nz[o], 1u << i);
+  }
+  const int run = kp * V3_NT * 2;               // 16-byte chunks of a column's run
+  for (; u < nunits; u += gridDim.x) {
+    __syncthreads();   // the previous unit has been mixed and written
+#pragma unroll
+    for (int k = 0; k < MS_MAX / 2; ++k) {
+      const int i = (t >> 7) + 2 * k;
+      if (i < ni) X[i * MS_C + (t & (MS_C - 1))] = pre[k];
+    }
+    __syncthreads();
+    if (u + gridDim.x < nunits) load(u + gridDim.x);
+    const int row = u / chunks;
+    const int64_t r0 = (int64_t)(u - row * chunks) * MS_R;
+    const int c = 64 * (wave & 1) + lane, ll = c / MS_R, rr = c % MS_R;
+    const bool in = (int64_t)row * MS_L + ll < nl;
+    for (int o = wave >> 1; o < no; o += 2) {
+      float yr = 0, yi = 0;
+      for (unsigned int m = __builtin_amdgcn_readfirstlane(nz[o]); m; m &= m - 1) {
+        const int i = __builtin_ctz(m);
+        const float2 w = W[o * ni + i], v = X[i * MS_C + c];
+        yr += w.x * v.x - w.y * v.y;
+        yi += w.x * v.y + w.y * v.x;
+      }
+      const int m = o / ns, s = o - m * ns;
+      Y[(s * MS_R + rr) * ys + ll * kp + m] = in ? make_float2(yr, yi) : make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    for (int q = t; q < ns * MS_R * run; q += 256) {
+      const int col = q / run, w = q - col * run;
+      const int kb = w / (2 * V3_NT), term = (w % (2 * V3_NT)) >> 1, half = w & 1;
+      const int64_t kbg = (int64_t)row * kp + kb, r = r0 + col % MS_R;
+      if (r >= nr || kbg * V3_BK >= K2p) continue;
+      const float2* v = Y + col * ys + 8 * kb + 4 * half;
+      float a[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        a[2 * j] = v[j].x;
+        a[2 * j + 1] = v[j].y;
+      }
+      *(bf16x8_t*)(P + v3_chunk((int64_t)(col / MS_R) * nr + r, kbg, term, half, K2p)) =
+          term8(a, term);
+    }
+  }
+}
+
+// the B terms of a pre-split product in its scratch, after the A terms
+inline __bf16* v3_b_terms(const ZGemm& z) {
+  const int64_t pza = v2_round(z.M, V2_BM) * v3_kpad(z.K) * V3_NT;
+  return (__bf16*)(((uintptr_t)z.sws + 255) & ~(uintptr_t)255) + z.batch * pza;
+}
+
+inline bool use_bf16_v3(const ZGemm& z, void* mws);
+
+int mode_mix_split3(ZGemm& z, int64_t nl, int64_t ni, int64_t no, int64_t kp, int64_t nr,
+                    const void* wm, int64_t bw, bool wtrans, const void* x, void* mws,
+                    hipStream_t s, bool* done) {
+  *done = false;
+  if (ni < 1 || no < 1 || ni > MS_MAX || no > MS_MAX || no % kp || nl > 65535) return PTN_OK;
+  const int64_t nunits = ((nl + MS_L - 1) / MS_L) * ((nr + MS_R - 1) / MS_R);
+  // X, Y and W of a workgroup; beyond 64 KiB (more than 24 x 24) the two passes
+  const size_t lds = (size_t)(ni * MS_C + (no / kp) * MS_R * (MS_L * kp + 1) + ni * no) * 8;
+  if (!use_bf16_v3(z, mws) || nunits > 0x3fffffff || lds > 65000) return PTN_OK;
+  const int64_t K2p = v3_kpad(z.K), pz = v2_round(2 * z.N, V2_BN) / 2 * K2p * V3_NT;
+  const int64_t cap = 1024 / z.batch > 256 ? 1024 / z.batch : 256;
+  const SkipFlag sk = skip_flag();
+  k_mix_split3<<<dim3((unsigned)(nunits < cap ? nunits : cap), (unsigned)z.batch), 256, lds, s>>>(
+      nl, (int)ni, (int)no, (int)kp, nr, (int)nunits, (const double2*)wm, wtrans, (const float2*)x,
+      bw, K2p, pz, v3_b_terms(z), sk.p, sk.stride);
+  PTN_LAUNCH_CHECK();
+  z.b_terms = *done = true;
+  return PTN_OK;
+}
+
 // 256 x 256 real tiles, 8 waves (2 x 4) of 128 x 64 as in zgemm_bf16x3_v2. The
 // 16-deep k-stages (256 rows of A and 128 of B, 96 bytes each: 36 KiB) are
 // loaded straight into LDS, four buffers deep, with one barrier per stage: no
@@ -887,13 +1009,14 @@ inline int launch_bf16_v3(const ZGemm& z, hipStream_t s) {
   const int64_t pza = Mp * K2p * V3_NT, pzb = N2p / 2 * K2p * V3_NT;
   char* base = (char*)(((uintptr_t)z.sws + 255) & ~(uintptr_t)255);
   __bf16* pa = (__bf16*)base;
-  __bf16* pb = pa + z.batch * pza;
+  __bf16* pb = v3_b_terms(z);
   const unsigned bt = (unsigned)z.batch;
   const unsigned kblk = (unsigned)((K2p + 63) / 64);   // 32 complex k per block
   k_split3<TA><<<dim3(kblk, (unsigned)(Mp / 64), bt), 256, 0, s>>>(
       z.M, z.K, (const TA*)z.A, z.a_m, z.a_k, z.conjA, z.bz_a, K2p, pza, pa);
-  k_split3<TB><<<dim3(kblk, (unsigned)(N2p / 128), bt), 256, 0, s>>>(
-      z.N, z.K, (const TB*)z.B, z.b_n, z.b_k, z.conjB, z.bz_b, K2p, pzb, pb);
+  if (!z.b_terms)
+    k_split3<TB><<<dim3(kblk, (unsigned)(N2p / 128), bt), 256, 0, s>>>(
+        z.N, z.K, (const TB*)z.B, z.b_n, z.b_k, z.conjB, z.bz_b, K2p, pzb, pb);
   PTN_LAUNCH_CHECK();
   const int sk = v2_splitk(z.M, z.N, z.K, z.batch);
   V2Args g;

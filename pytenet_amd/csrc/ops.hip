@@ -151,13 +151,19 @@ int heff_apply(int prec, const Dims& D, const void* l, int tl, const void* w, co
               r, D.Mr * D.Dr, 1, 0,
               t1, D.Mr * D.Dr, 1, 0, batch, nA, nR, n1, sws, spb};
   if ((st = zgemm(g1, cp, ta1, tr, ct, mws, mb, s))) return st;
-  if ((st = mode_mix(D.Dl, D.d * D.Mr, D.Ml * D.d, D.Dr, w, t1, ct, t2, ct, s, batch,
-                     D.Ml * D.d * D.d * D.Mr)))
-    return st;
   ZGemm g3 = {D.Dl, D.d * D.Dr, D.Dl * D.Ml,
               l, 1, D.Dl, 0,
               t2, D.d * D.Dr, 1, 0,
               out, D.d * D.Dr, 1, 0, batch, nL, n2, nA, sws, spb};
+  bool mixed = false;
+  if (cp == PTN_BF16X6 &&
+      (st = mode_mix_split3(g3, D.Dl, D.d * D.Mr, D.Ml * D.d, D.Ml, D.Dr, w,
+                            D.Ml * D.d * D.d * D.Mr, false, t1, mws, s, &mixed)))
+    return st;
+  if (!mixed &&
+      (st = mode_mix(D.Dl, D.d * D.Mr, D.Ml * D.d, D.Dr, w, t1, ct, t2, ct, s, batch,
+                      D.Ml * D.d * D.d * D.Mr)))
+    return st;
   return zgemm(g3, cp, tl, ct, tout, mws, mb, s);
 }
 
@@ -238,15 +244,20 @@ int env_left(int prec, const Dims& D, const void* a, const void* b, const void* 
               b, D.d * D.Dr, 1, 1,
               t1, D.d * D.Dr, 1, 0, batch, nL, nA, n1, sws, spb};
   if ((st = zgemm(g1, cp, tl, PTN_T_C128, ct, mws, mb, s))) return st;
-  // T2[l, (s, m'), rb] = sum_{(m, sb)} W[m, sb, s, m'] T1[l, (m, sb), rb]: the mix
-  // with W read as the transpose of Wmat[(m, sb), (s, m')]
-  if ((st = mode_mix(D.Dl, D.Ml * D.d, D.d * D.Mr, D.Dr, w, t1, ct, t2, ct, s, batch, nW, true)))
-    return st;
   // out[r, (m', rb)] = sum_{(l, s)} A[(l, s), r] T2[(l, s), (m', rb)]
   ZGemm g3 = {D.Dr, D.Mr * D.Dr, D.Dl * D.d,
               a, 1, D.Dr, 0,
               t2, D.Mr * D.Dr, 1, 0,
               out, D.Mr * D.Dr, 1, 0, batch, nA, n2, nO, sws, spb};
+  // T2[l, (s, m'), rb] = sum_{(m, sb)} W[m, sb, s, m'] T1[l, (m, sb), rb]: the mix
+  // with W read as the transpose of Wmat[(m, sb), (s, m')]
+  bool mixed = false;
+  if (cp == PTN_BF16X6 && (st = mode_mix_split3(g3, D.Dl, D.Ml * D.d, D.d * D.Mr, D.d, D.Dr, w, nW,
+                                                true, t1, mws, s, &mixed)))
+    return st;
+  if (!mixed && (st = mode_mix(D.Dl, D.Ml * D.d, D.d * D.Mr, D.Dr, w, t1, ct, t2, ct, s, batch, nW,
+                               true)))
+    return st;
   return zgemm(g3, cp, PTN_T_C128, ct, PTN_T_C128, mws, mb, s);
 }
 
