@@ -720,8 +720,7 @@ __global__ __launch_bounds__(256) void k_split3(int64_t M, int64_t K, const TA* 
 // input, and kp whole k-blocks of 16 real k per column, a run of 96 kp bytes of the terms.
 // Sums as in mode_mix_kernel. The columns beyond N that fill up the last tile are not
 // written: they reach no output. Two-site H_eff at D = 1024 (20 x 20): mix and split
-// 59 + 77 -> 128 us, H_eff 1768 -> 1755 us; the splits' arithmetic and two workgroups' worth of
-// phases per CU keep it below the copy rate (3.3 TB/s).
+// 59 + 77 -> 119 us (3.5 TB/s; 129 us with a thread per term), the whole H_eff 1.4 % less.
 constexpr int MS_L = 8, MS_R = 16, MS_C = MS_L * MS_R, MS_MAX = 32;
 
 __global__ __launch_bounds__(256) void k_mix_split3(
@@ -763,7 +762,7 @@ __global__ __launch_bounds__(256) void k_mix_split3(
     W[e] = make_float2((float)w.x, (float)w.y);
     if (w.x != 0.0 || w.y != 0.0) atomicOr(&nz[o], 1u << i);
   }
-  const int run = kp * V3_NT * 2;               // 16-byte chunks of a column's run
+  const int run = 2 * kp;                       // half k-blocks of a column: a chunk of each term
   for (; u < nunits; u += gridDim.x) {
     __syncthreads();   // the previous unit has been mixed and written
 #pragma unroll
@@ -790,19 +789,23 @@ __global__ __launch_bounds__(256) void k_mix_split3(
     }
     __syncthreads();
     for (int q = t; q < ns * MS_R * run; q += 256) {
-      const int col = q / run, w = q - col * run;
-      const int kb = w / (2 * V3_NT), term = (w % (2 * V3_NT)) >> 1, half = w & 1;
-      const int64_t kbg = (int64_t)row * kp + kb, r = r0 + col % MS_R;
+      const int col = q / run, w = q - col * run, half = w & 1;
+      const int64_t kbg = (int64_t)row * kp + (w >> 1), r = r0 + col % MS_R;
       if (r >= nr || kbg * V3_BK >= K2p) continue;
-      const float2* v = Y + col * ys + 8 * kb + 4 * half;
-      float a[8];
+      const float2* v = Y + col * ys + 4 * w;
+      bf16x8_t hi, mid, lo;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        a[2 * j] = v[j].x;
-        a[2 * j + 1] = v[j].y;
+        __bf16 h, d, e;
+        split3(v[j].x, h, d, e);
+        hi[2 * j] = h; mid[2 * j] = d; lo[2 * j] = e;
+        split3(v[j].y, h, d, e);
+        hi[2 * j + 1] = h; mid[2 * j + 1] = d; lo[2 * j + 1] = e;
       }
-      *(bf16x8_t*)(P + v3_chunk((int64_t)(col / MS_R) * nr + r, kbg, term, half, K2p)) =
-          term8(a, term);
+      __bf16* to = P + v3_chunk((int64_t)(col / MS_R) * nr + r, kbg, 0, half, K2p);
+      *(bf16x8_t*)to = hi;
+      *(bf16x8_t*)(to + V3_BK) = mid;
+      *(bf16x8_t*)(to + 2 * V3_BK) = lo;
     }
   }
 }
