@@ -980,14 +980,16 @@ bool autotune_enabled();
 //  * 64 x 32 tiles from 192 up. Fewer than about two per CU leave the matrix cores
 //    waiting for operands: then k is split over two or four groups of the workgroup
 //    (256 tiles, 512 x 1024 x 2560: 50.1 / 61.8 / 62.9 TFLOP/s with 1 / 2 / 4 groups).
-//    With loads into LDS two groups pay up to 2048 tiles (1280 tiles, 1024 x 2560 x 512: 59.7 /
-//    62.6 / 56.9; 2048, 2048^3: 66.0 / 66.4; 10240: 67.2 / 66.5), staged through registers
-//    one group does from 600 on (1280 tiles: 59.0 / 55.9 / 51.2).
+//    FP64, loaded into LDS: two groups pay up to 2048 tiles (1280 tiles, 1024 x 2560 x 512: 59.7 /
+//    62.6 / 56.9; 2048, 2048^3: 66.0 / 66.4; 10240: 67.2 / 66.5). Staged through registers (all
+//    of FP32) one group does from 600 on (FP64, 1280 tiles: 59.0 / 55.9 / 51.2); masked or unaligned FP64
+//    products, which are staged so too, still take the groups of the others.
 //  * tile-skipping products (mask workspace given) never take the large tiles: the
 //    small one skips the zero blocks of sector-structured operands at finer
 //    granularity, which outweighs its lower efficiency per flop (U(1) two-site DMRG
-//    at L=128, D=2048: 76 s against 82 s per sweep). The split of k is that of the
-//    unmasked product, so both add in the same order.
+//    at L=128, D=2048: 76 s against 82 s per sweep).
+//  * the split of k depends on shape and type alone (k_groups), so that masked and
+//    unmasked products add in the same order.
 //  * 32 x 16 tiles for fewer, or where 64-row tiles would be a third padding (the
 //    32-row products of the blocked QR, 32 x 1984 x 248 x 8: 27.8 us against 42.2).
 inline double wave_fill(int64_t tiles, int64_t slots) {
@@ -997,6 +999,27 @@ inline int64_t tiles_of(const ZGemm& z, int BM, int BN) {
   return ((z.M + BM - 1) / BM) * ((z.N + BN - 1) / BN) * z.batch;
 }
 inline bool wave_tile_product(const ZGemm& z) { return tiles_of(z, 16, 8) <= 320; }
+// 128 x 128 tiles (FP32), 128 x 64 tiles, 64 x 32 tiles (else 32 x 16)
+template <typename Tc> inline bool wide_tiles(const ZGemm& z) {
+  const int64_t wide = tiles_of(z, 128, 128);
+  return sizeof(Tc) == 4 && wide >= 512 && wave_fill(wide, 512) >= 0.8;
+}
+inline bool large_tiles(const ZGemm& z) {
+  const int64_t t44 = tiles_of(z, 128, 64);
+  return t44 >= 512 && wave_fill(t44, 512) >= 0.96;
+}
+inline bool medium_tiles(const ZGemm& z) {   // tiles of 32 x 16 per one of 64 x 32: 4 without padding
+  const int64_t t22 = tiles_of(z, 64, 32);
+  return t22 >= 192 && 3 * t22 <= tiles_of(z, 32, 16);
+}
+// groups of k of a product beyond the wave tiles
+template <typename Tc> inline int k_groups(const ZGemm& z) {
+  if (z.K < 64 || wide_tiles<Tc>(z) || large_tiles(z)) return 1;
+  if (!medium_tiles(z)) return tiles_of(z, 32, 16) >= 512 ? 1 : z.K < 256 ? 2 : 4;
+  const int64_t t22 = tiles_of(z, 64, 32);
+  if (t22 >= (sizeof(Tc) == 8 ? 2048 : 600)) return 1;
+  return z.K < 256 || t22 >= 600 ? 2 : 4;
+}
 
 template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_heuristic(const ZGemm& z, hipStream_t s, void* mws, size_t mws_bytes) {
@@ -1005,23 +1028,17 @@ inline int launch_heuristic(const ZGemm& z, hipStream_t s, void* mws, size_t mws
     return launch_wave<Tc, TA, TB, TC, 1, 4>(z, s);
   }
   const bool masked = mws && z.batch == 1;
-  if constexpr (sizeof(Tc) == 4) {
-    const int64_t wide = tiles_of(z, 128, 128);
-    if (!masked && wide >= 512 && wave_fill(wide, 512) >= 0.8)
-      return launch_cfg<Tc, TA, TB, TC, 4, 8>(z, s);
-  }
-  const int64_t t44 = tiles_of(z, 128, 64), t22 = tiles_of(z, 64, 32), t11 = tiles_of(z, 32, 16);
-  const bool dma = sizeof(Tc) == 8 && !masked && dma_operands(z);
-  if (!masked && t44 >= 512 && wave_fill(t44, 512) >= 0.96)
-    return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s);
-  if (t22 >= 192 && 3 * t22 <= t11) {   // t11 / t22 is 4 without padding
-    if (t22 >= (dma ? 2048 : 600) || z.K < 64)
-      return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
-    if (z.K < 256 || t22 >= 600) return launch_cfg<Tc, TA, TB, TC, 2, 2, 2>(z, s, mws, mws_bytes);
+  if constexpr (sizeof(Tc) == 4)
+    if (!masked && wide_tiles<Tc>(z)) return launch_cfg<Tc, TA, TB, TC, 4, 8>(z, s);
+  if (!masked && large_tiles(z)) return launch_cfg<Tc, TA, TB, TC, 4, 4>(z, s);
+  const int groups = k_groups<Tc>(z);
+  if (medium_tiles(z)) {
+    if (groups == 1) return launch_cfg<Tc, TA, TB, TC, 2, 2>(z, s, mws, mws_bytes);
+    if (groups == 2) return launch_cfg<Tc, TA, TB, TC, 2, 2, 2>(z, s, mws, mws_bytes);
     return launch_cfg<Tc, TA, TB, TC, 2, 2, 4>(z, s, mws, mws_bytes);
   }
-  if (z.K < 64 || t11 >= 512) return launch_cfg<Tc, TA, TB, TC, 1, 1>(z, s, mws, mws_bytes);
-  if (z.K < 256) return launch_cfg<Tc, TA, TB, TC, 1, 1, 2>(z, s, mws, mws_bytes);
+  if (groups == 1) return launch_cfg<Tc, TA, TB, TC, 1, 1>(z, s, mws, mws_bytes);
+  if (groups == 2) return launch_cfg<Tc, TA, TB, TC, 1, 1, 2>(z, s, mws, mws_bytes);
   return launch_cfg<Tc, TA, TB, TC, 1, 1, 4>(z, s, mws, mws_bytes);
 }
 
