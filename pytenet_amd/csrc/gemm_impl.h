@@ -486,9 +486,12 @@ __global__ __launch_bounds__(256 * Ring::WK) void zgemm_kernel(GemmKArgs g) {
 #pragma unroll
   for (int i = 0; i < NB; ++i)
     offb[i] = (uint32_t)((min(bcol(wave * NB + i), nlast) * g.b_n + bk(wave * NB + i) * g.b_k) * 16);
-  const int nst = (int)(g.K / BK);                 // whole stages, `per` at most to a group
-  const int per = (nst + WK - 1) / WK, least = max(0, nst - (WK - 1) * per);
-  const int mine = WK == 1 ? per : min(per, max(0, nst - grp * per));
+  // the shares of k are those of zgemm_kernel: `per` of all stages to a group, the partial
+  // last one to the group in whose share it lies; nst, mine, least: whole stages in all, of this
+  // group and of the last one
+  const int nst = (int)(g.K / BK), per = (int)((g.K + BK - 1) / BK + WK - 1) / WK;
+  const int least = max(0, nst - (WK - 1) * per), most = min(per, nst);
+  const int mine = WK == 1 ? nst : min(per, max(0, nst - grp * per));
   const int64_t sta = g.a_k * (BK * 16), stb = g.b_k * (BK * 16);
   const char* Ag = A + (int64_t)(mine ? grp * per : 0) * sta;
   const char* Bg = B + (int64_t)(mine ? grp * per : 0) * stb;
@@ -569,7 +572,7 @@ __global__ __launch_bounds__(256 * Ring::WK) void zgemm_kernel(GemmKArgs g) {
     read(An, Bn, 0, cur);
     if (on) mul(nxt);
   };
-  if (per > 0) {
+  if (most > 0) {
     dma(A0, B0, 0);
     dma(A1, B1, 1);
     dma(A2, B2, 2);
@@ -582,18 +585,19 @@ __global__ __launch_bounds__(256 * Ring::WK) void zgemm_kernel(GemmKArgs g) {
       step(A1, B1, A2, B2, st + 1, true);
       step(A2, B2, A0, B0, st + 2, true);
     }
-    for (; st < per; st += 3) {
+    for (; st < most; st += 3) {
       step(A0, B0, A1, B1, st, st < mine);
-      if (st + 1 < per) step(A1, B1, A2, B2, st + 1, st + 1 < mine);
-      if (st + 2 < per) step(A2, B2, A0, B0, st + 2, st + 2 < mine);
+      if (st + 1 < most) step(A1, B1, A2, B2, st + 1, st + 1 < mine);
+      if (st + 2 < most) step(A2, B2, A0, B0, st + 2, st + 2 < mine);
     }
     __builtin_amdgcn_s_waitcnt(0x70);   // no load may land in LDS from here on
   }
   __syncthreads();
   const int rem = (int)(g.K - (int64_t)nst * BK);
-  if (rem) {   // the last, partial stage through registers, by the last group
+  if (rem) {   // the last, partial stage through registers
     const int64_t k0 = (int64_t)nst * BK;
-    if (grp == WK - 1) {
+    const int last = WK == 1 ? 0 : nst / per;
+    if (grp == last) {
 #pragma unroll
       for (int i = 0; i < NA; ++i) {
         const int c = wave * NA + i;
@@ -612,7 +616,7 @@ __global__ __launch_bounds__(256 * Ring::WK) void zgemm_kernel(GemmKArgs g) {
       }
     }
     __syncthreads();
-    if (grp == WK - 1) {
+    if (grp == last) {
       read(A0, B0, 0, cur);
       read(A0, B0, 1, nxt);
       mul(cur);
