@@ -125,7 +125,8 @@ size_t ptn_zgemm_workspace(int64_t M, int64_t N, int64_t K);
  * whose products are BLAS calls): with on != 0, the first product of each
  * shape times the tile configurations on the caller's stream (synchronising
  * it once) and keeps the fastest for that shape; products that accumulate
- * into C or skip zero tiles keep the fixed choice. C must not alias A or B
+ * into C, skip zero tiles or are split over k inside a workgroup keep the fixed
+ * choice. The result has the same bits in every case. C must not alias A or B
  * while it is on. Process-wide; returns the previous setting. */
 int ptn_set_autotune(int on);
 int ptn_zgemm(int64_t M, int64_t N, int64_t K,

@@ -1058,10 +1058,11 @@ inline int launch_choice(int c, const ZGemm& z, hipStream_t s) {
 // Tile autotuner: the first product of a given shape (M, N, K, batch and the
 // contiguity of the operands) times the rule's choice and the other large tiles (two timed
 // launches each after one untimed, HIP events on the caller's stream) and
-// keeps the fastest for that shape. Only products that overwrite C are tuned
-// (a repeated launch then leaves the same result); the tuning launch of the
-// chosen configuration is the product itself. It synchronises the stream
-// once per new shape, hence opt-in.
+// keeps the fastest for that shape. It synchronises the stream once per new shape, hence opt-in.
+// Tuned are products that overwrite C (a repeated launch then leaves the same result) and
+// for which the rule takes a single group of k: the candidates are single groups, and
+// with the division of k the sums are the same in every tile, so that the
+// result does not depend on what was timed. (Where the rule splits k, a single group is slower.)
 template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_tuned(const ZGemm& z, hipStream_t s) {
   struct Key {
@@ -1117,7 +1118,8 @@ template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_typed(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t mws_bytes = 0) {
   if (mws && z.batch == 1) return launch_heuristic<Tc, TA, TB, TC>(z, s, mws, mws_bytes);
   // (the wave tile is not in question for the products that the rule gives it)
-  if (!z.accumulate && autotune_enabled() && !noalloc_mode() && !wave_tile_product(z)) {
+  if (!z.accumulate && autotune_enabled() && !noalloc_mode() && !wave_tile_product(z) &&
+      k_groups<Tc>(z) == 1) {
     // tuning synchronises the stream, which a stream capture does not allow
     hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cst) == hipSuccess && cst == hipStreamCaptureStatusNone)

@@ -1,8 +1,11 @@
 """
 The order of the sums in a complex product (csrc/gemm_impl.h) depends on its shape and
-type alone: the same bits with and without tile masks, and for operands on and off the
-16-byte boundary (loads into LDS or through registers).
+type alone: the same bits with and without tile masks, for operands on and off the
+16-byte boundary (loads into LDS or through registers), and with the tile autotuner
+on or off, whose candidates all divide k as the rule's choice does.
 """
+
+import re
 
 import numpy as np
 import pytest
@@ -63,3 +66,35 @@ def test_sums_do_not_depend_on_the_alignment(fixed_rule, M, N, K):
         None, 0, backend.stream()))
     assert st == 0 and not any("LdsRing" in n for n in names), names
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES + [(200, 300, 40), (300, 500, 90)])
+def test_tuned_products_divide_k_as_the_rule_does(M, N, K):
+    rng = np.random.default_rng(M - K)
+    A, B = backend.as_dev(orc.crandn((M, K), rng)), backend.as_dev(orc.crandn((K, N), rng))
+    prev = backend.set_autotune(False)
+    try:
+        ref, rule = _names(lambda: backend.matmul(A, B))
+        backend.set_autotune(True)
+        tuned, names = _names(lambda: backend.matmul(A, B))
+        again = backend.matmul(A, B)
+    finally:
+        backend.set_autotune(prev)
+
+    def groups(n):   # the k groups of zgemm_kernel<types, tile, groups, layouts>
+        return re.search(r", (?:\d+, \d+|WaveTile<\d+>), (?:LdsRing<)?(\d+)", n).group(1)
+    assert {groups(n) for n in names} == {groups(n) for n in rule}, (rule, names)
+    assert torch.equal(tuned, ref) and torch.equal(again, ref)
+
+
+def test_tuned_fp32_matvec_has_the_bits_of_the_rule():
+    """One group in the first product (1280 tiles, tuned), four in the second."""
+    a, w, l, r, _ = _operator(np.random.default_rng(2), 512, 512, False)
+    prev = backend.set_autotune(False)
+    try:
+        ref = backend.heff_apply(a, w, l, r, "fp32")
+        backend.set_autotune(True)
+        for _ in range(2):
+            assert torch.equal(backend.heff_apply(a, w, l, r, "fp32"), ref)
+    finally:
+        backend.set_autotune(prev)
