@@ -987,7 +987,10 @@ bool autotune_enabled();
 //    FP64, loaded into LDS: two groups pay up to 2048 tiles (1280 tiles, 1024 x 2560 x 512: 59.7 /
 //    62.6 / 56.9; 2048, 2048^3: 66.0 / 66.4; 10240: 67.2 / 66.5). Staged through registers (all
 //    of FP32) one group does from 600 on (FP64, 1280 tiles: 59.0 / 55.9 / 51.2); masked or unaligned FP64
-//    products, which are staged so too, still take the groups of the others.
+//    products, which are staged so too, still take the groups of the others. Batches in
+//    FP64 take one group from 256 tiles on unless k is long (24 of 100 x 200 x 500, 336 tiles: 85 us with
+//    four groups, 77 with one; 64 of 128 x 320 x 64, 1280 tiles: 37 with two, 30 with one; 4 of 100 x 1000 x
+//    200, 256 tiles: 19 and 20; 4 of 240 x 960 x 2000, 480 tiles: four are no slower).
 //  * tile-skipping products (mask workspace given) never take the large tiles: the
 //    small one skips the zero blocks of sector-structured operands at finer
 //    granularity, which outweighs its lower efficiency per flop (U(1) two-site DMRG
@@ -1022,6 +1025,7 @@ template <typename Tc> inline int k_groups(const ZGemm& z) {
   if (!medium_tiles(z)) return tiles_of(z, 32, 16) >= 512 ? 1 : z.K < 256 ? 2 : 4;
   const int64_t t22 = tiles_of(z, 64, 32);
   if (t22 >= (sizeof(Tc) == 8 ? 2048 : 600)) return 1;
+  if (sizeof(Tc) == 8 && z.batch > 1 && t22 >= 256 && z.K <= 1024) return 1;
   return z.K < 256 || t22 >= 600 ? 2 : 4;
 }
 
@@ -1062,7 +1066,7 @@ inline int launch_choice(int c, const ZGemm& z, hipStream_t s) {
 // Tuned are products that overwrite C (a repeated launch then leaves the same result) and
 // for which the rule takes a single group of k: the candidates are single groups, and
 // with the division of k the sums are the same in every tile, so that the
-// result does not depend on what was timed. (Where the rule splits k, a single group is slower.)
+// result does not depend on what was timed.
 template <typename Tc, typename TA, typename TB, typename TC>
 inline int launch_tuned(const ZGemm& z, hipStream_t s) {
   struct Key {
