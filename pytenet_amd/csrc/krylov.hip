@@ -432,8 +432,8 @@ __device__ __forceinline__ bool tridiag_coefs(int n, const double* alpha, const 
   for (int l = 0; l < n; ++l) {
     int iter = 0;
     for (;;) {
-      const bool tiny = lane >= l && lane < n - 1 &&
-                        fabs(e) <= DBL_EPSILON * (fabs(d) + fabs(lane_shift<true>(d)));
+      const double dn = lane_shift<true>(d);   // by all lanes: a lane that is off reads as zero
+      const bool tiny = lane >= l && lane < n - 1 && fabs(e) <= DBL_EPSILON * (fabs(d) + fabs(dn));
       const unsigned long long at = __ballot(tiny);
       const int m = at ? __ffsll(at) - 1 : n - 1;
       if (m == l) break;
