@@ -39,6 +39,14 @@ def _absorb_right(a, c):
     return backend.matmul_batched(a.reshape(nb, Dl * d, D), c).reshape(nb, Dl, d, c.shape[2])
 
 
+def _stack(tensors):
+    """The MPO tensors of one site of all chains: host arrays stacked there and uploaded at
+    once; with device or host tensors among them (lazily conjugated ones too) on the device."""
+    if any(isinstance(t, torch.Tensor) for t in tensors):
+        return torch.stack([backend.as_dev(t) for t in tensors])
+    return backend.as_dev(np.stack(tensors))
+
+
 class _Bucket:
     """Stacked device state of chains with identical shapes, with its own HIP
     stream: the buckets of a call advance site step by site step together,
@@ -56,9 +64,7 @@ class _Bucket:
             for p in psis:
                 for a in p.a:
                     a.record_stream(self.stream)
-            # one upload per site: the MPO tensors of the chains stacked on the host
-            self.W = [backend.as_dev(np.stack([backend.to_host(H.a[i]) for H in hamiltonians]))
-                      for i in range(self.n)]
+            self.W = [_stack([H.a[i] for H in hamiltonians]) for i in range(self.n)]
         self.status = []
 
     def site_expm(self, a, l, w, r, dt):
