@@ -348,7 +348,7 @@ int ptn_svd_precond32(int64_t batch, int64_t m, int64_t n, const void* a, void* 
  * algorithmic flops (8 per complex multiply-add) and bytes (each operand
  * once). */
 typedef struct {
-  char name[160];    /* e.g. "zgemm_kernel<float, c64, c64, c128, 4, 8, true, true>" */
+  char name[160];    /* e.g. "zgemm_kernel<float, c64, c64, c128, 4, 8, 1, true, true>" */
   int64_t launches;
   double total_ms;
   double flop;

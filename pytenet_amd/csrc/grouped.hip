@@ -432,6 +432,9 @@ struct SectorPlan {
 // against both on 32 x 16 tiles: D = 96 40 / 35 us, 512 78 / 59, 1024 138 / 112,
 // 1500 261 / 248, 2048 493 / 503 (and 473 with the output product alone on 32 x 16:
 // 811 tiles of 64 x 32 are 3.2 per CU).
+// FP32 products take the choice of the FP64 rates, which was not measured tile by
+// tile there: with the staging of this kernel two-site H_eff in FP32 went from 41 to 38 us at D = 96, 100 to 68
+// at 512, 219 to 167 at 1024 and 784 to 668 at 2048.
 static void finish_product(GProduct& P, size_t csz_a, size_t csz_b, size_t csz_c) {
   static const struct { int code; int64_t bm, bn; double rate; } tile[3] = {
       {4, 128, 64, 65.0}, {2, 64, 32, 63.0}, {1, 32, 16, 52.0}};

@@ -867,8 +867,7 @@ __global__ void k_ns_update(int64_t n, const double2* __restrict__ Q, const doub
 
 static inline size_t al(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// pinned words for the rotation count, flags and the singular values of small splits,
-// allocated once per thread
+// pinned words for the counters (rotations, flags, sweeps), allocated once per thread
 constexpr int PINNED_INTS = 4;
 static int* pinned_counter() {
   static thread_local int* p = nullptr;
@@ -1147,25 +1146,10 @@ static void jacobi_sweep(const SvdLayout& L, char* base, typename JacT<T>::c2* X
   }
 }
 
-// Thin SVD of `batch` m x n matrices of identical shape (problem b at a + b sa,
-// u + b su, s + b ss, vh + b svh). The Jacobi sweeps run on all problems at
-// once and stop together, after the first sweep in which no problem needed a
-// rotation above `big` (relative); those of k_jac_small stop each by itself. info (if given) receives the number of
-// sweeps, whether the sweep limit was hit, and whether any singular value was
-// not finite.
-// With `precond32` (and at least PRE32_MIN_Q columns) the Jacobi phase starts
-// with FP32 sweeps: X32 = X / max column norm in complex64 is orthogonalised
-// on FP32 MFMA until no pair needs a rotation above 1e-3 relative, with the
-// rotations accumulated in V32. V32 is unitary only to FP32 rounding, so it is
-// replaced by its unitary polar factor Q (two Newton-Schulz steps in FP64,
-// Q <- 1.5 Q - 0.5 Q (Q^H Q), each squaring the distance from unitarity), and
-// the FP64 sweeps continue from X Q with V = Q. The FP64 sweeps and their
-// stopping rule are those of the plain path, so the result has the same FP64
-// accuracy; the FP32 sweeps only remove most of the rotation work.
 // Jacobi phase on X (q x qp column-major per problem, the preconditioned
 // matrix R2^H). With want_v the rotations are accumulated into V (qp x qp per
-// problem); FP32 preconditioning (L.pre32) needs V. On return X points at the orthogonalised columns (another buffer
-// of the workspace after FP32 preconditioning).
+// problem); FP32 preconditioning (L.pre32, see svd_run) needs V. On return X points at the
+// orthogonalised columns (another buffer of the workspace after FP32 preconditioning).
 struct JacobiResult {
   int sweeps = 0, sweeps32 = 0, converged = 0;
   bool ranked = false;   // k_jac_small: norms, order and singular values are done, and the
