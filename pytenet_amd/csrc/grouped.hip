@@ -42,6 +42,7 @@
 #include <mutex>
 #include <string>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 #include "gemm_impl.h"
 #include "ops.h"
@@ -391,6 +392,7 @@ static bool sectors_of(const int64_t* q, int64_t n, std::map<int64_t, Sector>& o
 
 struct GProduct {
   std::vector<GBlock> blocks;
+  std::vector<std::pair<int64_t, int32_t>> order;   // (-K, block), as uploaded
   int64_t tiles = 0;
   int tile = 2;         // TileCfg<tile, tile>: 128 x 64 (4), 64 x 32 (2) or 32 x 16 (1)
   double flop = 0.0;    // 8 M N K summed over the blocks
@@ -466,11 +468,14 @@ static void finish_product(GProduct& P, size_t csz_a, size_t csz_b, size_t csz_c
     pick = cost(2) < cost(1) ? 2 : 1;
   }
   P.tile = tile[pick].code;
-  // the tiles with the longest sums first, so that the last workgroups are short ones
-  std::stable_sort(P.blocks.begin(), P.blocks.end(),
-                   [&](const GBlock& x, const GBlock& y) { return total_k(x) > total_k(y); });
+  // the tiles with the longest sums first, so that the last workgroups are short ones: the
+  // blocks' order in the device array (the descriptors themselves are 424 bytes each)
+  P.order.resize(P.blocks.size());
+  for (size_t i = 0; i < P.blocks.size(); ++i) P.order[i] = {-total_k(P.blocks[i]), (int32_t)i};
+  std::sort(P.order.begin(), P.order.end());
   int64_t tiles = 0;
-  for (GBlock& b : P.blocks) {
+  for (const auto& o : P.order) {
+    GBlock& b = P.blocks[o.second];
     b.tiles_n = (int32_t)((b.N + tile[pick].bn - 1) / tile[pick].bn);
     b.tile0 = tiles;
     tiles += ((b.M + tile[pick].bm - 1) / tile[pick].bm) * b.tiles_n;
@@ -755,8 +760,10 @@ int sector_plan_get(const ptn_local_op* op, int kind, SectorPlanRef* out) {
     g_plans.emplace(key, nullptr);
     return PTN_OK;
   }
-  std::vector<GBlock> all(sp->p1.blocks);
-  all.insert(all.end(), sp->p3.blocks.begin(), sp->p3.blocks.end());
+  std::vector<GBlock> all;
+  all.reserve(sp->p1.blocks.size() + sp->p3.blocks.size());
+  for (const GProduct* p : {&sp->p1, &sp->p3})
+    for (const auto& o : p->order) all.push_back(p->blocks[o.second]);
   const size_t bb = (all.size() * sizeof(GBlock) + 255) & ~(size_t)255;
   const size_t mb = sp->mix.size() * sizeof(MixUnit);
   hipError_t e = hipMalloc((void**)&sp->dev, bb + mb);
