@@ -908,6 +908,10 @@ inline bool fill_args(const ZGemm& z, GemmKArgs& g, int BM, int BN) {
     return PTN_OK;                                                                              \
   } while (0)
 
+inline int64_t tiles_of(const ZGemm& z, int BM, int BN) {
+  return ((z.M + BM - 1) / BM) * ((z.N + BN - 1) / BN) * z.batch;
+}
+
 // loads of 16 bytes into LDS need operands on 16-byte boundaries
 inline bool dma_operands(const ZGemm& z) { return (((uintptr_t)z.A | (uintptr_t)z.B) & 15) == 0; }
 template <int TM, int TN, int WK>
@@ -948,7 +952,13 @@ inline int launch_cfg(const ZGemm& z, hipStream_t s, void* mws = nullptr, size_t
   if (st) return st;
   if constexpr (sizeof(Tc) == 8 && TM >= 2) {
     static_assert(sizeof(TA) == 16 && sizeof(TB) == 16 && sizeof(TC) == 16, "complex128 operands");
-    if (g.fast && !g.maskA && dma_operands(z)) return launch_dma<TM, TN, WK>(z, g, s);
+    // At most two whole stages leave nothing to keep in flight, and with more tiles than the chip
+    // holds with three stage buffers each the two of the register-staged kernel let more of them in:
+    // 1095 x 2249 x 5 (1278 tiles of 64 x 32) 12.3 -> 10.6 us, 8000 x 500 x 3 15.8 -> 14.1, 4000 x 3000 x 5
+    // (1504 of 128 x 64) 42.1 -> 39.0; from K = 24 on the ring is as fast or faster.
+    const int64_t fit = 256 * (160 * 1024 / (3 * (T::BM + T::BN) * T::BK * (int64_t)sizeof(TA)));
+    const bool brief = WK == 1 && z.K < 3 * T::BK && tiles_of(z, T::BM, T::BN) > fit;
+    if (g.fast && !g.maskA && dma_operands(z) && !brief) return launch_dma<TM, TN, WK>(z, g, s);
   }
   auto nm = [](bool ak, bool bn) {   // formatted once per instance
     static const char* const n[4] = {gemm_kernel_name<Tc, TA, TB, TC, TM, TN, WK>(false, false),
@@ -1010,9 +1020,6 @@ bool autotune_enabled();
 //    32-row products of the blocked QR, 32 x 1984 x 248 x 8: 27.8 us against 42.2).
 inline double wave_fill(int64_t tiles, int64_t slots) {
   return (double)tiles / (double)((tiles + slots - 1) / slots * slots);
-}
-inline int64_t tiles_of(const ZGemm& z, int BM, int BN) {
-  return ((z.M + BM - 1) / BM) * ((z.N + BN - 1) / BN) * z.batch;
 }
 inline bool wave_tile_product(const ZGemm& z) { return tiles_of(z, 16, 8) <= 320; }
 // 128 x 128 tiles (FP32), 128 x 64 tiles, 64 x 32 tiles (else 32 x 16)
